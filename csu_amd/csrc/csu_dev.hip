@@ -15,6 +15,7 @@
 #include <vector>
 #include "csu.h"
 #include "kernels.h"
+#include "kern_stage.h"
 #include "kern_implicit.h"
 #include "kern_setup.h"
 
@@ -76,11 +77,17 @@ struct csu_dev {
   double *res_hist, *coef_hist;
   int hist_cap;
   int fresh;                   // state set from the host: P and dt not yet derived
-  int pu;                      // RK stages recover the primitives from the state (k_grad's PU form)
+  int pu;                      // RK stages pass primitives, not states, to the next (k_update's PO form)
   int sblk;                    // threads per workgroup of k_grad and k_flux
   int lblk;                    // threads per workgroup of an LU-SGS level launch
-  int tile_ok;                 // the tile form's LDS list length (CSU_TILE_FACES_S or CSU_TILE_FACES), 0: no tile form
-  int tile;                    // face fluxes evaluated per cell tile inside k_update, no k_flux (1)
+  int tile_ok;                 // 1: the tile form exists (an inviscid second-order RK run whose tiles fit)
+  int tile;                    // 1: each stage one kernel over cell tiles (k_stage) instead of the split kernels
+  Tile tl;                     // the tile form's lists
+  int quads;                   // 1: the mesh has cells of four edges
+  int tile_nt;                 // threads per tile
+  int tl_capb;                 // boundary entries its LDS array holds
+  size_t tl_n;                 // interior entries in all
+  double* P2;                  // tile form: second primitive buffer (a stage never writes the buffer it reads)
   int tuned;                   // launch shapes from the autotuner (1) or the defaults (0)
   // implicit schemes
   double *Dp, *dW0, *dW1, *A;  // diagonal (without the dt term), increments, DPLUR blocks
@@ -93,7 +100,7 @@ struct csu_dev {
   // step x which buffer holds U; implicit keyed by nothing
   int* hctr;                   // device iteration counter: slot of res/coef history
   hipGraphExec_t gexec[4];
-  double* gU[4];               // d->U at capture
+  double *gU[4], *gP[4];       // d->U, d->st.P at capture
   double* Ubase;               // the buffer U starts in (graph parity key)
   size_t bytes;                // device bytes allocated by this context
   // asynchronous iteration: history rows copied to pinned host memory
@@ -668,14 +675,18 @@ static void tune_lookup(csu_dev* d) {
   d->tuned = 1;
 }
 
-// Face lists of the tile form (k_update TILE): the interior faces of each
-// 256-cell tile (of a batch's solves: their real faces only), a face shared
-// by two tiles in both lists, and each cell slot's face as its place in its
-// own tile's list (signed like cface: + where the cell is the face's e0).
-// False when a tile has more faces than the workgroup's LDS list holds.
-static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, std::vector<int>& toff,
-                       std::vector<int>& tface, std::vector<short>& tsl, int* maxf) {
-  const int nc = H.nc, nt = (nc + CSU_BLOCK - 1) / CSU_BLOCK;
+// Lists of the tile form (k_stage, struct Tile) over the 256-cell tiles of a
+// mesh or of a batch's solves.  False when a tile has more interior faces
+// than CSU_TILE_FACES or its LDS arrays do not fit.
+struct HostTile {
+  std::vector<int> toff, boff, bown, hoff, tbq, tbc, hcell;
+  std::vector<double> fx, fy, fs;
+  std::vector<short> csl, hsl, cel, hel;
+  int capf = 0, capb = 0;
+};
+
+static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, HostTile& T) {
+  const int nc = H.nc, B = CSU_CHUNK, nt = (nc + B - 1) / B;
   auto each_face = [&](auto fn) {
     if (sol && !sol->empty()) {
       for (const SolveP& q : *sol)
@@ -684,44 +695,98 @@ static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, std::v
       for (int f = 0; f < H.nf; f++) fn(f);
     }
   };
-  std::vector<int> cnt(nt, 0);
+  T.toff.assign(nt + 1, 0);
   each_face([&](int f) {
-    const int a = H.fe0[f] / CSU_BLOCK, b = H.fe1[f] / CSU_BLOCK;
-    cnt[a]++;
-    if (b != a) cnt[b]++;
+    const int a = H.fe0[f] / B, b = H.fe1[f] / B;
+    T.toff[a + 1]++;
+    if (b != a) T.toff[b + 1]++;
   });
-  toff.assign(nt + 1, 0);
-  *maxf = 0;
   for (int t = 0; t < nt; t++) {
-    if (cnt[t] > CSU_TILE_FACES) return false;
-    *maxf = std::max(*maxf, cnt[t]);
-    toff[t + 1] = toff[t] + cnt[t];
+    if (T.toff[t + 1] > CSU_TILE_FACES) return false;
+    T.capf = std::max(T.capf, T.toff[t + 1]);
+    T.toff[t + 1] += T.toff[t];
   }
-  tface.assign(toff[nt] > 0 ? toff[nt] : 1, 0);
-  std::vector<int> fill(toff.begin(), toff.end() - 1), loc0(H.nf > 0 ? H.nf : 1, -1), loc1(H.nf > 0 ? H.nf : 1, -1);
+  const size_t ne = T.toff[nt];
+  std::vector<int> ent(ne ? ne : 1), fill(T.toff.begin(), T.toff.end() - 1);
   each_face([&](int f) {
-    const int a = H.fe0[f] / CSU_BLOCK, b = H.fe1[f] / CSU_BLOCK;
-    loc0[f] = fill[a] - toff[a];
-    tface[fill[a]++] = f;
-    if (b != a) {
-      loc1[f] = fill[b] - toff[b];
-      tface[fill[b]++] = f;
-    } else {
-      loc1[f] = loc0[f];
-    }
+    const int a = H.fe0[f] / B, b = H.fe1[f] / B;
+    ent[fill[a]++] = f;
+    if (b != a) ent[fill[b]++] = f;
   });
-  tsl.assign(4 * (size_t)nc, 0);
-  for (int j = 0; j < 4; j++)
-    for (int i = 0; i < nc; i++) {
-      const int cf = H.cface[(size_t)j * nc + i];
-      if (cf == 0) continue;
-      const int f = cf > 0 ? cf - 1 : -cf - 1;
-      const int l = cf > 0 ? loc0[f] : loc1[f];  // cf > 0: i is the face's e0
-      const int t = i / CSU_BLOCK;
-      if (l < 0 || l >= cnt[t] || (cf > 0 ? H.fe0[f] : H.fe1[f]) != i) return false;
-      tsl[(size_t)j * nc + i] = (short)(cf > 0 ? l + 1 : -(l + 1));
+  T.fx.resize(ne ? ne : 1); T.fy.resize(ne ? ne : 1); T.fs.resize(ne ? ne : 1);
+  for (size_t e = 0; e < ne; e++) { T.fx[e] = H.fdsx[ent[e]]; T.fy[e] = H.fdsy[ent[e]]; T.fs[e] = H.fds[ent[e]]; }
+  // halo cells of each tile, ascending
+  T.hoff.assign(nt + 1, 0);
+  std::vector<int> hc;
+  for (int t = 0; t < nt; t++) {
+    hc.clear();
+    for (int e = T.toff[t]; e < T.toff[t + 1]; e++) {
+      const int a = H.fe0[ent[e]], b = H.fe1[ent[e]];
+      if (a / B != t) hc.push_back(a);
+      if (b / B != t) hc.push_back(b);
     }
-  return true;
+    std::sort(hc.begin(), hc.end());
+    hc.erase(std::unique(hc.begin(), hc.end()), hc.end());
+    T.hcell.insert(T.hcell.end(), hc.begin(), hc.end());
+    T.hoff[t + 1] = (int)T.hcell.size();
+  }
+  const size_t nh = T.hcell.size();
+  if (nh == 0) T.hcell.push_back(0);
+  const size_t NH = nh ? nh : 1;
+  T.csl.assign(4 * (size_t)nc, 0); T.cel.assign(4 * (size_t)nc, 0);
+  T.hsl.assign(4 * NH, 0); T.hel.assign(4 * NH, 0);
+  // edge places: where each cell's reconstructed edge states go
+  for (int t = 0; t < nt; t++) {
+    const auto h0 = T.hcell.begin() + T.hoff[t], h1 = T.hcell.begin() + T.hoff[t + 1];
+    auto put = [&](int cell, int edge, int v) {
+      if (cell / B == t) T.cel[(size_t)edge * nc + cell] = (short)v;
+      else T.hel[(size_t)edge * NH + (std::lower_bound(h0, h1, cell) - T.hcell.begin())] = (short)v;
+    };
+    for (int e = T.toff[t]; e < T.toff[t + 1]; e++) {
+      const int f = ent[e], k = e - T.toff[t] + 1;
+      put(H.fe0[f], H.fsl[f] & 3, k);
+      put(H.fe1[f], H.fsl[f] >> 2, -k);
+    }
+  }
+  // slot places: interior slots by the face's place, boundary slots by the
+  // place in the tile's boundary list (own cells' first)
+  std::vector<int> loc0(H.nf > 0 ? H.nf : 1, -1), loc1(H.nf > 0 ? H.nf : 1, -1);
+  for (int t = 0; t < nt; t++)
+    for (int e = T.toff[t]; e < T.toff[t + 1]; e++) {
+      const int f = ent[e];
+      if (H.fe0[f] / B == t) loc0[f] = e - T.toff[t];
+      if (H.fe1[f] / B == t) loc1[f] = e - T.toff[t];
+    }
+  T.boff.assign(nt + 1, 0);
+  T.bown.assign(nt, 0);
+  for (int t = 0; t < nt; t++) {
+    const int c1 = std::min(nc, (t + 1) * B), nown = c1 - t * B, n = nown + T.hoff[t + 1] - T.hoff[t];
+    int nb = 0;
+    for (int k = 0; k < n; k++) {
+      const bool own = k < nown;
+      const int h = T.hoff[t] + k - nown, i = own ? t * B + k : T.hcell[h];
+      for (int j = 0; j < 4; j++) {
+        short* v = own ? &T.csl[(size_t)j * nc + i] : &T.hsl[(size_t)j * NH + h];
+        const int cf = H.cface[(size_t)j * nc + i];
+        if (cf != 0) {
+          if (!own) continue;
+          const int f = cf > 0 ? cf - 1 : -cf - 1, l = cf > 0 ? loc0[f] : loc1[f];
+          if (l < 0 || (cf > 0 ? H.fe0[f] : H.fe1[f]) != i || ((H.bmask[i] >> j) & 1)) return false;
+          *v = (short)(cf > 0 ? l + 1 : -(l + 1));
+        } else if ((H.bmask[i] >> j) & 1) {
+          T.tbq.push_back(-1 - H.cnbr[(size_t)j * nc + i]);
+          T.tbc.push_back(i);
+          *v = (short)++nb;
+        }
+      }
+      if (own) T.bown[t] = nb;
+    }
+    T.capb = std::max(T.capb, nb);
+    T.boff[t + 1] = (int)T.tbq.size();
+  }
+  if (T.tbq.empty()) { T.tbq.push_back(0); T.tbc.push_back(0); }
+  T.capf = (T.capf + 7) & ~7;
+  return 64 * (size_t)(T.capf + T.capb) <= CSU_TILE_LDS;
 }
 
 // Device state of a context from its host arrays: uploads, allocations, wall
@@ -758,9 +823,9 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   d->tuned = 0;
   tune_lookup(d);
   // inviscid ideal-gas second-order RK with the default limiter (any
-  // precision): the stage kernels recover the primitives from the state
-  // (k_grad PU); first order, the global-range limiter and the axisymmetric
-  // source read stored primitives, so those keep them.
+  // precision): the stages before the last store the next stage's
+  // primitives r u v p instead of its state (k_update PO), and the tile form
+  // exists; the other runs store both.
   // CSU_STORED_PRIMITIVES=1 in the environment selects the stored form
   // everywhere (same results; for comparisons of the two forms).
   const char* sp = getenv("CSU_STORED_PRIMITIVES");
@@ -781,6 +846,10 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   kp.gas.cc[0] = 1.81716e3; kp.gas.cc[1] = 9.890504e2 - 287.0530; kp.gas.cc[2] = -9.595592e-3;
   kp.gas.cc[3] = 1.041469e-4; kp.gas.cc[4] = -4.433065e-8; kp.gas.cc[5] = 5.879263e-12;
   kp.gas.tp = p->tp;
+  kp.gas.rCv = 1.0 / kp.gas.Cv;
+  kp.gas.rgm1 = 1.0 / (kp.gas.gamma - 1.0);
+  kp.gas.gam0 = (kp.gas.Cv + kp.gas.R) / kp.gas.Cv;
+  kp.gas.gam0f = ((float)kp.gas.Cv + (float)kp.gas.R) / (float)kp.gas.Cv;
   std::vector<double> pref(6 * (size_t)ns, 0.0);
   for (int s = 0; s < ns; s++) limiter_pref(ps[s], &pref[6 * (size_t)s]);
   if (sol)
@@ -843,19 +912,45 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   }
   if (p->order == 2 && !kp.mixed && (rc = dalloc(d, &s.rec, 4 * nvc))) return rc;
   if (d->pu) {
-    std::vector<int> toff, tface;
-    std::vector<short> tsl;
-    int maxf = 0;
-    if (tile_lists(H, sol, toff, tface, tsl, &maxf)) {
-      if ((rc = upload(d, &g.toff, toff)) || (rc = upload(d, &g.tface, tface)) || (rc = upload(d, &g.tsl, tsl)))
+    d->quads = 0;
+    for (int n : H.cnp) d->quads |= n == 4;
+    HostTile T;
+    if (tile_lists(H, sol, T)) {
+      Tile& tl = d->tl;
+      // Threads per tile: 512 let a tile's halo run beside its own cells and
+      // both rounds of faces at once, which wins while the tiles leave the
+      // chip idle (40k cells 77 -> 68 us per RK5 iteration, 100k quads 130 ->
+      // 116) or where the halo is as large as the tile (column order: 200k
+      // cells 205 -> 181 us); above that, more tiles per CU win (200k cells
+      // in Morton order: 146 us with 256 threads, 157 with 512).
+      const size_t halo = T.hoff.back();
+      d->tile_nt = nc <= 131072 || 2 * halo > (size_t)nc ? 512 : 256;
+      tl.nh = (int)T.hcell.size();
+      tl.capf = T.capf;
+      d->tl_capb = T.capb;
+      d->tl_n = T.fx.size();
+      if ((rc = upload(d, &tl.toff, T.toff)) || (rc = upload(d, &tl.boff, T.boff)) ||
+          (rc = upload(d, &tl.bown, T.bown)) || (rc = upload(d, &tl.hoff, T.hoff)) || (rc = upload(d, &tl.tbq, T.tbq)) || (rc = upload(d, &tl.tbc, T.tbc)) ||
+          (rc = upload(d, &tl.hcell, T.hcell)) || (rc = upload(d, &tl.fx, T.fx)) || (rc = upload(d, &tl.fy, T.fy)) ||
+          (rc = upload(d, &tl.fs, T.fs)) || (rc = upload(d, &tl.csl, T.csl)) || (rc = upload(d, &tl.hsl, T.hsl)) ||
+          (rc = upload(d, &tl.cel, T.cel)) || (rc = upload(d, &tl.hel, T.hel)) || (rc = dalloc(d, &d->P2, 5 * (size_t)nc)))
         return rc;
-      d->tile_ok = maxf <= CSU_TILE_FACES_S ? CSU_TILE_FACES_S : CSU_TILE_FACES;
+      if (kp.mixed) {
+        auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
+        if ((rc = upload(d, &tl.fx32, f32(T.fx))) || (rc = upload(d, &tl.fy32, f32(T.fy))) ||
+            (rc = upload(d, &tl.fs32, f32(T.fs))))
+          return rc;
+      }
+      d->tile_ok = 1;
     }
   }
   if (!d->tile_ok) d->tile = 0;
-  // untuned default: the tile form from 200k cells on, where it measured
-  // 4-6 % faster in every shape (below that, launch latency decides)
-  else if (!d->tuned && nc >= 200000) d->tile = 1;
+  // untuned default: the tile form wherever it exists, unless the halos hold
+  // clearly more cells than the tiles (a scattered numbering): columns
+  // longer than a tile have one halo cell per cell, and there the two forms
+  // measure alike at 2.0M cells (1,309 us, split 1,321) and the tile form
+  // wins below (406k cells 288 against 340)
+  else if (!d->tuned && (double)d->tl.nh <= 1.25 * nc) d->tile = 1;
   if (kp.mixed) {
     auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
     if ((rc = upload(d, &g.lwx32, f32(H.lwx))) || (rc = upload(d, &g.lwy32, f32(H.lwy))) ||
@@ -955,10 +1050,12 @@ static csu_dev* dev_new() {
   d->Dp = d->dW0 = d->dW1 = d->A = d->caux = nullptr; d->jstate = nullptr; d->jred = nullptr; d->cellsL = d->cellsU = nullptr;
   d->hctr = nullptr; d->use_graphs = 1; d->bytes = 0; d->tstate = nullptr;
   d->hres = d->hcoef = nullptr; d->hcap = 0; d->async_start = 0; d->async_n = 0;
-  for (int k = 0; k < 4; k++) { d->gexec[k] = nullptr; d->gU[k] = nullptr; }
+  for (int k = 0; k < 4; k++) { d->gexec[k] = nullptr; d->gU[k] = d->gP[k] = nullptr; }
   memset((void*)&d->kp, 0, sizeof(KP));
   memset((void*)&d->geo, 0, sizeof(Geo));
   memset((void*)&d->st, 0, sizeof(St));
+  memset((void*)&d->tl, 0, sizeof(Tile));
+  d->P2 = nullptr; d->quads = 1; d->tl_capb = 0; d->tl_n = 0;
   return d;
 }
 
@@ -1150,68 +1247,10 @@ extern "C" int csu_dev_kernel_times(csu_dev* d, const char** names, double* avg_
 // orchestration
 // ---------------------------------------------------------------------------
 // One residual evaluation (solverCalcR) with P valid, then the fused update.
-// Us non-null: the primitives-from-state form (k_grad's PU), where Us is the
-// stage's conservative state and P is neither read nor written.
 template <int NV, bool VISC>
-static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, double* Uout,
-                 const double* Us = nullptr) {
+static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, double* Uout) {
   const KP& kp = d->kp;
   const int nc = d->nc;
-  if constexpr (NV == 4 && !VISC) {
-    if (Us) {
-      St st = d->st;
-      st.Us = Us;
-      if (d->nb > 0) {
-        Prof p(d, "k_bcflux");
-        hipLaunchKernelGGL((k_bcflux<4, true>), dim3(nblk(d->nb)), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo, st);
-      }
-      {
-        Prof p(d, "k_grad");
-        if (kp.mixed)
-          hipLaunchKernelGGL((k_grad<4, false, false, true, true>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp,
-                             d->geo, st);
-        else if (kp.lsq_ld)
-          hipLaunchKernelGGL((k_grad<4, false, true, false, true>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp,
-                             d->geo, st);
-        else
-          hipLaunchKernelGGL((k_grad<4, false, false, false, true>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp,
-                             d->geo, st);
-      }
-      if (d->nf > 0 && !d->tile) {
-        Prof p(d, "k_flux");
-        if (kp.mixed)
-          hipLaunchKernelGGL((k_flux<4, false, true>), dim3((d->nf + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo, st);
-        else
-          hipLaunchKernelGGL((k_flux<4, false>), dim3((d->nf + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo, st);
-      }
-      {
-        Prof p(d, "k_update");
-        const dim3 gu(nblk(nc)), bu(CSU_BLOCK);
-        double* const rdt = d->red + (size_t)NV * d->nred;
-        const bool ts = d->tile_ok == CSU_TILE_FACES_S;
-        if (kp.mixed && d->tile && ts)
-          hipLaunchKernelGGL((k_update<4, false, true, true, CSU_TILE_FACES_S>), gu, bu, 0, d->stream, kp, d->geo, st,
-                             flags, sigma, rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red, rdt);
-        else if (kp.mixed && d->tile)
-          hipLaunchKernelGGL((k_update<4, false, true, true, CSU_TILE_FACES>), gu, bu, 0, d->stream, kp, d->geo, st,
-                             flags, sigma, rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red, rdt);
-        else if (kp.mixed)
-          hipLaunchKernelGGL((k_update<4, false, true, true>), gu, bu, 0, d->stream, kp, d->geo, st, flags, sigma,
-                             rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red, rdt);
-        else if (d->tile && ts)
-          hipLaunchKernelGGL((k_update<4, false, false, true, CSU_TILE_FACES_S>), gu, bu, 0, d->stream, kp, d->geo, st,
-                             flags, sigma, rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red, rdt);
-        else if (d->tile)
-          hipLaunchKernelGGL((k_update<4, false, false, true, CSU_TILE_FACES>), gu, bu, 0, d->stream, kp, d->geo, st,
-                             flags, sigma, rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red, rdt);
-        else
-          hipLaunchKernelGGL((k_update<4, false, false, true>), gu, bu, 0, d->stream, kp, d->geo, st, flags, sigma,
-                             rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red, rdt);
-      }
-      HIPCHK(hipGetLastError());
-      return CSU_OK;
-    }
-  }
   if (kp.order == 2 && kp.limiter == 1) {
     Prof p(d, "k_lim1");
     hipLaunchKernelGGL(k_lim1_partial<NV>, dim3(nblk(nc)), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo, d->st.P, d->red);
@@ -1243,7 +1282,15 @@ static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, d
   }
   {
     Prof p(d, "k_update");
-    if (kp.mixed)
+    double* const rdt = d->red + (size_t)NV * d->nred;
+    if (NV == 4 && !VISC && d->pu && (flags & F_RK)) {
+      if (kp.mixed)
+        hipLaunchKernelGGL((k_update<4, false, true, true>), dim3(nblk(nc)), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo,
+                           d->st, flags, sigma, rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red, rdt);
+      else
+        hipLaunchKernelGGL((k_update<4, false, false, true>), dim3(nblk(nc)), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo,
+                           d->st, flags, sigma, rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red, rdt);
+    } else if (kp.mixed)
       hipLaunchKernelGGL((k_update<NV, VISC, true>), dim3(nblk(nc)), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo, d->st,
                          flags, sigma, rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red,
                          d->red + (size_t)NV * d->nred);
@@ -1252,6 +1299,31 @@ static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, d
                          flags, sigma, rk_a, d->prm.cfl, d->dtl, d->dtg, Un, Uout, d->R, d->red,
                          d->red + (size_t)NV * d->nred);
   }
+  HIPCHK(hipGetLastError());
+  return CSU_OK;
+}
+
+// One RK stage in the tile form; the buffer it wrote becomes the current
+// primitives.
+template <int NT>
+static int tile_stage(csu_dev* d, int flags, double sigma, double rk_a) {
+  const KP& kp = d->kp;
+  const St& st = d->st;
+  const size_t lds = 8 * ((kp.mixed ? 4 : 8) * (size_t)d->tl.capf + 8 * (size_t)d->tl_capb);
+  double* const rdt = d->red + 4 * (size_t)d->nred;
+  const dim3 gu(nblk(d->nc)), bu(NT);
+  Prof p(d, "k_stage");
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, gu, bu, lds, d->stream, kp, d->geo, st, d->tl, flags, sigma, rk_a, d->prm.cfl, d->dtl,
+                       d->dtg, d->U, d->Uaux, d->P2, d->red, rdt);
+  };
+  const bool roe = kp.flux == 0;
+  if (kp.lsq_ld) go(k_stage<NT, 4, -1, false, true>);
+  else if (kp.mixed && !d->quads) roe ? go(k_stage<NT, 3, 0, true, false>) : go(k_stage<NT, 3, -1, true, false>);
+  else if (kp.mixed) roe ? go(k_stage<NT, 4, 0, true, false>) : go(k_stage<NT, 4, -1, true, false>);
+  else if (!d->quads) roe ? go(k_stage<NT, 3, 0, false, false>) : go(k_stage<NT, 3, -1, false, false>);
+  else roe ? go(k_stage<NT, 4, 0, false, false>) : go(k_stage<NT, 4, -1, false, false>);
+  std::swap(d->st.P, d->P2);
   HIPCHK(hipGetLastError());
   return CSU_OK;
 }
@@ -1381,10 +1453,10 @@ static int is_local(const csu_dev* d, int it) {
 // replay slot k when it was captured with the same U buffer.
 template <typename F>
 static int run_graph(csu_dev* d, int k, F body) {
-  if (!d->gexec[k] || d->gU[k] != d->U) {
+  if (!d->gexec[k] || d->gU[k] != d->U || d->gP[k] != d->st.P) {
     if (d->gexec[k]) (void)hipGraphExecDestroy(d->gexec[k]);
     d->gexec[k] = nullptr;
-    double* u0 = d->U;
+    double *u0 = d->U, *p0 = d->st.P;
     HIPCHK(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
     int rc = body();
     hipGraph_t graph = nullptr;
@@ -1395,6 +1467,7 @@ static int run_graph(csu_dev* d, int k, F body) {
     (void)hipGraphDestroy(graph);
     if (e != hipSuccess) { d->gexec[k] = nullptr; return set_err(CSU_ERR_HIP, "graph instantiate: %s", hipGetErrorString(e)); }
     d->gU[k] = u0;
+    d->gP[k] = p0;
     d->U = u0;  // the body's host-side pointer swaps are replayed by the graph
     // a capture records work without running it: replay once now
   }
@@ -1413,28 +1486,29 @@ static int rk_iteration(csu_dev* d, int it_index) {
   int first_flags = F_CLAMP_UN;
   if (d->fresh) {
     // time step from the unclamped state (solverCalcDt), then primitives
-    // (the primitives-from-state form recovers them in the stage kernels
-    // and clamps U^n in the first update, as after any other iteration)
     Prof p(d, "k_dt");
     hipLaunchKernelGGL(k_dt<NV>, dim3(nblk(nc)), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->geo, cur_local, d->prm.cfl,
                        d->U, d->dtl, red_dt);
     if (!cur_local)
       hipLaunchKernelGGL(k_dt_final, dim3(d->nsolve), dim3(CSU_BLOCK), 0, d->stream, nblk(nc), d->prm.cfl, red_dt,
                          d->dtg, d->geo.sol);
-    if (!d->pu) {
-      int rc = prim_pass<NV>(d);
-      if (rc) return rc;
-      first_flags = 0;
-    }
+    int rc = prim_pass<NV>(d);
+    if (rc) return rc;
+    first_flags = 0;
     d->fresh = 0;
   }
   if (d->st.tube)
     hipLaunchKernelGGL(k_time_clamp, dim3(1), dim3(64), 0, d->stream, d->tstate, d->dtg, d->prm.stages);
   for (int s = 0; s < d->prm.stages; s++) {
     const bool last = s == d->prm.stages - 1;
-    int flags = F_RK | (cur_local ? F_CUR_LOCAL : 0) | (s == 0 ? first_flags : 0);
-    if (last) flags |= F_LAST | F_STORE_R | (next_local ? F_NEXT_LOCAL : 0);
-    int rc = stage<NV, VISC>(d, flags, sigma, a[s], d->U, d->Uaux, d->pu ? (s == 0 ? d->U : d->Uaux) : nullptr);
+    int flags = F_RK | (cur_local ? F_CUR_LOCAL : 0) | (s == 0 || d->tile ? first_flags : 0);
+    if (last) flags |= F_LAST | (next_local ? F_NEXT_LOCAL : 0);
+    if (d->tile) {
+      int rc = d->tile_nt == 512 ? tile_stage<512>(d, flags, sigma, a[s]) : tile_stage<256>(d, flags, sigma, a[s]);
+      if (rc) return rc;
+      continue;
+    }
+    int rc = stage<NV, VISC>(d, flags, sigma, a[s], d->U, d->Uaux);
     if (rc) return rc;
   }
   std::swap(d->U, d->Uaux);
@@ -1638,7 +1712,7 @@ extern "C" int csu_dev_autotune(csu_dev* d, int32_t iters, int32_t* choice) {
   TuneVal best{d->sblk, d->lblk, d->kp.xcd, d->tile};
   float best_ms = 1e30f;
   for (int u = 0; u < (d->tile_ok ? 2 : 1) && !rc; u++)
-  for (int a = 0; a < 3 && !rc; a++)
+  for (int a = u ? 2 : 0; a < 3 && !rc; a++)  // the tile form has no gradient and face workgroups
     for (int b = 0; b < (lus ? 3 : 1) && !rc; b++)
       for (int x = 1; x >= 0 && !rc; x--) {
         d->tile = u;
@@ -1933,6 +2007,10 @@ extern "C" int csu_dev_set_precision(csu_dev* d, int32_t prec) {
       return rc;
     if (!s.fflux32 && (rc = dalloc(d, &s.fflux32, (size_t)d->nv * nf))) return rc;
     if (d->prm.order == 2 && !s.rec32 && (rc = dalloc(d, &s.rec32, 4 * nvc))) return rc;
+    if (d->tile_ok && !d->tl.fx32 && ((rc = f32(d->tl.fx, &d->tl.fx32, d->tl_n)) ||
+                                      (rc = f32(d->tl.fy, &d->tl.fy32, d->tl_n)) ||
+                                      (rc = f32(d->tl.fs, &d->tl.fs32, d->tl_n))))
+      return rc;
   } else if (d->prm.order == 2 && !s.rec && (rc = dalloc(d, &s.rec, 4 * nvc))) {
     return rc;
   }
@@ -2212,7 +2290,13 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
   if (p->time_scheme == CSU_TIME_LUSGS) b += nc * 24 + nf * 24;
   if (p->time_scheme == CSU_TIME_DPLUR) b += 32 * nv * nv * nc + 8.0 * (p->nlinear > 0 ? p->nlinear : 1) * (nc / 256 + 1);
   if (p->precision == 1) b += nc * 64 + nf * (12 + 4 * nv) + (p->order == 2 ? 16 * nv * nc : 0);  // FP32 copies
-  if (p->time_scheme == CSU_TIME_RK && !visc && p->order == 2) b += 8 * nc + 8 * nf + 4 * (nc / 256 + 2);  // tile lists
+  if (p->time_scheme == CSU_TIME_RK && !visc && p->order == 2 && p->limiter != 1 && m->axi == 0 && p->tp == 0) {
+    // tile form: second primitive buffer, places, face copies, halo cells (at
+    // most one per tile and face between two tiles)
+    double cross = 0;
+    for (int f = 0; f < m->nface; f++) cross += m->face[4 * (size_t)f] / CSU_CHUNK != m->face[4 * (size_t)f + 1] / CSU_CHUNK;
+    b += nc * (40 + 16) + (nf + cross) * (p->precision == 1 ? 36 : 24) + 2 * cross * 20 + 12 * nb + 16 * (nc / 256 + 2);
+  }
   b += (nv + 4) * 8 * (double)(hist > 0 ? hist : 1);
   // allocation granularity: every array rounds up (at most 2 MiB slack per large array)
   return (int64_t)(b * 1.02) + (int64_t)64 * 4096;

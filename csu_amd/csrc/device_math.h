@@ -19,7 +19,70 @@ struct GasD {
   double gamma, R, Cp, Cv;
   double cc[6];
   int tp;
+  // derived once on the host: 1/Cv, 1/(gamma-1) (rounded; see Den), and
+  // (Cv+R)/Cv as the double and the float forms below round it
+  double rCv, rgm1, gam0;
+  float gam0f;
 };
+
+// Quotients that share a denominator.  b is inverted once (two Newton steps
+// from the hardware estimate); a quotient is then a*r corrected by its exact
+// remainder (a fused multiply-add), which rounds correctly (Markstein 1990),
+// so each equals a / b bit for bit as long as neither b nor the quotient is
+// near the ends of the exponent range; zeros, infinities and NaN go
+// through the hardware's fix-up as in a / b.  4 instructions per FP64
+// quotient after 5 for the reciprocal, against 11 for a / b.
+template <typename T>
+struct Den;
+template <>
+struct Den<double> {
+  double b, r;
+  __device__ __forceinline__ explicit Den(double d) : b(d) {
+    r = __builtin_amdgcn_rcp(d);
+    r = __fma_rn(__fma_rn(-b, r, 1.0), r, r);
+    r = __fma_rn(__fma_rn(-b, r, 1.0), r, r);
+  }
+  __device__ __forceinline__ Den(double d, double rd) : b(d), r(rd) {}  // rd: 1/d, rounded
+  __device__ __forceinline__ double operator()(double a) const {
+    const double q = a * r;
+    return __builtin_amdgcn_div_fixup(__fma_rn(__fma_rn(-b, q, a), r, q), b, a);
+  }
+};
+template <>
+struct Den<float> {  // one Newton step, two remainder corrections
+  float b, r;
+  __device__ __forceinline__ explicit Den(float d) : b(d) {
+    r = __builtin_amdgcn_rcpf(d);
+    r = __fmaf_rn(__fmaf_rn(-b, r, 1.0f), r, r);
+  }
+  __device__ __forceinline__ float operator()(float a) const {
+    float q = a * r;
+    q = __fmaf_rn(__fmaf_rn(-b, q, a), r, q);
+    return __builtin_amdgcn_div_fixupf(__fmaf_rn(__fmaf_rn(-b, q, a), r, q), b, a);
+  }
+};
+// Square root, correctly rounded as sqrt() is: Goldschmidt's coupled
+// iteration from the hardware's reciprocal root, then two corrections by the
+// exact remainder (Markstein 1990).  Half of sqrt()'s instructions: no
+// scaling of the argument, which only values near the ends of the exponent
+// range need (below 2^-767).
+__device__ __forceinline__ double fsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __fma_rn(-h, g, 0.5);
+  g = __fma_rn(g, r, g);
+  h = __fma_rn(h, r, h);
+  g = __fma_rn(__fma_rn(-g, g, x), h, g);
+  g = __fma_rn(__fma_rn(-g, g, x), h, g);
+  return x == 0.0 || x == __builtin_inf() ? x : g;
+}
+__device__ __forceinline__ float fsqrt(float x) { return sqrtf(x); }
+
+template <typename T>
+__device__ __forceinline__ Den<T> den_gm1(const GasD& g) {
+  if constexpr (sizeof(T) == 8) return Den<double>(g.gamma - 1.0, g.rgm1);
+  else return Den<float>((float)g.gamma - 1.0f);
+}
 
 template <typename T>
 __device__ __forceinline__ T gas_T2e(const GasD& g, T Tk) {
@@ -57,7 +120,9 @@ __device__ __forceinline__ void gas_T2eCv(const GasD& g, T Tk, T& e, T& Cv) {
 template <typename T>
 __device__ __forceinline__ T gas_e2T(const GasD& g, T e) {
   // gasprop.c:144-166: Newton on e(T), at most 8 steps, |dT| > 1e-14
-  T Tk = e / (T)g.Cv;
+  T Tk;
+  if constexpr (sizeof(T) == 8) Tk = Den<double>(g.Cv, g.rCv)(e);
+  else Tk = e / (T)g.Cv;
   if (g.tp) {
     T err = 1, e1, Cv;
     int i = 0;
@@ -73,13 +138,17 @@ __device__ __forceinline__ T gas_e2T(const GasD& g, T e) {
 
 template <typename T>
 __device__ __forceinline__ T gas_T2gamma(const GasD& g, T Tk) {
+  if (!g.tp) {
+    if constexpr (sizeof(T) == 8) return g.gam0;
+    else return g.gam0f;
+  }
   T Cv = gas_T2Cv<T>(g, Tk);
   return (Cv + (T)g.R) / Cv;
 }
 
 template <typename T>
 __device__ __forceinline__ T gas_T2c(const GasD& g, T Tk) {
-  return sqrt(gas_T2gamma<T>(g, Tk) * (T)g.R * Tk);
+  return fsqrt(gas_T2gamma<T>(g, Tk) * (T)g.R * Tk);
 }
 
 template <typename T>
@@ -189,6 +258,13 @@ __device__ __forceinline__ void rotate(T& u, T& v, T dSx, T dSy, T dS) {
   v = (-u * dSy + v * dSx) / dS;
   u = aux;
 }
+// the same with the length inverted once for a face's six quotients
+template <typename T>
+__device__ __forceinline__ void rotate(T& u, T& v, T dSx, T dSy, const Den<T>& dS) {
+  T aux = dS(u * dSx + v * dSy);
+  v = dS(-u * dSy + v * dSx);
+  u = aux;
+}
 
 // ---------------------------------------------------------------------------
 // Convective fluxes in the face frame (reference flux.c).  Primitive inputs
@@ -207,33 +283,36 @@ __device__ __forceinline__ void flux_roe(const GasD& g, T efix, T rL, T uL, T vL
   // flux.c:59-129 (Roe 1981); ideal-gas gamma only, as the reference
   const T gm1 = (T)g.gamma - (T)1;
   T U0L = rL, U1L = rL * uL, U2L = rL * vL;
-  T U3L = pL / gm1 + (uL * uL + vL * vL) * rL / (T)2;
+  const Den<T> dg = den_gm1<T>(g);
+  T U3L = dg(pL) + (uL * uL + vL * vL) * rL / (T)2;
   T HL = (U3L + pL) / rL;
   T U0R = rR, U1R = rR * uR, U2R = rR * vR;
-  T U3R = pR / gm1 + (uR * uR + vR * vR) * rR / (T)2;
+  T U3R = dg(pR) + (uR * uR + vR * vR) * rR / (T)2;
   T HR = (U3R + pR) / rR;
-  T rqL = sqrt(rL), rqR = sqrt(rR);
-  T ub = (rqL * uL + rqR * uR) / (rqL + rqR);
-  T vb = (rqL * vL + rqR * vR) / (rqL + rqR);
-  T Hb = (rqL * HL + rqR * HR) / (rqL + rqR);
-  T ab = sqrt(gm1 * (Hb - (ub * ub + vb * vb) / (T)2));
-  T l1 = ub - ab, l2 = ub, l4 = ub, l5 = ub + ab;
+  T rqL = fsqrt(rL), rqR = fsqrt(rR);
+  const Den<T> dq(rqL + rqR);
+  T ub = dq(rqL * uL + rqR * uR);
+  T vb = dq(rqL * vL + rqR * vR);
+  T Hb = dq(rqL * HL + rqR * HR);
+  T ab = fsqrt(gm1 * (Hb - (ub * ub + vb * vb) / (T)2));
+  T l1 = ub - ab, l2 = ub, l5 = ub + ab;
   T e1[4] = {(T)1, ub - ab, vb, Hb - ub * ab};
   T e2v[4] = {(T)0, (T)0, (T)1, vb};
   T e4[4] = {(T)1, ub, vb, (T)0.5 * (ub * ub + vb * vb)};
   T e5[4] = {(T)1, ub + ab, vb, Hb + ub * ab};
   T d1 = U0R - U0L, d2 = U1R - U1L, d3 = U2R - U2L, d5 = U3R - U3L;
   T a4 = (Hb - (ub * ub + vb * vb)) * d1 + ub * d2 + vb * d3 - d5;
-  a4 /= (ab * ab) / gm1;
+  a4 /= dg(ab * ab);
   T a2v = d3 - d1 * vb;
-  T a5 = ((d1 - a4) + (d2 - ub * d1) / ab) * (T)0.5;
-  T a1 = ((d1 - a4) - (d2 - ub * d1) / ab) * (T)0.5;
+  const T dn = (d2 - ub * d1) / ab;
+  T a5 = ((d1 - a4) + dn) * (T)0.5;
+  T a1 = ((d1 - a4) - dn) * (T)0.5;
   T fL[4] = {U1L, U1L * uL + pL, U1L * vL, uL * (U3L + pL)};
   T fR[4] = {U1R, U1R * uR + pR, U1R * vR, uR * (U3R + pR)};
   entropy_fix<T>(efix, l1);
   entropy_fix<T>(efix, l2);
-  entropy_fix<T>(efix, l4);
   entropy_fix<T>(efix, l5);
+  const T l4 = l2;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
     f[i] = (T)0.5 * (fR[i] + fL[i] - a1 * fabs(l1) * e1[i] - a2v * fabs(l2) * e2v[i] -
@@ -287,8 +366,10 @@ __device__ __forceinline__ void flux_ausmdv(const GasD& g, T rL, T uL, T vL, T p
   state_HTc<T>(g, rR, uR, vR, pR, kR, HR, TR);
   T cL = gas_T2c<T>(g, TL), cR = gas_T2c<T>(g, TR);
   T cm = fmax(cL, cR);
-  T alphaL = ((T)2.0 * pL / rL) / (pL / rL + pR / rR);
-  T alphaR = ((T)2.0 * pR / rR) / (pL / rL + pR / rR);
+  const T prL = pL / rL, prR = pR / rR;  // 2 p / r is twice p / r exactly
+  const Den<T> ds(prL + prR);
+  T alphaL = ds((T)2.0 * prL);
+  T alphaR = ds((T)2.0 * prR);
   T uLPlus, pLPlus;
   aux = (T)0.5 * (uL + fabs(uL));
   if (fabs(uL) < cm) {
@@ -491,7 +572,7 @@ __device__ __forceinline__ void bc_wall(const GasD& g, const double* Pd, double*
 }
 
 // Venkatakrishnan-type limiter function, reference limiter.c:98-147
-template <typename T>
+template <typename T, bool REF = false>
 __device__ __forceinline__ T limiter_v2d(T d1max, T d1min, T d2, T ee);
 
 template <typename T>
@@ -504,9 +585,20 @@ __device__ __forceinline__ T limiter_v2(T Ui, T Umin, T Umax, T d2, T ee) {
 // use, so one straight-line evaluation with that difference selected gives
 // the same operations per lane without divergent branches (each holding
 // two divisions) in a wavefront.
-template <typename T>
+// REF: the reference's sequence of roundings (the long double least-squares
+// mode, whose histories match the reference's where one-ulp differences
+// grow); else the FP64 form below.
+template <typename T, bool REF>
 __device__ __forceinline__ T limiter_v2d(T d1max, T d1min, T d2, T ee) {
   const T d1 = d2 > (T)0 ? d1max : d1min;
+  if constexpr (sizeof(T) == 8 && !REF) {
+    // the common factor d2 of numerator and denominator taken out: the same
+    // function with one division and fewer roundings (d1 d2 >= 0, so every
+    // term is a sum of non-negative ones)
+    const T a = d1 * d1 + ee, b = d1 * d2;
+    const T ans = (a + (T)2 * b) / (a + b + (T)2 * (d2 * d2));
+    return d2 == (T)0 ? (T)1 : ans;
+  }
   T ans = (d1 * d1 + ee) * d2 + (T)2 * d2 * d2 * d1;
   ans /= d1 * d1 + (T)2 * d2 * d2 + d1 * d2 + ee;
   ans /= d2;

@@ -13,12 +13,10 @@ namespace csu {
 // solve, and a solve's per-block reduction partials are those of its own
 // run alone.
 #define CSU_CHUNK 256
-// tile form of the face flux + update: the LDS face lists of a 256-cell
-// tile (its cells' interior faces, those shared with other tiles included):
-// the short one where every tile of the mesh fits (a triangle mesh in
-// column order has ~513), else the long one
-#define CSU_TILE_FACES_S 640
+// tile form (kern_stage.h): interior faces of a 256-cell tile (its cells'
+// faces, those shared with other tiles included) and LDS bytes at most
 #define CSU_TILE_FACES 1024
+#define CSU_TILE_LDS 155648
 
 // Scalar options and free-stream data, passed by value.  nc, nf, nb are the
 // array strides (the whole batch); cend, fend, bend the end of the
@@ -125,8 +123,6 @@ struct Geo {
   const int *csolk, *fsolk, *bsolk, *csol;
   const int *cnp, *cnbr, *cface;                        // [nc], [4][nc], [4][nc]
   const int* cfn;  // implicit schemes: [4][nc] the other cell of face slot j, -1 where cface is 0
-  const int *toff, *tface;  // tile form: faces of tile t are tface[toff[t] .. toff[t+1])
-  const short* tsl;         // tile form: [4][nc] +-(1 + the slot's face's place in its tile's list), 0: none
   const double *xc, *yc, *omega, *dsxm, *dsym, *dslat;  // [nc]
   const double *edx, *edy;                              // [4][nc] own-edge midpoint offsets
   const double *lwx, *lwy;                              // [4][nc] LSQ weights per neighbour slot
@@ -156,7 +152,6 @@ struct St {
   double *wten;         // viscous: wall shear tensor txx txy tyy yp per boundary face [4][nb]
   double *bflux;        // convective boundary-face flux times dS [NV][nb]
   const double *tube;   // time-accurate run: t, tmax, state (0 running, 1 last step, 2 past it), steps
-  const double *Us;     // primitives-from-state stages: the stage's conservative state [NV][nc]
 };
 
 // Primitive recovery of one cell with the positivity clamps, reference
@@ -167,17 +162,18 @@ template <int NV>
 __device__ __forceinline__ void prim_point(const KP& kp, double* u, double* p) {
   const double r0 = fmax(u[0], kp.rlim);
   u[0] = r0;
+  const Den<double> dr(r0);
   double k = 0;
   if (NV == 6) {
-    k = u[4] / r0;
+    k = dr(u[4]);
     if (k < 1e-14) { k = 1e-14; u[4] = r0 * k; }
     p[5] = k;
-    double om = u[5] / r0;
+    double om = dr(u[5]);
     if (om <= 0.0) { om = 0.0; u[5] = r0 * om; }
     p[6] = om;
   }
-  const double uu = u[1] / r0, vv = u[2] / r0;
-  double e = u[3] / r0 - 0.5 * (uu * uu + vv * vv) - k;
+  const double uu = dr(u[1]), vv = dr(u[2]);
+  double e = dr(u[3]) - 0.5 * (uu * uu + vv * vv) - k;
   e = fmax(e, 7.176325e+02);
   double T = gas_e2T<double>(kp.gas, e);
   if (T < 1) {
@@ -189,7 +185,7 @@ __device__ __forceinline__ void prim_point(const KP& kp, double* u, double* p) {
   p[3] = kp.gas.R * T * r0;
   p[4] = T;
   if (NV == 5) {
-    double n = u[4] / r0;
+    double n = dr(u[4]);
     n = fmax(n, 0.0);
     u[4] = n * r0;
     p[5] = n;
@@ -314,10 +310,11 @@ __device__ __forceinline__ void bc_flux(const KP& kp, int type, double dSx, doub
 template <int NV>
 __device__ __forceinline__ double cell_dt(const KP& kp, const double* u, double om, double sx, double sy) {
   double k = 0;
-  if (NV == 6) k = u[4] / u[0];
-  double E = u[3] / u[0];
-  double uu = u[1] / u[0];
-  double vv = u[2] / u[0];
+  const Den<double> dr(u[0]);
+  if (NV == 6) k = dr(u[4]);
+  double E = dr(u[3]);
+  double uu = dr(u[1]);
+  double vv = dr(u[2]);
   double aux = (E - (uu * uu + vv * vv) / 2 - k);
   double T = gas_e2T<double>(kp.gas, aux);
   double c = gas_T2c<double>(kp.gas, T);

@@ -69,13 +69,7 @@ __device__ __forceinline__ void lsq_grad(int np, const double* dx, const double*
 // (boundary.c:695-742).
 // MIX (mixed precision): gradients, limiter and reconstruction in FP32 from
 // FP64 differences; edge states stored in FP32.
-// PU (inviscid second-order RK runs): the primitives of the cell and its
-// neighbours are recovered here from the stage's conservative state s.Us,
-// which the update kernel then writes unclamped, instead of being stored
-// by the update kernel and read back: the same function of the same values
-// (solverCalcPrimitive on the unclamped stage state), 40 bytes per cell
-// less written and 8 less read per stage.
-template <int NV, bool VISC, bool LD, bool MIX = false, bool PU = false>
+template <int NV, bool VISC, bool LD, bool MIX = false>
 __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   using TF = typename std::conditional<MIX, float, double>::type;
   constexpr int NS = NV + 1;
@@ -91,13 +85,8 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   const int np = g.cnp[i];
   const double x0 = g.xc[i], y0 = g.yc[i];
   double Pi[NS];
-  if (PU) {
-    double u[4] = {s.Us[i], s.Us[nc + i], s.Us[2 * nc + i], s.Us[3 * nc + i]};
-    prim_point<4>(kp, u, Pi);
-  } else {
 #pragma unroll
-    for (int m = 0; m < NS; m++) Pi[m] = s.P[m * nc + i];
-  }
+  for (int m = 0; m < NS; m++) Pi[m] = s.P[m * nc + i];
   // neighbours: cells, or the ghost states of boundary faces (k_bcflux)
   double dx[4], dy[4];
   int gb[4], nbr[4];
@@ -123,35 +112,6 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   // them inside the variable loop would serialise one memory round trip
   // per variable.  Slots past np read the cell itself and are not used.
   double vnb[4][NV], vT[4];
-  if (PU) {
-    // all neighbour states first, then their primitives; ghost states as
-    // stored; slots past np take the cell's own values
-    double un[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const bool act = j < np;
-      const int n = act ? nbr[j] : i;
-      const double* base = n >= 0 ? s.Us + n : s.Pb + (-1 - n);
-      const int st = n >= 0 ? nc : nb;
-#pragma unroll
-      for (int kk = 0; kk < 4; kk++) un[j][kk] = base[kk * st];
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const bool act = j < np;
-      const int n = act ? nbr[j] : i;
-      if (act && n >= 0) {
-        double pp[5];
-        prim_point<4>(kp, un[j], pp);
-#pragma unroll
-        for (int kk = 0; kk < NV; kk++) vnb[j][kk] = pp[kk];
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < NV; kk++) vnb[j][kk] = act ? un[j][kk] : Pi[kk];
-      }
-      vT[j] = 0.0;
-    }
-  } else {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const bool act = j < np;
@@ -165,7 +125,6 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
       }
       vT[j] = VISC ? base[4 * st] : 0.0;
     }
-  }
   // every cell has slots 0-2; slot 3 (quads only) is read only by quads,
   // a branch that is uniform on triangle and quad meshes alike
   TF ex[4] = {0, 0, 0, 0}, ey[4] = {0, 0, 0, 0};
@@ -286,7 +245,7 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           if (j >= np) break;
-          const TF p0 = limiter_v2d<TF>(d1max, d1min, d2[j], (TF)pref2);
+          const TF p0 = limiter_v2d<TF, LD>(d1max, d1min, d2[j], (TF)pref2);
           ph = (j == 0) ? p0 : fmin(ph, p0);
         }
       }
@@ -459,13 +418,14 @@ __device__ __forceinline__ void conv_flux(const KP& kp, const Geo& g, const St& 
       PR[kk] = (TF)s.P[m * nc + e1];
     }
   }
-  rotate<TF>(PL[1], PL[2], dSx, dSy, dS);
-  rotate<TF>(PR[1], PR[2], dSx, dSy, dS);
+  const Den<TF> dl(dS);
+  rotate<TF>(PL[1], PL[2], dSx, dSy, dl);
+  rotate<TF>(PR[1], PR[2], dSx, dSy, dl);
   TF fl[NV];
   constexpr int NSC = NV - 4;
   flux_dispatch<TF, NSC>(kp.gas, kp.flux, (TF)kp.efix, (TF)kp.minf, PL[0], PL[1], PL[2], PL[3], PL + 4, PR[0],
                          PR[1], PR[2], PR[3], PR + 4, NV == 6 ? PL[4] : (TF)0, NV == 6 ? PR[4] : (TF)0, fl);
-  rotate<TF>(fl[1], fl[2], dSx, -dSy, dS);
+  rotate<TF>(fl[1], fl[2], dSx, -dSy, dl);
 #pragma unroll
   for (int kk = 0; kk < NV; kk++) out[kk] = fl[kk] * dS;
 }
@@ -551,7 +511,7 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_flux(KP kp, Geo g, St s) {
 // (boundaryCalcPrimitive, boundary.c:514-693) into Pb, and the convective
 // flux from the first-order state, boundaryCalc / _sa / _sst
 // (boundary.c:143-446): f*dS, or 0 when dS = 0.
-template <int NV, bool PU = false>
+template <int NV>
 __global__ __launch_bounds__(CSU_BLOCK) void k_bcflux(KP kp, Geo g, St s) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   const int nc = kp.nc, nb = kp.nb;
@@ -559,13 +519,8 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_bcflux(KP kp, Geo g, St s) {
   if (q >= kp.bend) return;
   const int i = g.be0[q];
   double Pi[NV + 1], R[NV], Pg[NV + 1];
-  if (PU) {  // primitives of the stage state (see k_grad)
-    double u[4] = {s.Us[i], s.Us[nc + i], s.Us[2 * nc + i], s.Us[3 * nc + i]};
-    prim_point<4>(kp, u, Pi);
-  } else {
 #pragma unroll
-    for (int m = 0; m < NV + 1; m++) Pi[m] = s.P[m * nc + i];
-  }
+  for (int m = 0; m < NV + 1; m++) Pi[m] = s.P[m * nc + i];
   ghost_state<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, NV == 6 ? g.wdist[i] : 0.0, Pg);
 #pragma unroll
   for (int m = 0; m < NV + 1; m++) s.Pb[m * nb + q] = Pg[m];
@@ -584,14 +539,8 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_bcflux(KP kp, Geo g, St s) {
 // fused with the next stage's solverCalcPrimitive, and on the last stage
 // the next time step (solver.c:895-950) and solverCalcRes partials
 // (solver.c:867-892).
-// TILE > 0 (inviscid runs): no face-flux kernel.  The workgroup of a 256-cell
-// tile first evaluates the convective flux of every interior face of its
-// cells into LDS (conv_flux, as the face kernel does; a face between two
-// tiles is evaluated by both), then each cell sums its faces' fluxes from
-// LDS in its slot order: the same values in the same order, without the
-// face-flux array's write and gather.  TILE is the LDS list's length (the
-// smaller one where every tile of the mesh fits: more workgroups per CU).
-template <int NV, bool VISC, bool MIX = false, bool PU = false, int TILE = 0>
+// PO (inviscid second-order RK runs): see the stores below.
+template <int NV, bool VISC, bool MIX = false, bool PO = false>
 __global__ __launch_bounds__(CSU_BLOCK) void k_update(KP kp, Geo g, St s, int flags, double sigma, double rk_a,
                                                       double cfl, double* dtl, const double* dtg, double* Un,
                                                       double* __restrict__ Uout, double* __restrict__ Rout,
@@ -610,22 +559,6 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_update(KP kp, Geo g, St s, int fl
     held = !q.active;
   }
   const bool active = i < kp.cend;
-  using TS = typename std::conditional<MIX, float, double>::type;
-  __shared__ TS sfl[TILE > 0 ? TILE * NV : 1];
-  if (TILE > 0) {
-    static_assert(TILE == 0 || !VISC, "tile form: inviscid runs only");
-    // the tile's faces (its cells' interior faces): g.tface[g.toff[tile] ..)
-    const int f0 = g.toff[tile], nft = g.toff[tile + 1] - f0;
-    for (int k = t; k < nft; k += blockDim.x) {
-      const int f = g.tface[f0 + k];
-      const int sl = g.fsl[f];
-      TS fl[NV];
-      conv_flux<NV, MIX>(kp, g, s, f, g.fe0[f], g.fe1[f], sl & 3, sl >> 2, fl);
-#pragma unroll
-      for (int kk = 0; kk < NV; kk++) sfl[k * NV + kk] = fl[kk];
-    }
-    __syncthreads();
-  }
   double R[NV];
 #pragma unroll
   for (int kk = 0; kk < NV; kk++) R[kk] = 0.0;
@@ -633,19 +566,17 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_update(KP kp, Geo g, St s, int fl
   if (active) {
     // all face indices, then all face fluxes, then the sums in slot order:
     // two memory round trips instead of one pair per slot (slots without
-    // a face read face 0 and add nothing).  Tile form: the slot's face as
-    // +-(its place in the tile's list + 1), with the face id's sign.
+    // a face read face 0 and add nothing).
     int cf[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) cf[j] = TILE > 0 ? (int)g.tsl[j * nc + i] : g.cface[j * nc + i];
+    for (int j = 0; j < 4; j++) cf[j] = g.cface[j * nc + i];
     double fv[4][NV];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const int f = cf[j], q = f > 0 ? f - 1 : (f < 0 ? -f - 1 : 0);
 #pragma unroll
       for (int kk = 0; kk < NV; kk++) {
-        if (TILE > 0) fv[j][kk] = (double)sfl[q * NV + kk];
-        else fv[j][kk] = MIX ? (double)s.fflux32[(size_t)q * NV + kk] : s.fflux[(size_t)q * NV + kk];
+        fv[j][kk] = MIX ? (double)s.fflux32[(size_t)q * NV + kk] : s.fflux[(size_t)q * NV + kk];
       }
     }
 #pragma unroll
@@ -768,30 +699,24 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_update(KP kp, Geo g, St s, int fl
       const double dt = (flags & F_CUR_LOCAL) ? dtl[i] : dtg[0];
       const double om = g.omega[i];
       double unew[NV];
+      const Den<double> dom(om);
 #pragma unroll
-      for (int kk = 0; kk < NV; kk++) unew[kk] = hold ? un0[kk] : un[kk] - dt * sigma * rk_a * R[kk] / om;
+      for (int kk = 0; kk < NV; kk++) unew[kk] = hold ? un0[kk] : un[kk] - dom(dt * sigma * rk_a * R[kk]);
       if (flags & F_LAST) {
         // U^{n+1} stays unclamped until the next residual, as in the reference
         dt_next = cell_dt<NV>(kp, unew, om, g.dsxm[i], g.dsym[i]);
         if (flags & F_NEXT_LOCAL) dtl[i] = cfl * dt_next;
-#pragma unroll
-        for (int kk = 0; kk < NV; kk++) Uout[kk * nc + i] = unew[kk];
-        if (!PU) prim_point<NV>(kp, unew, p);
-      } else if (PU) {
-        // the next stage recovers its primitives from this state; its clamps
-        // only ever reach the primitives (the reference's RK overwrites the
-        // clamped intermediate state), so it is stored as computed
-#pragma unroll
-        for (int kk = 0; kk < NV; kk++) Uout[kk * nc + i] = unew[kk];
-      } else {
-        prim_point<NV>(kp, unew, p);
+      }
+      // PO: the next stage reads the primitives r u v p only (its gradients
+      // and fluxes take nothing else of an inviscid state), so a stage
+      // before the last stores those instead of the state
+      if (!PO || (flags & F_LAST)) {
 #pragma unroll
         for (int kk = 0; kk < NV; kk++) Uout[kk * nc + i] = unew[kk];
       }
-      if (!PU) {
+      prim_point<NV>(kp, unew, p);
 #pragma unroll
-        for (int m = 0; m < NV + 1; m++) s.P[m * nc + i] = p[m];
-      }
+      for (int m = 0; m < (PO ? 4 : NV + 1); m++) s.P[m * nc + i] = p[m];
     }
   }
   if (!(flags & (F_LAST | F_RES))) return;

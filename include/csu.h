@@ -282,14 +282,14 @@ int  csu_batch_run(csu_dev* dev, double drop, int32_t max_iter, int32_t chunk,
  * first iteration, time every candidate -- workgroup size of the gradient
  * and face kernels (64, 128, 256), of the LU-SGS level launches (64, 128,
  * 256), XCD-contiguous or plain tile order, and for inviscid second-order
- * RK runs the tile form (the face fluxes of each 256-cell tile evaluated
- * into LDS by the update kernel, no face-flux kernel or array) -- over
- * `iters` iterations (the better of two runs) and keep the fastest; the
- * context then continues from the state it had, and later contexts of the
- * same kind of run and mesh-size bucket (log2 of the cell count) in the
- * process take the same choice without timing.  Results do not depend on
- * these choices (an untuned context takes the tile form from 200k cells
- * on).  choice: [4] (block, LU-SGS block, XCD map, tile) or NULL.
+ * RK runs the tile form (each stage one kernel over 256-cell tiles, edge
+ * states and face fluxes kept in LDS) -- over `iters` iterations (the better
+ * of two runs) and keep the fastest; the context then continues from the
+ * state it had, and later contexts of the same kind of run and mesh-size
+ * bucket (log2 of the cell count) in the process take the same choice
+ * without timing.  Results do not depend on these choices (an untuned
+ * context takes the tile form unless its numbering scatters neighbours over
+ * the tiles).  choice: [4] (block, LU-SGS block, XCD map, tile) or NULL.
  * csu_dev_launch_shape reports the shapes in use (returns 1 if tuned). */
 int  csu_dev_autotune(csu_dev* dev, int32_t iters, int32_t* choice);
 int  csu_dev_launch_shape(const csu_dev* dev, int32_t* choice);
