@@ -1257,11 +1257,6 @@ static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, d
     hipLaunchKernelGGL(k_lim1_final<NV>, dim3(d->nsolve), dim3(CSU_BLOCK), 0, d->stream, kp, nblk(nc), nblk(nc),
                        d->geo.sol, d->red, d->st.pref2);
   }
-  if (d->nb > 0) {
-    // ghost states first: the gradients read them
-    Prof p(d, "k_bcflux");
-    hipLaunchKernelGGL(k_bcflux<NV>, dim3(nblk(d->nb)), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo, d->st);
-  }
   {
     Prof p(d, "k_grad");
     if (kp.mixed)
@@ -1269,16 +1264,21 @@ static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, d
                          d->st);
     else if (kp.lsq_ld)
       hipLaunchKernelGGL((k_grad<NV, VISC, true>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo, d->st);
+    else if (d->prm.time_scheme == CSU_TIME_RK && NV == 4)
+      hipLaunchKernelGGL((k_grad<NV, VISC, false, false, NV != 4>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0,
+                         d->stream, kp, d->geo, d->st);
     else
       hipLaunchKernelGGL((k_grad<NV, VISC, false>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo, d->st);
   }
-  if (d->nf > 0) {
+  {
     Prof p(d, "k_flux");
-    if (kp.mixed)
-      hipLaunchKernelGGL((k_flux<NV, VISC, true>), dim3((d->nf + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo,
-                         d->st);
+    const int nfb = (d->nf + d->sblk - 1) / d->sblk, nbb = (d->nb + d->sblk - 1) / d->sblk;
+    const dim3 gf(nfb + nbb), bf(d->sblk);
+    if (nfb + nbb == 0) {
+    } else if (kp.mixed)
+      hipLaunchKernelGGL((k_flux<NV, VISC, true>), gf, bf, 0, d->stream, kp, d->geo, d->st, nfb);
     else
-      hipLaunchKernelGGL((k_flux<NV, VISC>), dim3((d->nf + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo, d->st);
+      hipLaunchKernelGGL((k_flux<NV, VISC>), gf, bf, 0, d->stream, kp, d->geo, d->st, nfb);
   }
   {
     Prof p(d, "k_update");
@@ -1390,14 +1390,13 @@ extern "C" int csu_dev_residual(csu_dev* d, double* R, double* dPx, double* dPy,
 // solverCalcPrimitive(solver, U) (solver.c:1153-1213) on the device state:
 // U clamped in place, P [nc][nv+1] to the host (NULL allowed).
 // solverCalcPrimitive: the cells, then the ghost states of the boundary
-// faces (its boundaryCalcPrimitive calls, solver.c:1215-1218); k_bcflux's
-// boundary fluxes are recomputed by the next stage before they are read.
+// faces (its boundaryCalcPrimitive calls, solver.c:1215-1218).
 template <int NV>
 static int prim_ghost_pass(csu_dev* d) {
   int rc = prim_pass<NV>(d);
   if (rc || d->nb == 0) return rc;
-  Prof p(d, "k_bcflux");
-  hipLaunchKernelGGL(k_bcflux<NV>, dim3(nblk(d->nb)), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->geo, d->st);
+  Prof p(d, "k_ghost");
+  hipLaunchKernelGGL(k_ghost<NV>, dim3(nblk(d->nb)), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->geo, d->st);
   HIPCHK(hipGetLastError());
   return CSU_OK;
 }

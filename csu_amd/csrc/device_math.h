@@ -585,9 +585,7 @@ __device__ __forceinline__ T limiter_v2(T Ui, T Umin, T Umax, T d2, T ee) {
 // use, so one straight-line evaluation with that difference selected gives
 // the same operations per lane without divergent branches (each holding
 // two divisions) in a wavefront.
-// REF: the reference's sequence of roundings (the long double least-squares
-// mode, whose histories match the reference's where one-ulp differences
-// grow); else the FP64 form below.
+// REF: the reference's sequence of roundings; else the FP64 form below.
 template <typename T, bool REF>
 __device__ __forceinline__ T limiter_v2d(T d1max, T d1min, T d2, T ee) {
   const T d1 = d2 > (T)0 ? d1max : d1min;

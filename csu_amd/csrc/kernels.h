@@ -6,7 +6,8 @@
 //                    Venkatakrishnan phi, the reconstructed state at every
 //                    edge; viscous: T gradient, boundary viscous fluxes, wall
 //                    friction (all need only the cell's own fresh data)
-//   k_flux    faces  Riemann flux of the two edge states (+ viscous face flux)
+//   k_flux    faces  Riemann flux of the two edge states (+ viscous face flux);
+//                    boundary faces: their convective flux
 //   k_update  cells  per-cell sums in the reference's order, then the RK
 //                    update fused with the next stage's primitive recovery;
 //                    on the last stage also the next time step and the
@@ -69,7 +70,10 @@ __device__ __forceinline__ void lsq_grad(int np, const double* dx, const double*
 // (boundary.c:695-742).
 // MIX (mixed precision): gradients, limiter and reconstruction in FP32 from
 // FP64 differences; edge states stored in FP32.
-template <int NV, bool VISC, bool LD, bool MIX = false>
+// REFL: the limiter function in the reference's sequence of roundings.  The
+// implicit schemes keep it: DPLUR's finite differences (h = 1e-6) and the SST
+// source terms turn one-ulp differences of the gradients into 1e-9.
+template <int NV, bool VISC, bool LD, bool MIX = false, bool REFL = true>
 __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   using TF = typename std::conditional<MIX, float, double>::type;
   constexpr int NS = NV + 1;
@@ -82,12 +86,27 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
     s.pref2 += 6 * sid;
   }
   if (i >= kp.cend) return;
-  const int np = g.cnp[i];
+  const int np = g.cnp[i], bm = g.bmask[i];
   const double x0 = g.xc[i], y0 = g.yc[i];
   double Pi[NS];
 #pragma unroll
   for (int m = 0; m < NS; m++) Pi[m] = s.P[m * nc + i];
-  // neighbours: cells, or the ghost states of boundary faces (k_bcflux)
+  // Ghost states of the cell's boundary faces (few cells have one): written
+  // out for k_flux, and read back below as any neighbour's state.  One
+  // rolled loop before the gathers: unrolled among them it doubled the
+  // registers.
+  if (bm) {
+#pragma unroll 1
+    for (int j = 0; j < np; j++) {
+      if (!((bm >> j) & 1)) continue;
+      const int q = -1 - g.cnbr[j * nc + i];
+      double Pg[NS];
+      ghost_state<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, NV == 6 ? g.wdist[i] : 0.0, Pg);
+#pragma unroll
+      for (int m = 0; m < NS; m++) s.Pb[m * nb + q] = Pg[m];
+    }
+  }
+  // neighbours: cells, or the ghost states of boundary faces
   double dx[4], dy[4];
   int gb[4], nbr[4];
 #pragma unroll
@@ -245,7 +264,7 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           if (j >= np) break;
-          const TF p0 = limiter_v2d<TF, LD>(d1max, d1min, d2[j], (TF)pref2);
+          const TF p0 = limiter_v2d<TF, REFL>(d1max, d1min, d2[j], (TF)pref2);
           ph = (j == 0) ? p0 : fmin(ph, p0);
         }
       }
@@ -430,12 +449,47 @@ __device__ __forceinline__ void conv_flux(const KP& kp, const Geo& g, const St& 
   for (int kk = 0; kk < NV; kk++) out[kk] = fl[kk] * dS;
 }
 
+// A workgroup's boundary faces from q0 on, from their cells' primitives: the
+// ghost state into Pb (boundaryCalcPrimitive, boundary.c:514-693), or the
+// convective flux from the first-order state, boundaryCalc / _sa / _sst
+// (boundary.c:143-446): f*dS, or 0 when dS = 0.
+template <int NV>
+__device__ __forceinline__ void bc_face(KP kp, const Geo& g, const St& s, int q0, bool ghost) {
+  const int q = q0 + threadIdx.x;
+  const int nc = kp.nc, nb = kp.nb;
+  if (g.sol) solve_kp(kp, g.sol[solve_of(g.bsolk, q0)]);
+  if (q >= kp.bend) return;
+  const int i = g.be0[q];
+  double Pi[NV + 1];
+#pragma unroll
+  for (int m = 0; m < NV + 1; m++) Pi[m] = s.P[m * nc + i];
+  if (ghost) {
+    double Pg[NV + 1];
+    ghost_state<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, NV == 6 ? g.wdist[i] : 0.0, Pg);
+#pragma unroll
+    for (int m = 0; m < NV + 1; m++) s.Pb[m * nb + q] = Pg[m];
+    return;
+  }
+  double R[NV];
+#pragma unroll
+  for (int kk = 0; kk < NV; kk++) R[kk] = 0.0;
+  bc_flux<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, R);
+#pragma unroll
+  for (int kk = 0; kk < NV; kk++) s.bflux[kk * nb + q] = R[kk];
+}
+
 // Interior face flux, reference inter() face loop (solver.c:550-644), and
 // for viscous runs the laminar face flux (laminar.c:17-75).
 // MIX: the convective flux in FP32 from FP32 edge states, stored in FP32.
+// The workgroups from nfb on take the boundary faces (bc_face): as a launch
+// of its own that work cost 4-5 us per stage, of which it ran under one.
 template <int NV, bool VISC, bool MIX = false>
-__global__ __launch_bounds__(CSU_BLOCK) void k_flux(KP kp, Geo g, St s) {
-  const int e0f = (kp.xcd ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x) * blockDim.x;
+__global__ __launch_bounds__(CSU_BLOCK) void k_flux(KP kp, Geo g, St s, int nfb) {
+  if ((int)blockIdx.x >= nfb) {
+    bc_face<NV>(kp, g, s, (blockIdx.x - nfb) * blockDim.x, false);
+    return;
+  }
+  const int e0f = (kp.xcd ? xcd_tile(blockIdx.x, nfb) : (int)blockIdx.x) * blockDim.x;
   const int f = e0f + threadIdx.x;
   const int nc = kp.nc, nf = kp.nf;
   if (g.sol) solve_kp(kp, g.sol[solve_of(g.fsolk, e0f)]);
@@ -507,28 +561,12 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_flux(KP kp, Geo g, St s) {
   }
 }
 
-// Per boundary face, from its cell's primitives: the ghost state
-// (boundaryCalcPrimitive, boundary.c:514-693) into Pb, and the convective
-// flux from the first-order state, boundaryCalc / _sa / _sst
-// (boundary.c:143-446): f*dS, or 0 when dS = 0.
+// Ghost states of every boundary face from its cell's primitives
+// (boundaryCalcPrimitive), for the entry point that recomputes the
+// primitives outside an iteration.
 template <int NV>
-__global__ __launch_bounds__(CSU_BLOCK) void k_bcflux(KP kp, Geo g, St s) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  const int nc = kp.nc, nb = kp.nb;
-  if (g.sol) solve_kp(kp, g.sol[solve_of(g.bsolk, blockIdx.x * blockDim.x)]);
-  if (q >= kp.bend) return;
-  const int i = g.be0[q];
-  double Pi[NV + 1], R[NV], Pg[NV + 1];
-#pragma unroll
-  for (int m = 0; m < NV + 1; m++) Pi[m] = s.P[m * nc + i];
-  ghost_state<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, NV == 6 ? g.wdist[i] : 0.0, Pg);
-#pragma unroll
-  for (int m = 0; m < NV + 1; m++) s.Pb[m * nb + q] = Pg[m];
-#pragma unroll
-  for (int kk = 0; kk < NV; kk++) R[kk] = 0.0;
-  bc_flux<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, R);
-#pragma unroll
-  for (int kk = 0; kk < NV; kk++) s.bflux[kk * nb + q] = R[kk];
+__global__ __launch_bounds__(CSU_BLOCK) void k_ghost(KP kp, Geo g, St s) {
+  bc_face<NV>(kp, g, s, blockIdx.x * blockDim.x, true);
 }
 
 // Residual sums + RK update.  Order of the per-cell sums follows
@@ -585,7 +623,7 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_update(KP kp, Geo g, St s, int fl
 #pragma unroll
       for (int kk = 0; kk < NV; kk++) R[kk] = f > 0 ? R[kk] + fv[j][kk] : (f < 0 ? R[kk] - fv[j][kk] : R[kk]);
     }
-    // boundary fluxes (k_bcflux), in the cell's slot order = marker order
+    // boundary fluxes (k_flux), in the cell's slot order = marker order
     int gbq[4];
     const int bm = g.bmask[i];  // most cells have no boundary face: skip their neighbour list
 #pragma unroll
