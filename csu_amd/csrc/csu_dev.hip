@@ -98,7 +98,7 @@ struct csu_dev {
   int *cellsL, *cellsU;        // cells sorted by level
   // iteration graphs (captured once, replayed): RK keyed by local time
   // step x which buffer holds U; implicit keyed by nothing
-  int* hctr;                   // device iteration counter: slot of res/coef history
+  int* hctr;                   // device iteration counter (slot of res/coef history), k_tail's finished workgroups
   hipGraphExec_t gexec[4];
   double *gU[4], *gP[4];       // d->U, d->st.P at capture
   double* Ubase;               // the buffer U starts in (graph parity key)
@@ -838,7 +838,9 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     kp.sst_g1 = 0.075 / 0.09 - 0.5 * kap * kap / sqrt(0.09);
     kp.sst_g2 = 0.0828 / 0.09 - 0.856 * kap * kap / sqrt(0.09);
   }
-  kp.limK = p->lim_k; kp.volmax = H.volmax; kp.pr = p->pr; kp.pr_t = p->pr_t; kp.wimp = p->wimp;
+  kp.limK = p->lim_k; kp.volmax = H.volmax; kp.pr = p->pr; kp.pr_t = p->pr_t;
+  kp.rpr = 1.0 / p->pr; kp.rpr_t = 1.0 / p->pr_t;
+  kp.wimp = p->wimp;
   for (int k = 0; k < 7; k++) kp.pin[k] = p->pin[k];
   kp.gas.gamma = p->gamma; kp.gas.R = p->gas_r;
   kp.gas.Cp = kp.gas.gamma * kp.gas.R / (kp.gas.gamma - 1);
@@ -1025,8 +1027,8 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     if ((rc = build(H.levL, d->lvlL, &d->cellsL)) || (rc = build(H.levU, d->lvlU, &d->cellsU))) return rc;
   }
   d->Ubase = d->U;
-  if ((rc = dalloc(d, &d->hctr, 1)) || (rc = dalloc(d, &d->tstate, 4))) return rc;
-  HIPCHK(hipMemsetAsync(d->hctr, 0, sizeof(int), d->stream));
+  if ((rc = dalloc(d, &d->hctr, 2)) || (rc = dalloc(d, &d->tstate, 4))) return rc;
+  HIPCHK(hipMemsetAsync(d->hctr, 0, 2 * sizeof(int), d->stream));
   // free-stream initial state (solverInitU); a batch's padding cells take
   // their solve's, so that every value in the arrays stays finite
   std::vector<double> U0(nvc);
@@ -1246,9 +1248,10 @@ extern "C" int csu_dev_kernel_times(csu_dev* d, const char** names, double* avg_
 // ---------------------------------------------------------------------------
 // orchestration
 // ---------------------------------------------------------------------------
-// One residual evaluation (solverCalcR) with P valid, then the fused update.
+// One residual evaluation (solverCalcR) with P valid (ghosts: and the ghost
+// states, k_prim's), then the fused update.
 template <int NV, bool VISC>
-static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, double* Uout) {
+static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, double* Uout, bool ghosts) {
   const KP& kp = d->kp;
   const int nc = d->nc;
   if (kp.order == 2 && kp.limiter == 1) {
@@ -1259,16 +1262,14 @@ static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, d
   }
   {
     Prof p(d, "k_grad");
-    if (kp.mixed)
-      hipLaunchKernelGGL((k_grad<NV, VISC, false, true>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo,
-                         d->st);
-    else if (kp.lsq_ld)
-      hipLaunchKernelGGL((k_grad<NV, VISC, true>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo, d->st);
+    const dim3 gg((nc + d->sblk - 1) / d->sblk), bg(d->sblk);
+    const bool ex = !ghosts;
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, gg, bg, 0, d->stream, kp, d->geo, d->st); };
+    if (kp.mixed) ex ? go(k_grad<NV, VISC, false, true, true>) : go(k_grad<NV, VISC, false, true, false>);
+    else if (kp.lsq_ld) ex ? go(k_grad<NV, VISC, true, false, true>) : go(k_grad<NV, VISC, true, false, false>);
     else if (d->prm.time_scheme == CSU_TIME_RK && NV == 4)
-      hipLaunchKernelGGL((k_grad<NV, VISC, false, false, NV != 4>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0,
-                         d->stream, kp, d->geo, d->st);
-    else
-      hipLaunchKernelGGL((k_grad<NV, VISC, false>), dim3((nc + d->sblk - 1) / d->sblk), dim3(d->sblk), 0, d->stream, kp, d->geo, d->st);
+      ex ? go(k_grad<NV, VISC, false, false, true, NV != 4>) : go(k_grad<NV, VISC, false, false, false, NV != 4>);
+    else ex ? go(k_grad<NV, VISC, false, false, true>) : go(k_grad<NV, VISC, false, false, false>);
   }
   {
     Prof p(d, "k_flux");
@@ -1331,8 +1332,8 @@ static int tile_stage(csu_dev* d, int flags, double sigma, double rk_a) {
 template <int NV>
 static int prim_pass(csu_dev* d) {
   Prof p(d, "k_prim");
-  hipLaunchKernelGGL(k_prim<NV>, dim3(nblk(d->nc)), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->U, d->st.P, d->geo.sol,
-                     d->geo.csolk);
+  hipLaunchKernelGGL(k_prim<NV>, dim3(nblk(d->nc)), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->geo, d->U, d->st.P,
+                     d->st.Pb);
   HIPCHK(hipGetLastError());
   return CSU_OK;
 }
@@ -1341,7 +1342,7 @@ template <int NV, bool VISC>
 static int residual_t(csu_dev* d) {
   int rc = prim_pass<NV>(d);
   d->kp.store_grad = 1;  // the caller may ask for dPx, dPy, phi
-  if (!rc) rc = stage<NV, VISC>(d, F_STORE_R, 0.0, 0.0, nullptr, nullptr);
+  if (!rc) rc = stage<NV, VISC>(d, F_STORE_R, 0.0, 0.0, nullptr, nullptr, true);
   d->kp.store_grad = 0;
   d->fresh = 1;
   return rc;
@@ -1389,22 +1390,10 @@ extern "C" int csu_dev_residual(csu_dev* d, double* R, double* dPx, double* dPy,
 
 // solverCalcPrimitive(solver, U) (solver.c:1153-1213) on the device state:
 // U clamped in place, P [nc][nv+1] to the host (NULL allowed).
-// solverCalcPrimitive: the cells, then the ghost states of the boundary
-// faces (its boundaryCalcPrimitive calls, solver.c:1215-1218).
-template <int NV>
-static int prim_ghost_pass(csu_dev* d) {
-  int rc = prim_pass<NV>(d);
-  if (rc || d->nb == 0) return rc;
-  Prof p(d, "k_ghost");
-  hipLaunchKernelGGL(k_ghost<NV>, dim3(nblk(d->nb)), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->geo, d->st);
-  HIPCHK(hipGetLastError());
-  return CSU_OK;
-}
-
 extern "C" int csu_dev_primitives(csu_dev* d, double* P) {
   if (!d) return set_err(CSU_ERR_ARG, "null argument");
   if (d->nsolve > 1) return set_err(CSU_ERR_UNSUPPORTED, "%s: not on a batch context (use csu_batch_*)", __func__);
-  int rc = d->nv == 6 ? prim_ghost_pass<6>(d) : d->nv == 5 ? prim_ghost_pass<5>(d) : prim_ghost_pass<4>(d);
+  int rc = d->nv == 6 ? prim_pass<6>(d) : d->nv == 5 ? prim_pass<5>(d) : prim_pass<4>(d);
   if (rc) return rc;
   d->fresh = 1;
   if (P) {
@@ -1426,22 +1415,18 @@ static const double RK4[] = {0.0833, 0.2069, 0.4265, 1.0};
 static const double RK5[] = {0.0533, 0.1263, 0.2375, 0.4414, 1.0};
 
 // Residual norms and force coefficients of the iteration just done, into
-// the history slot the device counter names (k_forces advances it).
+// the history slot the device counter names, and with dt the global time
+// step from the stage's (or the implicit diagonal's) block minima.
 template <int NV>
-static void iteration_tail(csu_dev* d, int nblocks_cells) {
-  {
-    Prof p(d, "k_res");
-    hipLaunchKernelGGL(k_res_final<NV>, dim3(d->nsolve), dim3(RES_THREADS), 0, d->stream, d->nc, nblocks_cells,
-                       nblocks_cells, d->geo.sol, d->red,
-                       d->res_hist, d->hist_cap, (const int*)d->hctr);
-  }
-  {
-    Prof p(d, "k_forces");
-    hipLaunchKernelGGL(k_forces, dim3(d->nsolve), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->nwall, d->wall, d->st.Pb,
-                       d->st.wfric, d->geo.bdsx, d->geo.bdsy, d->prm.sref, d->visc, d->coef_hist, d->hist_cap,
-                       d->hctr, d->geo.sol);
-  }
-  if (d->geo.sol) hipLaunchKernelGGL(k_next_slot, dim3(1), dim3(64), 0, d->stream, d->hctr);
+static void iteration_tail(csu_dev* d, bool dt) {
+  Prof p(d, "k_tail");
+  TailP a;
+  a.nc = d->nc; a.nblocks = nblk(d->nc); a.nsolve = d->nsolve; a.nwall = d->nwall; a.cap = d->hist_cap;
+  a.visc = d->visc; a.cfl = d->prm.cfl; a.sref = d->prm.sref; a.sol = d->geo.sol;
+  a.red = d->red; a.red_dt = d->red + (size_t)NV * d->nred; a.wall = d->wall; a.Pb = d->st.Pb; a.wfric = d->st.wfric;
+  a.bdsx = d->geo.bdsx; a.bdsy = d->geo.bdsy; a.res = d->res_hist; a.coef = d->coef_hist; a.dtg = d->dtg;
+  a.ctr = d->hctr; a.done = d->hctr + 1;
+  hipLaunchKernelGGL(k_tail<NV>, dim3(d->nsolve * (dt ? 3 : 2)), dim3(RES_THREADS), 0, d->stream, d->kp, a);
 }
 
 static int is_local(const csu_dev* d, int it) {
@@ -1507,14 +1492,11 @@ static int rk_iteration(csu_dev* d, int it_index) {
       if (rc) return rc;
       continue;
     }
-    int rc = stage<NV, VISC>(d, flags, sigma, a[s], d->U, d->Uaux);
+    int rc = stage<NV, VISC>(d, flags, sigma, a[s], d->U, d->Uaux, s == 0 && first_flags == 0);
     if (rc) return rc;
   }
   std::swap(d->U, d->Uaux);
-  if (!next_local)
-    hipLaunchKernelGGL(k_dt_final, dim3(d->nsolve), dim3(CSU_BLOCK), 0, d->stream, nblk(nc), d->prm.cfl, red_dt,
-                       d->dtg, d->geo.sol);
-  iteration_tail<NV>(d, nblk(nc));
+  iteration_tail<NV>(d, !next_local);
   HIPCHK(hipGetLastError());
   return CSU_OK;
 }
@@ -1554,15 +1536,14 @@ static int implicit_iteration(csu_dev* d) {
   const int nc = d->nc, nb = nblk(nc);
   double* red_min = d->red + (size_t)NV * d->nred;
   int rc = prim_pass<NV>(d);
-  if (!rc) rc = stage<NV, VISC>(d, F_STORE_R | F_RES, 0.0, 0.0, nullptr, nullptr);
+  if (!rc) rc = stage<NV, VISC>(d, F_STORE_R | F_RES, 0.0, 0.0, nullptr, nullptr, true);
   if (rc) return rc;
   {
     Prof p(d, "k_impD");
     hipLaunchKernelGGL((k_impD<NV, VISC>), dim3(nb), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo, d->st, d->prm.wimp,
                        d->Dp, red_min, d->caux);
-    hipLaunchKernelGGL(k_dt_final, dim3(d->nsolve), dim3(CSU_BLOCK), 0, d->stream, nb, d->prm.cfl, red_min, d->dtg,
-                       d->geo.sol);
   }
+  iteration_tail<NV>(d, true);
   if (d->prm.time_scheme == CSU_TIME_LUSGS) {
     Prof p(d, "k_lusgs");
     // a level holds a fraction of the cells (a colour of the renumbered
@@ -1594,7 +1575,6 @@ static int implicit_iteration(csu_dev* d) {
     hipLaunchKernelGGL(k_jac_base, dim3((d->nsolve + 63) / 64), dim3(64), 0, d->stream, d->jstate,
                        (const double*)d->jred, d->prm.nlinear, nb, d->geo.sol, d->nsolve);
   }
-  iteration_tail<NV>(d, nb);
   HIPCHK(hipGetLastError());
   return CSU_OK;
 }
@@ -1673,7 +1653,7 @@ static int tune_reset(csu_dev* d, const double* saved) {
   graphs_drop(d);
   HIPCHK(hipMemcpyAsync(d->U, saved, nvc * sizeof(double), hipMemcpyDeviceToDevice, d->stream));
   HIPCHK(hipMemcpyAsync(d->Uaux, saved, nvc * sizeof(double), hipMemcpyDeviceToDevice, d->stream));
-  HIPCHK(hipMemsetAsync(d->hctr, 0, sizeof(int), d->stream));
+  HIPCHK(hipMemsetAsync(d->hctr, 0, 2 * sizeof(int), d->stream));
   if (d->dW0) HIPCHK(hipMemsetAsync(d->dW0, 0, nvc * sizeof(double), d->stream));
   if (d->dW1) HIPCHK(hipMemsetAsync(d->dW1, 0, nvc * sizeof(double), d->stream));
   if (d->A) HIPCHK(hipMemsetAsync(d->A, 0, (size_t)4 * d->nv * d->nv * d->nc * sizeof(double), d->stream));

@@ -31,6 +31,7 @@ struct KP {
   int sst_trans;  // SST: the transition variant's eddy viscosity and sources (sstTrans.c)
   int sa_cc;      // SA: the saCC.c form, with density-gradient terms in the nu~ flux and source
   double rlim, pout, twall, efix, minf, limK, volmax, pr, pr_t, wimp;
+  double rpr, rpr_t;  // 1/pr, 1/pr_t, rounded (Den)
   double sst_owall, sst_g1, sst_g2;  // SST: oWallFactor, blended gamma constants (sst.c:18-38)
   double pin[7];
   GasD gas;

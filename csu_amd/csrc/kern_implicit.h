@@ -74,11 +74,13 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_impD(KP kp, Geo g, St s, double w
       double v = (Pa[2] + Pb[j][2]) * 0.5;
       double T = (Pa[3] + Pb[j][3]) * 0.5;
       double c = gas_T2c<double>(kp.gas, T);
-      double nx = dSx / dS, ny = dSy / dS;
+      const Den<double> dl(dS);
+      double nx = dl(dSx), ny = dl(dSy);
       Lc += (fabs(nx * u + ny * v) + c) * dS;
       if (VISC) {
         double mi = sutherland(T);
-        double mt = NV == 4 ? mi / kp.pr : mi / kp.pr + s.miT[fi] / kp.pr_t;
+        const double mp = Den<double>(kp.pr, kp.rpr)(mi);
+        double mt = NV == 4 ? mp : mp + Den<double>(kp.pr_t, kp.rpr_t)(s.miT[fi]);
         Lv += fmax(4 / (3 * r), gamma_of(kp.gas, T) / r) * mt * dS * dS;
       }
     }
@@ -119,6 +121,12 @@ __device__ __forceinline__ double diag(const double* Dp, const double* omega, co
   return Dp[i] + omega[i] / dtg[sid];
 }
 
+// x / Cv(T): the ideal gas's Cv inverted once on the host
+__device__ __forceinline__ double over_cv(const GasD& g, double x, double T) {
+  if (!g.tp) return Den<double>(g.Cv, g.rCv)(x);
+  return x / gas_T2Cv<double>(g, T);
+}
+
 // implicitCalcDeltaFlux_sa (implicit.c:495-553): with the positivity clamps
 __device__ __forceinline__ void delta_flux_sa(const KP& kp, const double* Pj, const double* d, double nx, double ny,
                                               double* dF) {
@@ -134,10 +142,11 @@ __device__ __forceinline__ void delta_flux_sa(const KP& kp, const double* Pj, co
   rho = U[0];
   rho = fmax(rho, kp.rlim);
   U[0] = rho;
-  u = U[1] / rho; v = U[2] / rho; E = U[3] / rho;
+  const Den<double> dr(rho);
+  u = dr(U[1]); v = dr(U[2]); E = dr(U[3]);
   double e1 = E - (u * u + v * v) * 0.5;
   e1 = fmax(e1, 7.176325e+02);
-  T = T + (e1 - e0) / gas_T2Cv<double>(kp.gas, T);
+  T = T + over_cv(kp.gas, e1 - e0, T);
   if (T < 1) {
     T = 1;
     e1 = gas_T2e<double>(kp.gas, T);
@@ -145,10 +154,10 @@ __device__ __forceinline__ void delta_flux_sa(const KP& kp, const double* Pj, co
     U[3] = rho * E;
   }
   p = kp.gas.R * T * rho;
-  n = U[4] / rho;
+  n = dr(U[4]);
   n = fmax(n, 0.0);
   U[4] = rho * n;
-  V = (nx * U[1] + ny * U[2]) / U[0];
+  V = dr(nx * U[1] + ny * U[2]);
   dF[0] = U[0] * V - F0[0];
   dF[1] = (U[1] * V + nx * p) - F0[1];
   dF[2] = (U[2] * V + ny * p) - F0[2];
@@ -170,15 +179,16 @@ __device__ __forceinline__ void delta_flux_sst(const KP& kp, const double* Pj, c
   for (int q = 0; q < 6; q++) U[q] = U[q] + d[q];
   rho = fmax(U[0], kp.rlim);
   U[0] = rho;
-  u = U[1] / rho; v = U[2] / rho;
-  k = U[4] / rho;
+  const Den<double> dr(rho);
+  u = dr(U[1]); v = dr(U[2]);
+  k = dr(U[4]);
   if (k < 1e-14) { k = 1e-14; U[4] = rho * k; }
-  om = U[5] / rho;
+  om = dr(U[5]);
   if (om < 0.0) { om = 0.0; U[5] = rho * om; }
-  E = U[3] / rho;
+  E = dr(U[3]);
   double e1 = E - (u * u + v * v) * 0.5 - k;
   e1 = fmax(e1, 7.176325e+02);
-  T = T + (e1 - e0) / gas_T2Cv<double>(kp.gas, T);
+  T = T + over_cv(kp.gas, e1 - e0, T);
   if (T < 1) {
     T = 1;
     e1 = gas_T2e<double>(kp.gas, T);
@@ -186,7 +196,7 @@ __device__ __forceinline__ void delta_flux_sst(const KP& kp, const double* Pj, c
     U[3] = rho * E;
   }
   p = kp.gas.R * T * rho;
-  V = (nx * U[1] + ny * U[2]) / U[0];
+  V = dr(nx * U[1] + ny * U[2]);
   dF[0] = U[0] * V - F0[0];
   dF[1] = (U[1] * V + nx * p) - F0[1];
   dF[2] = (U[2] * V + ny * p) - F0[2];
@@ -216,11 +226,13 @@ __device__ __forceinline__ void delta_flux(const KP& kp, const double* Pj, const
   double F0[4] = {U[0] * V, U[1] * V + nx * p, U[2] * V + ny * p, (U[3] + p) * V};
 #pragma unroll
   for (int k = 0; k < 4; k++) U[k] = U[k] + d[k];
-  rho = U[0]; u = U[1] / rho; v = U[2] / rho; E = U[3] / rho;
+  rho = U[0];
+  const Den<double> dr(rho);
+  u = dr(U[1]); v = dr(U[2]); E = dr(U[3]);
   double e1 = E - 0.5 * (u * u + v * v);
-  T = T + (e1 - e0) / gas_T2Cv<double>(kp.gas, T);
+  T = T + over_cv(kp.gas, e1 - e0, T);
   p = kp.gas.R * T * rho;
-  V = (nx * U[1] + ny * U[2]) / U[0];
+  V = dr(nx * U[1] + ny * U[2]);
   dF[0] = U[0] * V - F0[0];
   dF[1] = (U[1] * V + nx * p) - F0[1];
   dF[2] = (U[2] * V + ny * p) - F0[2];
@@ -320,7 +332,7 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_lusgs(KP kp, Geo g, St s, const i
     double ra = kp.wimp * (fabs(nx * Pj[1] + ny * Pj[2]) + c) * dS;
     if (NV >= 5) {
       // implicitFunc_sa / _sst (implicit.c:555-595, 1120-1161)
-      ra += caux[nc + nb] * (caux[2 * nc + nb] + s.miT[fi] / kp.pr_t) * dS / ddj[j];
+      ra += caux[nc + nb] * (caux[2 * nc + nb] + Den<double>(kp.pr_t, kp.rpr_t)(s.miT[fi])) * dS / ddj[j];
     } else if (VISC && kp.laminar) {
       ra += caux[nc + nb] * caux[2 * nc + nb] * dS / ddj[j];
     }
@@ -328,15 +340,16 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_lusgs(KP kp, Geo g, St s, const i
     for (int k = 0; k < NV; k++) acc[k] -= 0.5 * (dF[k] * dS - ra * d[k]);
   }
   double out[NV];
+  const Den<double> dD(D);
 #pragma unroll
-  for (int k = 0; k < NV; k++) out[k] = acc[k] / D;
+  for (int k = 0; k < NV; k++) out[k] = dD(acc[k]);
   if (NV == 6) {
     // SST: k-omega block with the source Jacobians, Cramer's rule
     // (implicit.c:326-351, 447-472).  The reference divides by a long double
     // determinant that holds a double value; the quotient here is the
     // correctly rounded double one.
     constexpr int K = NV > 4 ? 4 : 0, O = NV > 5 ? 5 : 0;
-    const double x0 = acc[0] / D;
+    const double x0 = out[0];
     const double A = acc[K] + s.dq[i] * x0;
     const double B = acc[O] + s.dq[3 * nc + i] * x0;
     const double a = D - s.dq[nc + i], b = -s.dq[2 * nc + i], c = -s.dq[4 * nc + i], dd = D - s.dq[5 * nc + i];

@@ -22,17 +22,50 @@ namespace csu {
 
 enum { F_RK = 1, F_CLAMP_UN = 2, F_LAST = 4, F_NEXT_LOCAL = 8, F_STORE_R = 16, F_CUR_LOCAL = 32, F_RES = 64 };
 
+// Ghost states of cell i's boundary faces (bm: its boundary slots) from its
+// primitives, into Pb.
+template <int NV>
+__device__ __forceinline__ void cell_ghosts(const KP& kp, const Geo& g, int i, int bm, const double* Pi,
+                                            double* Pb) {
+  const int nc = kp.nc, nb = kp.nb;
+#pragma unroll 1
+  for (int j = 0; j < 4; j++) {
+    if (!((bm >> j) & 1)) continue;
+    const int q = -1 - g.cnbr[j * nc + i];
+    double Pg[NV + 1];
+    ghost_state<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, NV == 6 ? g.wdist[i] : 0.0, Pg);
+#pragma unroll
+    for (int m = 0; m < NV + 1; m++) Pb[m * nb + q] = Pg[m];
+  }
+}
+
 // Standalone primitive pass (first stage after the state was set from the
 // host).  Clamped values are written back to U, as the reference does.
 // Batch: the cells of a held solve keep their state (a batch's padding
 // cells hold their solve's free stream and are converted like the rest).
+// Also the ghost states of the boundary faces.
 template <int NV>
-__global__ __launch_bounds__(CSU_BLOCK) void k_prim(KP kp, double* __restrict__ U, double* __restrict__ P,
-                                                    const SolveP* __restrict__ sol, const int* __restrict__ csolk) {
+__global__ __launch_bounds__(CSU_BLOCK) void k_prim(KP kp, Geo g, double* __restrict__ U, double* __restrict__ P,
+                                                    double* __restrict__ Pb) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int nc = kp.nc;
   if (i >= nc) return;
-  if (sol && !sol[solve_of(csolk, blockIdx.x * blockDim.x)].active) return;
+  const int bm = g.bmask[i];
+  bool held = false;
+  if (g.sol) {
+    const SolveP& q = g.sol[solve_of(g.csolk, blockIdx.x * blockDim.x)];
+    solve_kp(kp, q);
+    held = !q.active;
+  }
+  if (held) {  // the state stays as it is, and so do its primitives
+    if (bm) {
+      double p[NV + 1];
+#pragma unroll
+      for (int m = 0; m < NV + 1; m++) p[m] = P[m * nc + i];
+      cell_ghosts<NV>(kp, g, i, bm, p, Pb);
+    }
+    return;
+  }
   double u[NV], u0[NV], p[NV + 1];
 #pragma unroll
   for (int k = 0; k < NV; k++) u0[k] = u[k] = U[k * nc + i];
@@ -42,6 +75,7 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_prim(KP kp, double* __restrict__ 
     if (__double_as_longlong(u[k]) != __double_as_longlong(u0[k])) U[k * nc + i] = u[k];
 #pragma unroll
   for (int m = 0; m < NV + 1; m++) P[m * nc + i] = p[m];
+  if (bm) cell_ghosts<NV>(kp, g, i, bm, p, Pb);
 }
 
 // LSQ gradient of one variable from its differences to the neighbours, with
@@ -73,7 +107,10 @@ __device__ __forceinline__ void lsq_grad(int np, const double* dx, const double*
 // REFL: the limiter function in the reference's sequence of roundings.  The
 // implicit schemes keep it: DPLUR's finite differences (h = 1e-6) and the SST
 // source terms turn one-ulp differences of the gradients into 1e-9.
-template <int NV, bool VISC, bool LD, bool MIX = false, bool REFL = true>
+// GH: a stage not preceded by k_prim (explicit runs), which would have made
+// the ghost states; elsewhere their registers would cost this kernel a
+// wavefront per SIMD (SA, 250k cells: 49 us with them, 43 without).
+template <int NV, bool VISC, bool LD, bool MIX, bool GH, bool REFL = true>
 __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   using TF = typename std::conditional<MIX, float, double>::type;
   constexpr int NS = NV + 1;
@@ -91,21 +128,10 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   double Pi[NS];
 #pragma unroll
   for (int m = 0; m < NS; m++) Pi[m] = s.P[m * nc + i];
-  // Ghost states of the cell's boundary faces (few cells have one): written
-  // out for k_flux, and read back below as any neighbour's state.  One
-  // rolled loop before the gathers: unrolled among them it doubled the
-  // registers.
-  if (bm) {
-#pragma unroll 1
-    for (int j = 0; j < np; j++) {
-      if (!((bm >> j) & 1)) continue;
-      const int q = -1 - g.cnbr[j * nc + i];
-      double Pg[NS];
-      ghost_state<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, NV == 6 ? g.wdist[i] : 0.0, Pg);
-#pragma unroll
-      for (int m = 0; m < NS; m++) s.Pb[m * nb + q] = Pg[m];
-    }
-  }
+  // Ghost states of the cell's boundary faces (few cells have one), read back
+  // below as any neighbour's state.  One rolled loop before the gathers:
+  // unrolled among them it doubled the registers.
+  if (GH && bm) cell_ghosts<NV>(kp, g, i, bm, Pi, s.Pb);
   // neighbours: cells, or the ghost states of boundary faces
   double dx[4], dy[4];
   int gb[4], nbr[4];
@@ -449,12 +475,11 @@ __device__ __forceinline__ void conv_flux(const KP& kp, const Geo& g, const St& 
   for (int kk = 0; kk < NV; kk++) out[kk] = fl[kk] * dS;
 }
 
-// A workgroup's boundary faces from q0 on, from their cells' primitives: the
-// ghost state into Pb (boundaryCalcPrimitive, boundary.c:514-693), or the
-// convective flux from the first-order state, boundaryCalc / _sa / _sst
-// (boundary.c:143-446): f*dS, or 0 when dS = 0.
+// A workgroup's boundary faces from q0 on: the convective flux from the
+// first-order state, boundaryCalc / _sa / _sst (boundary.c:143-446): f*dS, or
+// 0 when dS = 0.
 template <int NV>
-__device__ __forceinline__ void bc_face(KP kp, const Geo& g, const St& s, int q0, bool ghost) {
+__device__ __forceinline__ void bc_face(KP kp, const Geo& g, const St& s, int q0) {
   const int q = q0 + threadIdx.x;
   const int nc = kp.nc, nb = kp.nb;
   if (g.sol) solve_kp(kp, g.sol[solve_of(g.bsolk, q0)]);
@@ -463,13 +488,6 @@ __device__ __forceinline__ void bc_face(KP kp, const Geo& g, const St& s, int q0
   double Pi[NV + 1];
 #pragma unroll
   for (int m = 0; m < NV + 1; m++) Pi[m] = s.P[m * nc + i];
-  if (ghost) {
-    double Pg[NV + 1];
-    ghost_state<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, NV == 6 ? g.wdist[i] : 0.0, Pg);
-#pragma unroll
-    for (int m = 0; m < NV + 1; m++) s.Pb[m * nb + q] = Pg[m];
-    return;
-  }
   double R[NV];
 #pragma unroll
   for (int kk = 0; kk < NV; kk++) R[kk] = 0.0;
@@ -486,7 +504,7 @@ __device__ __forceinline__ void bc_face(KP kp, const Geo& g, const St& s, int q0
 template <int NV, bool VISC, bool MIX = false>
 __global__ __launch_bounds__(CSU_BLOCK) void k_flux(KP kp, Geo g, St s, int nfb) {
   if ((int)blockIdx.x >= nfb) {
-    bc_face<NV>(kp, g, s, (blockIdx.x - nfb) * blockDim.x, false);
+    bc_face<NV>(kp, g, s, (blockIdx.x - nfb) * blockDim.x);
     return;
   }
   const int e0f = (kp.xcd ? xcd_tile(blockIdx.x, nfb) : (int)blockIdx.x) * blockDim.x;
@@ -559,14 +577,6 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_flux(KP kp, Geo g, St s, int nfb)
     for (int k = 0; k < 5; k++) s.vflux[k * nf + f] = F[k];
     s.miT[f] = mi_t;
   }
-}
-
-// Ghost states of every boundary face from its cell's primitives
-// (boundaryCalcPrimitive), for the entry point that recomputes the
-// primitives outside an iteration.
-template <int NV>
-__global__ __launch_bounds__(CSU_BLOCK) void k_ghost(KP kp, Geo g, St s) {
-  bc_face<NV>(kp, g, s, blockIdx.x * blockDim.x, true);
 }
 
 // Residual sums + RK update.  Order of the per-cell sums follows
@@ -841,86 +851,96 @@ __global__ void k_time_clamp(double* __restrict__ ts, double* __restrict__ dtg, 
   ts[3] += 1.0;
 }
 
-// Final level of the residual norm: one block, each thread sums a strided
-// slice of the block partials for all variables at once, then a fixed tree.
+// End of an iteration: the final level of the residual norm, the wall force
+// coefficients Cx_p, Cx_v, Cy_p, Cy_v (solverCalcCoeff3, solver.c:1342-1401;
+// friction per face comes from k_grad) and, where the next step needs one,
+// the global time step (k_dt_final).  One workgroup each and per solve,
+// running beside each other: as three launches they cost 4-5 us apiece.
+// The norm's threads sum strided slices of the block partials (rows of
+// length stride), then a fixed tree; the other two do with the first
+// CSU_BLOCK threads what they did in workgroups of that size.
+// The history slot is ctr % cap: the iteration counter lives on the device
+// so that a captured graph writes each replay's rows to its own slot; the
+// last workgroup to finish (done) advances it.  Batch (sol non-null): a
+// solve's own blocks, wall-list range, free stream and CFL; a slot holds
+// nsolve rows.
 #define RES_THREADS 1024
+struct TailP {
+  int nc, nblocks, nsolve, nwall, cap, visc;
+  double cfl, sref;
+  const SolveP* sol;
+  const double *red, *red_dt;  // red_dt null: no time step
+  const int* wall;
+  const double *Pb, *wfric, *bdsx, *bdsy;
+  double *res, *coef, *dtg;
+  int *ctr, *done;
+};
 template <int NV>
-// res_hist slot = ctr % cap: the iteration counter lives on the device so
-// that a captured iteration graph writes each replay's norms to its own slot.
-// Partial rows have length stride.  Batch (sol non-null): one workgroup per
-// solve, over its own blocks; history slot rows hold gridDim.x solves.
-__global__ __launch_bounds__(RES_THREADS) void k_res_final(int nc, int nblocks, int stride, const SolveP* __restrict__ sol,
-                                                           const double* __restrict__ red,
-                                                           double* __restrict__ res_hist, int cap,
-                                                           const int* __restrict__ ctr) {
-  double* res = res_hist + ((size_t)(ctr[0] % cap) * gridDim.x + blockIdx.x) * NV;
-  if (sol) {
-    const SolveP& q = sol[blockIdx.x];
-    red += q.c0 / CSU_BLOCK;
-    nc = q.c1 - q.c0;
-    nblocks = (nc + CSU_BLOCK - 1) / CSU_BLOCK;
-  }
+__global__ __launch_bounds__(RES_THREADS) void k_tail(KP kp, TailP a) {
   __shared__ double sw[NV][RES_THREADS / 64];
-  const int t = threadIdx.x;
-  double a[NV];
-#pragma unroll
-  for (int kk = 0; kk < NV; kk++) a[kk] = 0.0;
-  for (int b = t; b < nblocks; b += RES_THREADS) {
-#pragma unroll
-    for (int kk = 0; kk < NV; kk++) a[kk] += red[kk * stride + b];
-  }
-  block_reduce<RES_THREADS, NV>(a, sw, RedSum());
-  if (t == 0)
-#pragma unroll
-    for (int kk = 0; kk < NV; kk++) res[kk] = sqrt(a[kk] / nc);
-}
-
-// Wall force coefficients Cx_p, Cx_v, Cy_p, Cy_v, reference solverCalcCoeff3
-// (solver.c:1342-1401); friction per face comes from k_grad.
-// Batch (sol non-null): one workgroup per solve over its wall-list range,
-// its free stream and reference length; the slot counter is then advanced
-// by k_next_slot (a workgroup cannot advance it while others read it).
-__global__ __launch_bounds__(CSU_BLOCK) void k_forces(KP kp, int nwall, const int* __restrict__ wall,
-                                                      const double* __restrict__ Pb, const double* __restrict__ wfric,
-                                                      const double* __restrict__ bdsx, const double* __restrict__ bdsy,
-                                                      double sref, int visc, double* __restrict__ coef_hist, int cap,
-                                                      int* __restrict__ ctr, const SolveP* __restrict__ sol) {
-  double* coef = coef_hist + ((size_t)(ctr[0] % cap) * gridDim.x + blockIdx.x) * 4;
-  if (sol) {
-    const SolveP& q = sol[blockIdx.x];
+  const int t = threadIdx.x, sid = blockIdx.x % a.nsolve, role = blockIdx.x / a.nsolve;
+  const size_t row = (size_t)(a.ctr[0] % a.cap) * a.nsolve + sid;
+  int stride = a.nblocks;
+  if (a.sol) {
+    const SolveP& q = a.sol[sid];
     solve_kp(kp, q);
-    wall += q.w0;
-    nwall = q.w1 - q.w0;
-    sref = q.sref;
+    a.red += q.c0 / CSU_BLOCK;
+    a.red_dt += q.c0 / CSU_BLOCK;
+    a.nc = q.c1 - q.c0;
+    a.nblocks = (a.nc + CSU_BLOCK - 1) / CSU_BLOCK;
+    a.wall += q.w0;
+    a.nwall = q.w1 - q.w0;
+    a.sref = q.sref;
+    a.cfl = q.cfl;
   }
-  __shared__ double sw[4][CSU_BLOCK / 64];
-  int t = threadIdx.x;
-  const double r = kp.pin[0], u = kp.pin[1], v = kp.pin[2], Pinf = kp.pin[3];
-  const double q = 0.5 * r * (u * u + v * v);
-  double ax = 0.0, ay = 0.0, vx = 0.0, vy = 0.0;
-  for (int w = t; w < nwall; w += CSU_BLOCK) {
-    int gq = wall[w];
-    double cp = (Pb[3 * kp.nb + gq] - Pinf) / q;
-    ax += cp * bdsx[gq];
-    ay += cp * bdsy[gq];
-    if (visc) {
-      vx -= wfric[gq] / q;
-      vy -= wfric[kp.nb + gq] / q;
+  if (role == 0) {
+    double v[NV];
+#pragma unroll
+    for (int kk = 0; kk < NV; kk++) v[kk] = 0.0;
+    for (int b = t; b < a.nblocks; b += RES_THREADS) {
+#pragma unroll
+      for (int kk = 0; kk < NV; kk++) v[kk] += a.red[kk * stride + b];
+    }
+    block_reduce<RES_THREADS, NV>(v, sw, RedSum());
+    if (t == 0)
+#pragma unroll
+      for (int kk = 0; kk < NV; kk++) a.res[row * NV + kk] = sqrt(v[kk] / a.nc);
+  } else if (role == 1) {
+    const double r = kp.pin[0], u = kp.pin[1], v = kp.pin[2], Pinf = kp.pin[3];
+    const double q = 0.5 * r * (u * u + v * v);
+    double f[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int w = t; w < a.nwall && t < CSU_BLOCK; w += CSU_BLOCK) {
+      const int gq = a.wall[w];
+      const double cp = (a.Pb[3 * kp.nb + gq] - Pinf) / q;
+      f[0] += cp * a.bdsx[gq];
+      f[2] += cp * a.bdsy[gq];
+      if (a.visc) {
+        f[1] -= a.wfric[gq] / q;
+        f[3] -= a.wfric[kp.nb + gq] / q;
+      }
+    }
+    block_reduce<RES_THREADS, 4>(f, sw, RedSum());
+    if (t == 0)
+      for (int k = 0; k < 4; k++) {
+        double c = f[k] / a.sref;
+        if (kp.axi && k < 2) c *= 2 * M_PI;
+        a.coef[row * 4 + k] = c;
+      }
+  } else {
+    double m[1] = {INFINITY};
+    for (int b = t; b < a.nblocks && t < CSU_BLOCK; b += CSU_BLOCK) m[0] = fmin(m[0], a.red_dt[b]);
+    block_reduce<RES_THREADS, 1>(m, sw, RedMin());
+    if (t == 0) a.dtg[sid] = m[0] * a.cfl;
+  }
+  if (t == 0) {
+    // the slot's rows are stored (their address needed ctr) before this
+    // workgroup counts itself as done
+    __threadfence();
+    if (atomicAdd(a.done, 1) == (int)gridDim.x - 1) {
+      a.done[0] = 0;
+      a.ctr[0] = a.ctr[0] + 1;
     }
   }
-  double f[4] = {ax, vx, ay, vy};
-  block_reduce<CSU_BLOCK, 4>(f, sw, RedSum());
-  if (t == 0) {
-    double c[4] = {f[0] / sref, f[1] / sref, f[2] / sref, f[3] / sref};
-    if (kp.axi) { c[0] *= 2 * M_PI; c[1] *= 2 * M_PI; }
-    for (int k = 0; k < 4; k++) coef[k] = c[k];
-    if (!sol) ctr[0] = ctr[0] + 1;  // last kernel of an iteration: advance the history slot
-  }
-}
-
-// Batch: advance the history slot after every solve's forces.
-__global__ void k_next_slot(int* __restrict__ ctr) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) ctr[0] = ctr[0] + 1;
 }
 
 // Per-cell SST fields of the solution2.csv writer, reference sstInterMiT
