@@ -816,7 +816,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   // small meshes: 64-thread workgroups for the gradient and face kernels
   // (no shared memory), so that a few hundred cell tiles reach every CU
   d->sblk = nc <= 262144 ? 64 : CSU_BLOCK;
-  d->lblk = 64;
+  d->lblk = 128;
   d->tile = 0;
   d->tile_ok = 0;
   kp.xcd = 1;
@@ -888,7 +888,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
       (rc = upload(d, &pref_d, pref)) ||
       (rc = dalloc(d, &d->U, nvc)) || (rc = dalloc(d, &d->Uaux, nvc)) || (rc = dalloc(d, &d->R, nvc)) ||
       (rc = dalloc(d, &d->dtl, nc + 1)) || (rc = dalloc(d, &d->dtg, ns)) ||
-      (rc = dalloc(d, &d->red, 2 * (size_t)nv * d->nred + 16)) ||
+      (rc = dalloc(d, &d->red, 2 * (size_t)nv * d->nred + (size_t)(nc / SLOT_CELLS) + 16)) ||
       (rc = dalloc(d, &s.P, (size_t)(nv + 1) * nc)) || (rc = dalloc(d, &s.Pb, (size_t)(nv + 1) * nb)) ||
       (rc = dalloc(d, &s.dPx, nvc)) || (rc = dalloc(d, &s.dPy, nvc)) || (rc = dalloc(d, &s.phi, nvc)) ||
       (rc = dalloc(d, &s.fflux, (size_t)nv * nf)) || (rc = dalloc(d, &s.bflux, (size_t)nv * nb)))
@@ -1248,8 +1248,8 @@ extern "C" int csu_dev_kernel_times(csu_dev* d, const char** names, double* avg_
 // ---------------------------------------------------------------------------
 // orchestration
 // ---------------------------------------------------------------------------
-// One residual evaluation (solverCalcR) with P valid (ghosts: and the ghost
-// states, k_prim's), then the fused update.
+// One residual evaluation (solverCalcR) with P valid (ghosts: by a k_prim
+// launch just before), then the fused update.
 template <int NV, bool VISC>
 static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, double* Uout, bool ghosts) {
   const KP& kp = d->kp;
@@ -1263,23 +1263,34 @@ static int stage(csu_dev* d, int flags, double sigma, double rk_a, double* Un, d
   {
     Prof p(d, "k_grad");
     const dim3 gg((nc + d->sblk - 1) / d->sblk), bg(d->sblk);
-    const bool ex = !ghosts;
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, gg, bg, 0, d->stream, kp, d->geo, d->st); };
-    if (kp.mixed) ex ? go(k_grad<NV, VISC, false, true, true>) : go(k_grad<NV, VISC, false, true, false>);
-    else if (kp.lsq_ld) ex ? go(k_grad<NV, VISC, true, false, true>) : go(k_grad<NV, VISC, true, false, false>);
-    else if (d->prm.time_scheme == CSU_TIME_RK && NV == 4)
-      ex ? go(k_grad<NV, VISC, false, false, true, NV != 4>) : go(k_grad<NV, VISC, false, false, false, NV != 4>);
-    else ex ? go(k_grad<NV, VISC, false, false, true>) : go(k_grad<NV, VISC, false, false, false>);
+    // without ghosts from k_prim (ghosts), k_grad makes them
+    constexpr bool G0 = NV != 4;
+    const bool rk = d->prm.time_scheme == CSU_TIME_RK && NV == 4;
+    if (ghosts && NV == 4) {
+      if (kp.mixed) go(k_grad<NV, VISC, false, true, G0>);
+      else if (kp.lsq_ld) go(k_grad<NV, VISC, true, false, G0>);
+      else if (rk) go(k_grad<NV, VISC, false, false, G0, NV != 4>);
+      else go(k_grad<NV, VISC, false, false, G0>);
+    } else {
+      if (kp.mixed) go(k_grad<NV, VISC, false, true, true>);
+      else if (kp.lsq_ld) go(k_grad<NV, VISC, true, false, true>);
+      else if (rk) go(k_grad<NV, VISC, false, false, true, NV != 4>);
+      else go(k_grad<NV, VISC, false, false, true>);
+    }
   }
   {
     Prof p(d, "k_flux");
-    const int nfb = (d->nf + d->sblk - 1) / d->sblk, nbb = (d->nb + d->sblk - 1) / d->sblk;
+    const int nfb = (d->nf + d->sblk - 1) / d->sblk;
+    // a multiple of the 8 XCDs, so that the face workgroups behind them run
+    // on the XCD of their cells (xcd_tile)
+    const int nbb = ((d->nb + d->sblk - 1) / d->sblk + 7) / 8 * 8;
     const dim3 gf(nfb + nbb), bf(d->sblk);
     if (nfb + nbb == 0) {
     } else if (kp.mixed)
-      hipLaunchKernelGGL((k_flux<NV, VISC, true>), gf, bf, 0, d->stream, kp, d->geo, d->st, nfb);
+      hipLaunchKernelGGL((k_flux<NV, VISC, true>), gf, bf, 0, d->stream, kp, d->geo, d->st, nbb);
     else
-      hipLaunchKernelGGL((k_flux<NV, VISC>), gf, bf, 0, d->stream, kp, d->geo, d->st, nfb);
+      hipLaunchKernelGGL((k_flux<NV, VISC>), gf, bf, 0, d->stream, kp, d->geo, d->st, nbb);
   }
   {
     Prof p(d, "k_update");
@@ -1329,10 +1340,10 @@ static int tile_stage(csu_dev* d, int flags, double sigma, double rk_a) {
   return CSU_OK;
 }
 
-template <int NV>
+template <int NV, bool GH = NV == 4>
 static int prim_pass(csu_dev* d) {
   Prof p(d, "k_prim");
-  hipLaunchKernelGGL(k_prim<NV>, dim3(nblk(d->nc)), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->geo, d->U, d->st.P,
+  hipLaunchKernelGGL((k_prim<NV, GH>), dim3(nblk(d->nc)), dim3(CSU_BLOCK), 0, d->stream, d->kp, d->geo, d->U, d->st.P,
                      d->st.Pb);
   HIPCHK(hipGetLastError());
   return CSU_OK;
@@ -1393,7 +1404,7 @@ extern "C" int csu_dev_residual(csu_dev* d, double* R, double* dPx, double* dPy,
 extern "C" int csu_dev_primitives(csu_dev* d, double* P) {
   if (!d) return set_err(CSU_ERR_ARG, "null argument");
   if (d->nsolve > 1) return set_err(CSU_ERR_UNSUPPORTED, "%s: not on a batch context (use csu_batch_*)", __func__);
-  int rc = d->nv == 6 ? prim_pass<6>(d) : d->nv == 5 ? prim_pass<5>(d) : prim_pass<4>(d);
+  int rc = d->nv == 6 ? prim_pass<6, true>(d) : d->nv == 5 ? prim_pass<5, true>(d) : prim_pass<4, true>(d);
   if (rc) return rc;
   d->fresh = 1;
   if (P) {
@@ -1418,11 +1429,11 @@ static const double RK5[] = {0.0533, 0.1263, 0.2375, 0.4414, 1.0};
 // the history slot the device counter names, and with dt the global time
 // step from the stage's (or the implicit diagonal's) block minima.
 template <int NV>
-static void iteration_tail(csu_dev* d, bool dt) {
+static void iteration_tail(csu_dev* d, bool dt, int dtc = CSU_BLOCK) {
   Prof p(d, "k_tail");
   TailP a;
   a.nc = d->nc; a.nblocks = nblk(d->nc); a.nsolve = d->nsolve; a.nwall = d->nwall; a.cap = d->hist_cap;
-  a.visc = d->visc; a.cfl = d->prm.cfl; a.sref = d->prm.sref; a.sol = d->geo.sol;
+  a.visc = d->visc; a.dtc = dtc; a.cfl = d->prm.cfl; a.sref = d->prm.sref; a.sol = d->geo.sol;
   a.red = d->red; a.red_dt = d->red + (size_t)NV * d->nred; a.wall = d->wall; a.Pb = d->st.Pb; a.wfric = d->st.wfric;
   a.bdsx = d->geo.bdsx; a.bdsy = d->geo.bdsy; a.res = d->res_hist; a.coef = d->coef_hist; a.dtg = d->dtg;
   a.ctr = d->hctr; a.done = d->hctr + 1;
@@ -1540,18 +1551,20 @@ static int implicit_iteration(csu_dev* d) {
   if (rc) return rc;
   {
     Prof p(d, "k_impD");
-    hipLaunchKernelGGL((k_impD<NV, VISC>), dim3(nb), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo, d->st, d->prm.wimp,
+    hipLaunchKernelGGL((k_impD<NV, VISC>), dim3((nc + SLOT_CELLS - 1) / SLOT_CELLS), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo, d->st, d->prm.wimp,
                        d->Dp, red_min, d->caux);
   }
-  iteration_tail<NV>(d, true);
+  iteration_tail<NV>(d, true, SLOT_CELLS);
   if (d->prm.time_scheme == CSU_TIME_LUSGS) {
     Prof p(d, "k_lusgs");
     // a level holds a fraction of the cells (a colour of the renumbered
-    // mesh): small workgroups (64 threads unless tuned) spread it over every CU
+    // mesh), four lanes per cell: small workgroups spread it over every CU
+    // (128 threads unless tuned: SA, 250k cells 5.41 ms a pass against 5.51
+    // with 64 and 5.49 with 256)
     const int LB = d->lblk;
     for (size_t l = 0; l + 1 < d->lvlL.size(); l++) {
       int off = d->lvlL[l], cnt = d->lvlL[l + 1] - off;
-      hipLaunchKernelGGL((k_lusgs<NV, VISC, 0>), dim3((cnt + LB - 1) / LB), dim3(LB), 0, d->stream, kp, d->geo, d->st,
+      hipLaunchKernelGGL((k_lusgs<NV, VISC, 0>), dim3((4 * cnt + LB - 1) / LB), dim3(LB), 0, d->stream, kp, d->geo, d->st,
                          d->cellsL + off, cnt, d->Dp, d->dtg, d->R, d->dW0, (const double*)nullptr, (double*)nullptr,
                          (const double*)d->caux);
     }
@@ -1559,7 +1572,7 @@ static int implicit_iteration(csu_dev* d) {
     // increment to the state themselves
     for (size_t l = 0; l + 1 < d->lvlU.size(); l++) {
       int off = d->lvlU[l], cnt = d->lvlU[l + 1] - off;
-      hipLaunchKernelGGL((k_lusgs<NV, VISC, 1>), dim3((cnt + LB - 1) / LB), dim3(LB), 0, d->stream, kp, d->geo, d->st,
+      hipLaunchKernelGGL((k_lusgs<NV, VISC, 1>), dim3((4 * cnt + LB - 1) / LB), dim3(LB), 0, d->stream, kp, d->geo, d->st,
                          d->cellsU + off, cnt, d->Dp, d->dtg, d->R, d->dW1, (const double*)d->dW0, d->U,
                          (const double*)d->caux);
     }
@@ -2261,7 +2274,7 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
   const bool visc = p->laminar || p->sa || p->sst;
   double b = 0;
   b += nc * (4 + 16 + 16 + 48 + 64 + 64 + 8) + nf * (8 + 1 + 24) + nb * (12 + 64 + 4);  // geometry
-  b += nc * (24 * nv + 8) + 2 * nv * 8 * (nc / 256 + 1) + 128;                           // U, Uaux, R, dt, reductions
+  b += nc * (24 * nv + 8) + 2 * nv * 8 * (nc / 256 + 1) + 8 * (nc / SLOT_CELLS) + 128;                           // U, Uaux, R, dt, reductions
   b += (nv + 1) * 8 * (nc + nb) + 24 * nv * nc + 8 * nv * nf;                             // P, Pb, grad, phi, fflux
   if (p->order == 2) b += 32 * nv * nc;                                                   // edge states
   if (visc) b += nc * (16 + 16 + 48) + nf * (8 * (nv - 1) + 8) + nb * (8 * (nv - 1) + 16);

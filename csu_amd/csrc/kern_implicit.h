@@ -15,100 +15,105 @@ namespace csu {
 
 __device__ __forceinline__ double gamma_of(const GasD& g, double T) { return gas_T2gamma<double>(g, T); }
 
+// Four lanes of a wavefront work on one cell, a lane per face slot, where a
+// thread per cell would walk its neighbours one memory round trip after the
+// other.  slot_val: lane q's value in all four lanes of its cell (a quad
+// permutation, no LDS), from which every lane takes the sums in slot order.
+#define SLOT_CELLS (CSU_BLOCK / 4)  // cells of a workgroup
+template <int Q>
+__device__ __forceinline__ double slot_val(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(hi, Q * 0x55, 0xF, 0xF, true),
+                          __builtin_amdgcn_mov_dpp(lo, Q * 0x55, 0xF, 0xF, true));
+}
+
 // implicitCalcD (implicit.c:19-181), everything but the global-time-step
-// term: writes Dp = 0.5 w Lc (+ Lv/Omega) and per-block min of Omega/Lc.
+// term: writes Dp = 0.5 w Lc (+ Lv/Omega) and the minimum of Omega/Lc per
+// SLOT_CELLS cells.
+// A lane per face slot (slot_val): SA, 250k cells 22.7 -> 21.8 us, bound by
+// its gathers' bytes; the smaller meshes' latency gains more.
 template <int NV, bool VISC>
 __global__ __launch_bounds__(CSU_BLOCK) void k_impD(KP kp, Geo g, St s, double wimp, double* __restrict__ Dp,
                                                     double* __restrict__ red_min, double* __restrict__ caux) {
   __shared__ double sw[1][CSU_BLOCK / 64];
-  const int t = threadIdx.x, i = blockIdx.x * blockDim.x + t;
+  const int t = threadIdx.x, c0 = blockIdx.x * SLOT_CELLS, i = c0 + (t >> 2), j = t & 3;
   const int nc = kp.nc;
-  if (g.sol) kp.cend = g.sol[solve_of(g.csolk, blockIdx.x * blockDim.x)].c1;
+  if (g.sol) kp.cend = g.sol[solve_of(g.csolk, c0)].c1;
   double val = INFINITY;
   if (i < kp.cend) {
     const double* P = s.P;
-    double Lc = 0, Lv = 0;
-    // all slots' face data and neighbours, then all states, then the sums
-    // in slot order.  The face's two states are the cell's and the
-    // neighbour's (cfn) in either order: the face means add them, and a sum
-    // of two doubles does not depend on their order.
-    int cfj[4], fij[4], nbj[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      cfj[j] = g.cface[j * nc + i];
-      nbj[j] = g.cfn[j * nc + i];
-      fij[j] = cfj[j] > 0 ? cfj[j] - 1 : (cfj[j] < 0 ? -cfj[j] - 1 : 0);
-    }
-    double sxj[4], syj[4], sj[4], Pa[4], Pb[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      sxj[j] = g.fdsx[fij[j]];
-      syj[j] = g.fdsy[fij[j]];
-      sj[j] = g.fds[fij[j]];
-    }
+    // The face's two states are the cell's and the neighbour's (cfn) in
+    // either order: the face means add them, and a sum of two doubles does
+    // not depend on their order.
+    const int cf = g.cface[j * nc + i], nbr = g.cnbr[j * nc + i], nb = cf == 0 ? i : g.cfn[j * nc + i];
+    const int np = g.cnp[i], fi = cf > 0 ? cf - 1 : (cf < 0 ? -cf - 1 : 0);
+    double Pa[4], Pb[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) Pa[q] = P[(q == 3 ? 4 : q) * nc + i];  // r u v T
-    if (caux) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) Pb[q] = P[(q == 3 ? 4 : q) * nc + nb];
+    const double om = g.omega[i];
+    double lc = 0.0, lv = 0.0, lcb = 0.0, lvb = 0.0;
+    if (cf != 0) {
+      const double dSx = g.fdsx[fi], dSy = g.fdsy[fi], dS = g.fds[fi];
+      double r = (Pa[0] + Pb[0]) * 0.5;
+      double u = (Pa[1] + Pb[1]) * 0.5;
+      double v = (Pa[2] + Pb[2]) * 0.5;
+      double T = (Pa[3] + Pb[3]) * 0.5;
+      double c = gas_T2c<double>(kp.gas, T);
+      const Den<double> dl(dS);
+      double nx = dl(dSx), ny = dl(dSy);
+      lc = (fabs(nx * u + ny * v) + c) * dS;
+      if (VISC) {
+        double mi = sutherland(T);
+        const double mp = Den<double>(kp.pr, kp.rpr)(mi);
+        double mt = NV == 4 ? mp : mp + Den<double>(kp.pr_t, kp.rpr_t)(s.miT[fi]);
+        lv = fmax(4 / (3 * r), gamma_of(kp.gas, T) / r) * mt * dS * dS;
+      }
+    }
+    if (j < np && nbr < 0) {
+      const int q = -1 - nbr;
+      const double dSx = g.bdsx[q], dSy = g.bdsy[q], dS = g.bds[q];
+      const double r = Pa[0], u = Pa[1], v = Pa[2], T = Pa[3];
+      const double c = gas_T2c<double>(kp.gas, T);
+      double nx, ny;
+      if (dS > 0) { nx = dSx / dS; ny = dSy / dS; } else { nx = 0.0; ny = 1.0; }
+      lcb = (fabs(nx * u + ny * v) + c) * dS;
+      if (VISC) {
+        double mi = sutherland(T);
+        lvb = fmax(4 / (3 * r), gamma_of(kp.gas, T) / r) * (mi / kp.pr) * dS * dS;
+      }
+    }
+    if (caux && j == 3) {
       // LU-SGS: the cell-state factors of its neighbour terms, evaluated
       // once per cell instead of once per face and sweep (same expressions
-      // of the same values: implicit.c:307-313, 555-595)
+      // of the same values: implicit.c:307-313, 555-595); by the lane that
+      // has no face on a triangle
       caux[i] = gas_T2c<double>(kp.gas, Pa[3]);
       if (VISC) {
         caux[nc + i] = fmax(4 / (3 * Pa[0]), gamma_of(kp.gas, Pa[3]) / Pa[0]);
         caux[2 * nc + i] = sutherland(Pa[3]) / kp.pr;
       }
     }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int b = cfj[j] == 0 ? i : nbj[j];
-#pragma unroll
-      for (int q = 0; q < 4; q++) Pb[j][q] = P[(q == 3 ? 4 : q) * nc + b];
-    }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      if (cfj[j] == 0) continue;
-      const int fi = fij[j];
-      const double dSx = sxj[j], dSy = syj[j], dS = sj[j];
-      double r = (Pa[0] + Pb[j][0]) * 0.5;
-      double u = (Pa[1] + Pb[j][1]) * 0.5;
-      double v = (Pa[2] + Pb[j][2]) * 0.5;
-      double T = (Pa[3] + Pb[j][3]) * 0.5;
-      double c = gas_T2c<double>(kp.gas, T);
-      const Den<double> dl(dS);
-      double nx = dl(dSx), ny = dl(dSy);
-      Lc += (fabs(nx * u + ny * v) + c) * dS;
-      if (VISC) {
-        double mi = sutherland(T);
-        const double mp = Den<double>(kp.pr, kp.rpr)(mi);
-        double mt = NV == 4 ? mp : mp + Den<double>(kp.pr_t, kp.rpr_t)(s.miT[fi]);
-        Lv += fmax(4 / (3 * r), gamma_of(kp.gas, T) / r) * mt * dS * dS;
-      }
-    }
-    const double om = g.omega[i];
+    // sums in slot order: interior faces, then boundary faces (slots
+    // without one hold 0, which changes no sum of non-negative terms)
+    const double Lc = ((slot_val<0>(lc) + slot_val<1>(lc)) + slot_val<2>(lc)) + slot_val<3>(lc);
+    const double Lv = ((slot_val<0>(lv) + slot_val<1>(lv)) + slot_val<2>(lv)) + slot_val<3>(lv);
     double dtl = Lc;
     double D = 0.5 * wimp * Lc;
     if (VISC) D += Lv / om;
-    const int np = g.cnp[i];
-    for (int j = 0; j < np; j++) {
-      const int n = g.cnbr[j * nc + i];
-      if (n >= 0) continue;
-      const int q = -1 - n;
-      const double dSx = g.bdsx[q], dSy = g.bdsy[q], dS = g.bds[q];
-      double r = P[i], u = P[nc + i], v = P[2 * nc + i], T = P[4 * nc + i];
-      double c = gas_T2c<double>(kp.gas, T);
-      double nx, ny;
-      if (dS > 0) { nx = dSx / dS; ny = dSy / dS; } else { nx = 0.0; ny = 1.0; }
-      double Lcb = (fabs(nx * u + ny * v) + c) * dS;
-      dtl += Lcb;
-      D += 0.5 * wimp * Lcb;
-      if (VISC) {
-        double mi = sutherland(T);
-        double Lvb = fmax(4 / (3 * r), gamma_of(kp.gas, T) / r) * (mi / kp.pr) * dS * dS;
-        D += Lvb / om;
-      }
+    const double bc[4] = {slot_val<0>(lcb), slot_val<1>(lcb), slot_val<2>(lcb), slot_val<3>(lcb)};
+    const double bv[4] = {slot_val<0>(lvb), slot_val<1>(lvb), slot_val<2>(lvb), slot_val<3>(lvb)};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      dtl += bc[q];
+      D += 0.5 * wimp * bc[q];
+      if (VISC) D += bv[q] / om;
     }
-    Dp[i] = D;
-    val = om / dtl;
+    if (j == 0) {
+      Dp[i] = D;
+      val = om / dtl;
+    }
   }
   double m[1] = {val};
   block_reduce<CSU_BLOCK, 1>(m, sw, RedMin());
@@ -260,13 +265,18 @@ __device__ __forceinline__ int face_from(const Geo& g, int nc, int i, int j, dou
 // once its level has run, so the level also applies it to the state
 // (solverUpdateUImplicit, solver.c:1945-1955; a held solve of a batch keeps
 // its state).
+// A level is a fraction of the cells, and what bounds it is the chain of
+// round trips of one wavefront; a lane per face slot (slot_val) loads and
+// evaluates a cell's neighbours side by side.  Passes of 25 iterations, a
+// thread per cell -> a lane per slot (with k_impD's): SST, 110k cells 4.57 ->
+// 4.28 ms, SA, 250k cells 5.65 -> 5.52 ms; no change for Euler ramps.
 template <int NV, bool VISC, int DIR>
 __global__ __launch_bounds__(CSU_BLOCK) void k_lusgs(KP kp, Geo g, St s, const int* __restrict__ cells, int ncell_lvl,
                                                      const double* __restrict__ Dp, const double* __restrict__ dtg,
                                                      const double* __restrict__ R, double* dW,
                                                      const double* __restrict__ dW0, double* __restrict__ U,
                                                      const double* __restrict__ caux) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int t = (blockIdx.x * blockDim.x + threadIdx.x) >> 2, j = threadIdx.x & 3;
   if (t >= ncell_lvl) return;
   const int nc = kp.nc;
   const int i = cells[t];
@@ -288,43 +298,23 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_lusgs(KP kp, Geo g, St s, const i
       }
     }
   }
-  // Face data of all slots is loaded before any slot is used (one round
-  // trip per dependency level, not per slot); neighbour states are loaded
-  // per slot, only for the neighbours this sweep uses (loading them all up
-  // front needs ~200 VGPRs and halves the occupancy, measured slower).
-  int cfj[4], nbj[4], fij[4];
+  // this lane's slot: its face and neighbour, then the neighbour term (0
+  // where the sweep does not use the slot: subtracting 0 changes nothing)
+  const int cf = g.cface[j * nc + i], e = g.cfn[j * nc + i], fi = cf > 0 ? cf - 1 : (cf < 0 ? -cf - 1 : 0);
+  const double dS = g.fds[fi], fx = g.fnx[fi], fy = g.fny[fi], fd = VISC ? g.fdd[fi] : 1.0;
+  const int nb = cf == 0 ? i : e;
+  double term[NV];
 #pragma unroll
-  for (int j = 0; j < 4; j++) cfj[j] = g.cface[j * nc + i];
-  double nxj[4], nyj[4], sj[4], ddj[4];
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int f = cfj[j];
-    const int fi = f > 0 ? f - 1 : (f < 0 ? -f - 1 : 0);
-    fij[j] = fi;
-    sj[j] = g.fds[fi];
-    nxj[j] = g.fnx[fi];
-    nyj[j] = g.fny[fi];
-    ddj[j] = VISC ? g.fdd[fi] : 1.0;
-    const int e = g.cfn[j * nc + i];  // loaded beside cface, not after it
-    nbj[j] = f == 0 ? i : e;
-  }
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    // the slot's neighbour and outward unit normal (face_from: negated when
-    // i is the face's e1, implicit.c:288-305; dS/|dS| with the sign of dS,
-    // stored per face)
-    if (cfj[j] == 0) continue;
-    const int nb = nbj[j], fi = fij[j];
-    const double dS = sj[j];
-    if (DIR == 0 ? !(nb < i) : !(nb > i)) continue;
-    const double nx = cfj[j] > 0 ? nxj[j] : -nxj[j], ny = cfj[j] > 0 ? nyj[j] : -nyj[j];
-    double Pj[NV + 1];
+  for (int k = 0; k < NV; k++) term[k] = 0.0;
+  if (cf != 0 && (DIR == 0 ? nb < i : nb > i)) {
+    // outward unit normal (face_from: negated when i is the face's e1,
+    // implicit.c:288-305; dS/|dS| with the sign of dS, stored per face)
+    const double nx = cf > 0 ? fx : -fx, ny = cf > 0 ? fy : -fy;
+    double Pj[NV + 1], d[NV], dF[NV];
 #pragma unroll
     for (int m = 0; m < NV + 1; m++) Pj[m] = s.P[m * nc + nb];
-    double d[NV];
 #pragma unroll
     for (int k = 0; k < NV; k++) d[k] = dW[k * nc + nb];
-    double dF[NV];
     delta_flux<NV>(kp, Pj, d, nx, ny, dF);
     // the neighbour's sound speed and viscous factors max(4/(3r), gamma/r)
     // and mu/Pr (k_impD, per cell)
@@ -332,12 +322,19 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_lusgs(KP kp, Geo g, St s, const i
     double ra = kp.wimp * (fabs(nx * Pj[1] + ny * Pj[2]) + c) * dS;
     if (NV >= 5) {
       // implicitFunc_sa / _sst (implicit.c:555-595, 1120-1161)
-      ra += caux[nc + nb] * (caux[2 * nc + nb] + Den<double>(kp.pr_t, kp.rpr_t)(s.miT[fi])) * dS / ddj[j];
+      ra += caux[nc + nb] * (caux[2 * nc + nb] + Den<double>(kp.pr_t, kp.rpr_t)(s.miT[fi])) * dS / fd;
     } else if (VISC && kp.laminar) {
-      ra += caux[nc + nb] * caux[2 * nc + nb] * dS / ddj[j];
+      ra += caux[nc + nb] * caux[2 * nc + nb] * dS / fd;
     }
 #pragma unroll
-    for (int k = 0; k < NV; k++) acc[k] -= 0.5 * (dF[k] * dS - ra * d[k]);
+    for (int k = 0; k < NV; k++) term[k] = 0.5 * (dF[k] * dS - ra * d[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    acc[k] -= slot_val<0>(term[k]);
+    acc[k] -= slot_val<1>(term[k]);
+    acc[k] -= slot_val<2>(term[k]);
+    acc[k] -= slot_val<3>(term[k]);
   }
   double out[NV];
   const Den<double> dD(D);
@@ -359,12 +356,14 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_lusgs(KP kp, Geo g, St s, const i
       out[O] = (-A * c + B * a) / det;
     }
   }
+  // every lane of the cell has all of out: each stores its share
+  const bool upd = DIR == 1 && (!g.sol || g.sol[sid].active);
 #pragma unroll
-  for (int k = 0; k < NV; k++) dW[k * nc + i] = out[k];
-  if (DIR == 1 && (!g.sol || g.sol[sid].active)) {
-#pragma unroll
-    for (int k = 0; k < NV; k++) U[k * nc + i] += out[k];
-  }
+  for (int k = 0; k < NV; k++)
+    if ((k & 3) == j) {
+      dW[k * nc + i] = out[k];
+      if (upd) U[k * nc + i] += out[k];
+    }
 }
 
 // DPLUR finite-difference blocks of every interior neighbour

@@ -4,10 +4,10 @@
 //   k_grad    cells  ghost states of the cell's boundary faces, least-squares
 //                    gradients (precomputed weights, or double-double sums),
 //                    Venkatakrishnan phi, the reconstructed state at every
-//                    edge; viscous: T gradient, boundary viscous fluxes, wall
-//                    friction (all need only the cell's own fresh data)
+//                    edge; viscous: T gradient, turbulence sources
 //   k_flux    faces  Riemann flux of the two edge states (+ viscous face flux);
-//                    boundary faces: their convective flux
+//                    boundary faces: their convective and viscous fluxes,
+//                    wall friction and shear
 //   k_update  cells  per-cell sums in the reference's order, then the RK
 //                    update fused with the next stage's primitive recovery;
 //                    on the last stage also the next time step and the
@@ -43,28 +43,18 @@ __device__ __forceinline__ void cell_ghosts(const KP& kp, const Geo& g, int i, i
 // host).  Clamped values are written back to U, as the reference does.
 // Batch: the cells of a held solve keep their state (a batch's padding
 // cells hold their solve's free stream and are converted like the rest).
-// Also the ghost states of the boundary faces.
-template <int NV>
+// GH: also the ghost states of the boundary faces (see k_grad; and for the
+// entry point that recomputes the primitives outside an iteration).
+template <int NV, bool GH>
 __global__ __launch_bounds__(CSU_BLOCK) void k_prim(KP kp, Geo g, double* __restrict__ U, double* __restrict__ P,
                                                     double* __restrict__ Pb) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int nc = kp.nc;
   if (i >= nc) return;
-  const int bm = g.bmask[i];
-  bool held = false;
   if (g.sol) {
     const SolveP& q = g.sol[solve_of(g.csolk, blockIdx.x * blockDim.x)];
-    solve_kp(kp, q);
-    held = !q.active;
-  }
-  if (held) {  // the state stays as it is, and so do its primitives
-    if (bm) {
-      double p[NV + 1];
-#pragma unroll
-      for (int m = 0; m < NV + 1; m++) p[m] = P[m * nc + i];
-      cell_ghosts<NV>(kp, g, i, bm, p, Pb);
-    }
-    return;
+    if (!q.active) return;
+    if (GH) solve_kp(kp, q);
   }
   double u[NV], u0[NV], p[NV + 1];
 #pragma unroll
@@ -75,6 +65,7 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_prim(KP kp, Geo g, double* __rest
     if (__double_as_longlong(u[k]) != __double_as_longlong(u0[k])) U[k * nc + i] = u[k];
 #pragma unroll
   for (int m = 0; m < NV + 1; m++) P[m * nc + i] = p[m];
+  const int bm = GH ? g.bmask[i] : 0;
   if (bm) cell_ghosts<NV>(kp, g, i, bm, p, Pb);
 }
 
@@ -99,17 +90,15 @@ __device__ __forceinline__ void lsq_grad(int np, const double* dx, const double*
 // Gradient + limiter (+ boundary work) kernel.  Reference solverUpdateGrad /
 // solverCalcGrad3 (solver.c:451-474, 1031-1074), solverGrad_T
 // (solver.c:477-490), the limiter loop of inter() (solver.c:496-548,
-// limiter.c:98-147), boundaryCalcPrimitive (boundary.c:514-693),
-// boundaryFaceViscFlux (laminar.c:128-346), boundaryCalcFrictionWall
-// (boundary.c:695-742).
+// limiter.c:98-147), boundaryCalcPrimitive (boundary.c:514-693).
 // MIX (mixed precision): gradients, limiter and reconstruction in FP32 from
 // FP64 differences; edge states stored in FP32.
 // REFL: the limiter function in the reference's sequence of roundings.  The
 // implicit schemes keep it: DPLUR's finite differences (h = 1e-6) and the SST
 // source terms turn one-ulp differences of the gradients into 1e-9.
-// GH: a stage not preceded by k_prim (explicit runs), which would have made
-// the ghost states; elsewhere their registers would cost this kernel a
-// wavefront per SIMD (SA, 250k cells: 49 us with them, 43 without).
+// GH: the ghost states are made here; without, k_prim has made them (four-
+// variable stages behind a k_prim launch, where that measured 2 % faster on
+// served Euler ramps; with turbulence variables it measured slower).
 template <int NV, bool VISC, bool LD, bool MIX, bool GH, bool REFL = true>
 __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   using TF = typename std::conditional<MIX, float, double>::type;
@@ -134,23 +123,16 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   if (GH && bm) cell_ghosts<NV>(kp, g, i, bm, Pi, s.Pb);
   // neighbours: cells, or the ghost states of boundary faces
   double dx[4], dy[4];
-  int gb[4], nbr[4];
+  int nbr[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    gb[j] = -1;
     nbr[j] = 0;
     if (j >= np) break;
-    int n = g.cnbr[j * nc + i];
+    const int n = g.cnbr[j * nc + i];
     nbr[j] = n;
-    if (n >= 0) {
-      dx[j] = g.xc[n] - x0;
-      dy[j] = g.yc[n] - y0;
-    } else {
-      int q = -1 - n;
-      gb[j] = q;
-      dx[j] = g.bxm[q] - x0;
-      dy[j] = g.bym[q] - y0;
-    }
+    if (!LD) continue;
+    dx[j] = (n >= 0 ? g.xc[n] : g.bxm[-1 - n]) - x0;
+    dy[j] = (n >= 0 ? g.yc[n] : g.bym[-1 - n]) - y0;
   }
   // Every neighbour value the cell reads, loaded before any store: the
   // compiler cannot tell the stores below from these loads, so loading
@@ -329,39 +311,6 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
       const double Qt = sa_source(Pi[5], mi_L / Pi[0], S, g.wdist[i], Pi[0], grx, gry, gnx, gny, kp.sa_cc != 0);
       s.src[i] = Qt * g.omega[i];
     }
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int q = gb[j];
-      if (q < 0) continue;
-      const int t = g.btype[q];
-      double f[5];
-      if (NV == 6) {
-        sst_bc_face(kp, t, g.bdsx[q], g.bdsy[q], g.bnx[q], g.bny[q], g.bds2[q], dx[j], dy[j], Pi, g.wdist[i], gx3,
-                    gy3, f);
-        s.bvflux[3 * nb + q] = f[3];
-        s.bvflux[4 * nb + q] = f[4];
-      } else if (NV == 5) {
-        sa_bc_face(kp, t, g.bdsx[q], g.bdsy[q], g.bnx[q], g.bny[q], g.bds2[q], dx[j], dy[j], Pi, gx3, gy3, grx, gry,
-                   f);
-        s.bvflux[3 * nb + q] = f[3];
-      } else {
-        laminar_bc_face(kp, t, g.bdsx[q], g.bdsy[q], g.bnx[q], g.bny[q], g.bds2[q], dx[j], dy[j], Pi, gx3, gy3, f);
-      }
-      s.bvflux[0 * nb + q] = f[0];
-      s.bvflux[1 * nb + q] = f[1];
-      s.bvflux[2 * nb + q] = f[2];
-      if (t == CSU_BC_WALL || t == CSU_BC_WALLT) {
-        double fx, fy;
-        wall_friction(g.bdsx[q], g.bdsy[q], dx[j], dy[j], Pi, gx3, gy3, fx, fy);
-        s.wfric[q] = fx;
-        s.wfric[nb + q] = fy;
-        double wt[4];
-        wall_tensor(NV > 4, g.bdsx[q], g.bdsy[q], dx[j], dy[j], g.bxm[q], Pi, NV > 4 ? g.wdist[i] : 0.0, gx3, gy3,
-                    wt);
-#pragma unroll
-        for (int k = 0; k < 4; k++) s.wten[k * nb + q] = wt[k];
-      }
-    }
   }
 }
 
@@ -477,11 +426,17 @@ __device__ __forceinline__ void conv_flux(const KP& kp, const Geo& g, const St& 
 
 // A workgroup's boundary faces from q0 on: the convective flux from the
 // first-order state, boundaryCalc / _sa / _sst (boundary.c:143-446): f*dS, or
-// 0 when dS = 0.
-template <int NV>
+// 0 when dS = 0; viscous runs: boundaryFaceViscFlux (laminar.c:128-346) and
+// its SA / SST forms, boundaryCalcFrictionWall (boundary.c:695-742) and the
+// wall shear.  The viscous part sat in k_grad, which has the gradients in
+// registers; but on a renumbered mesh nearly every wavefront holds a boundary
+// cell, and so ran all of it, once per slot (SA, 250k cells
+// in colour order: k_grad 43 -> 33 us; laminar plate, 100k cells: 19 -> 16 us).
+template <int NV, bool VISC>
 __device__ __forceinline__ void bc_face(KP kp, const Geo& g, const St& s, int q0) {
   const int q = q0 + threadIdx.x;
   const int nc = kp.nc, nb = kp.nb;
+  if (q0 >= nb) return;  // a workgroup of the launch's rounding
   if (g.sol) solve_kp(kp, g.sol[solve_of(g.bsolk, q0)]);
   if (q >= kp.bend) return;
   const int i = g.be0[q];
@@ -494,20 +449,50 @@ __device__ __forceinline__ void bc_face(KP kp, const Geo& g, const St& s, int q0
   bc_flux<NV>(kp, g.btype[q], g.bdsx[q], g.bdsy[q], g.bds[q], Pi, R);
 #pragma unroll
   for (int kk = 0; kk < NV; kk++) s.bflux[kk * nb + q] = R[kk];
+  if (!VISC) return;
+  // viscous flux, wall friction and wall shear from the cell's gradients
+  const int t = g.btype[q];
+  const double dSx = g.bdsx[q], dSy = g.bdsy[q], nx = g.bnx[q], ny = g.bny[q], dS2 = g.bds2[q];
+  const double dx = g.bxm[q] - g.xc[i], dy = g.bym[q] - g.yc[i];
+  const double d = NV > 4 ? g.wdist[i] : 0.0;
+  double gx[5] = {s.dPx[nc + i], s.dPx[2 * nc + i], s.dTx[i], 0.0, 0.0};
+  double gy[5] = {s.dPy[nc + i], s.dPy[2 * nc + i], s.dTy[i], 0.0, 0.0};
+#pragma unroll
+  for (int kk = 4; kk < NV; kk++) {
+    gx[kk - 1] = s.dPx[kk * nc + i];
+    gy[kk - 1] = s.dPy[kk * nc + i];
+  }
+  double f[5];
+  if (NV == 6) sst_bc_face(kp, t, dSx, dSy, nx, ny, dS2, dx, dy, Pi, d, gx, gy, f);
+  else if (NV == 5) sa_bc_face(kp, t, dSx, dSy, nx, ny, dS2, dx, dy, Pi, gx, gy, s.dPx[i], s.dPy[i], f);
+  else laminar_bc_face(kp, t, dSx, dSy, nx, ny, dS2, dx, dy, Pi, gx, gy, f);
+#pragma unroll
+  for (int kk = 0; kk < NV - 1; kk++) s.bvflux[kk * nb + q] = f[kk];
+  if (t == CSU_BC_WALL || t == CSU_BC_WALLT) {
+    double fx, fy, wt[4];
+    wall_friction(dSx, dSy, dx, dy, Pi, gx, gy, fx, fy);
+    s.wfric[q] = fx;
+    s.wfric[nb + q] = fy;
+    wall_tensor(NV > 4, dSx, dSy, dx, dy, g.bxm[q], Pi, d, gx, gy, wt);
+#pragma unroll
+    for (int k = 0; k < 4; k++) s.wten[k * nb + q] = wt[k];
+  }
 }
 
 // Interior face flux, reference inter() face loop (solver.c:550-644), and
 // for viscous runs the laminar face flux (laminar.c:17-75).
 // MIX: the convective flux in FP32 from FP32 edge states, stored in FP32.
-// The workgroups from nfb on take the boundary faces (bc_face): as a launch
-// of its own that work cost 4-5 us per stage, of which it ran under one.
+// The first nbb workgroups take the boundary faces (bc_face; a long chain, so
+// they start first): as a launch of its own that work cost 4-5 us per stage,
+// of which it ran under one.
 template <int NV, bool VISC, bool MIX = false>
-__global__ __launch_bounds__(CSU_BLOCK) void k_flux(KP kp, Geo g, St s, int nfb) {
-  if ((int)blockIdx.x >= nfb) {
-    bc_face<NV>(kp, g, s, (blockIdx.x - nfb) * blockDim.x);
+__global__ __launch_bounds__(CSU_BLOCK) void k_flux(KP kp, Geo g, St s, int nbb) {
+  if ((int)blockIdx.x < nbb) {
+    bc_face<NV, VISC>(kp, g, s, blockIdx.x * blockDim.x);
     return;
   }
-  const int e0f = (kp.xcd ? xcd_tile(blockIdx.x, nfb) : (int)blockIdx.x) * blockDim.x;
+  const int b = blockIdx.x - nbb;
+  const int e0f = (kp.xcd ? xcd_tile(b, gridDim.x - nbb) : b) * blockDim.x;
   const int f = e0f + threadIdx.x;
   const int nc = kp.nc, nf = kp.nf;
   if (g.sol) solve_kp(kp, g.sol[solve_of(g.fsolk, e0f)]);
@@ -857,8 +842,8 @@ __global__ void k_time_clamp(double* __restrict__ ts, double* __restrict__ dtg, 
 // the global time step (k_dt_final).  One workgroup each and per solve,
 // running beside each other: as three launches they cost 4-5 us apiece.
 // The norm's threads sum strided slices of the block partials (rows of
-// length stride), then a fixed tree; the other two do with the first
-// CSU_BLOCK threads what they did in workgroups of that size.
+// length stride), then a fixed tree; the forces' first CSU_BLOCK threads do
+// the same over the wall list.
 // The history slot is ctr % cap: the iteration counter lives on the device
 // so that a captured graph writes each replay's rows to its own slot; the
 // last workgroup to finish (done) advances it.  Batch (sol non-null): a
@@ -867,6 +852,7 @@ __global__ void k_time_clamp(double* __restrict__ ts, double* __restrict__ dtg, 
 #define RES_THREADS 1024
 struct TailP {
   int nc, nblocks, nsolve, nwall, cap, visc;
+  int dtc;  // cells behind one entry of red_dt
   double cfl, sref;
   const SolveP* sol;
   const double *red, *red_dt;  // red_dt null: no time step
@@ -885,7 +871,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_tail(KP kp, TailP a) {
     const SolveP& q = a.sol[sid];
     solve_kp(kp, q);
     a.red += q.c0 / CSU_BLOCK;
-    a.red_dt += q.c0 / CSU_BLOCK;
+    a.red_dt += q.c0 / a.dtc;
     a.nc = q.c1 - q.c0;
     a.nblocks = (a.nc + CSU_BLOCK - 1) / CSU_BLOCK;
     a.wall += q.w0;
@@ -909,6 +895,7 @@ __global__ __launch_bounds__(RES_THREADS) void k_tail(KP kp, TailP a) {
     const double r = kp.pin[0], u = kp.pin[1], v = kp.pin[2], Pinf = kp.pin[3];
     const double q = 0.5 * r * (u * u + v * v);
     double f[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
     for (int w = t; w < a.nwall && t < CSU_BLOCK; w += CSU_BLOCK) {
       const int gq = a.wall[w];
       const double cp = (a.Pb[3 * kp.nb + gq] - Pinf) / q;
@@ -928,7 +915,8 @@ __global__ __launch_bounds__(RES_THREADS) void k_tail(KP kp, TailP a) {
       }
   } else {
     double m[1] = {INFINITY};
-    for (int b = t; b < a.nblocks && t < CSU_BLOCK; b += CSU_BLOCK) m[0] = fmin(m[0], a.red_dt[b]);
+    const int n = (a.nc + a.dtc - 1) / a.dtc;
+    for (int b = t; b < n; b += RES_THREADS) m[0] = fmin(m[0], a.red_dt[b]);
     block_reduce<RES_THREADS, 1>(m, sw, RedMin());
     if (t == 0) a.dtg[sid] = m[0] * a.cfl;
   }
