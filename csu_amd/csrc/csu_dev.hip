@@ -22,6 +22,7 @@
 using namespace csu;
 
 #define CSU_MAX_DEVICES 64
+#define RESIDUAL_ONE_COPY (4u << 20)  // bytes up to which csu_dev_residual copies everything at once
 
 // ---------------------------------------------------------------------------
 // error reporting
@@ -72,6 +73,7 @@ struct csu_dev {
   int nwall;
   int* wall;                   // [nwall] boundary ids of wall/wallT faces
   double *U, *Uaux, *R, *dtl, *dtg;
+  double* fields;              // R, gradients, limiter, primitives, ghost states (csu_dev_residual)
   double* red;                 // reduction scratch
   int nred;                    // number of partial blocks of a cell launch
   double *res_hist, *coef_hist;
@@ -264,43 +266,68 @@ static double tri_omega(const csu_mesh_desc* m, int p0, int p1, int p2) {
   return 0.5 * ((x1 - x2) * (y1 + y2) + (x2 - x3) * (y2 + y3) + (x3 - x1) * (y3 + y1));
 }
 
-// Wall segments (p0x, p0y, p1x, p1y) SoA [4][nw] of the wall / wallT
-// boundary faces, in boundary-face order.
-static std::vector<double> wall_segments(const csu_mesh_desc* m, int* nw) {
+// What k_wall_dist reads of the wall / wallT boundary faces, in
+// boundary-face order: segments [6][nw], group boxes [4][ng] and the largest
+// coordinate's size.
+static std::vector<double> wall_segments(const csu_mesh_desc* m, int* nw, int* ng) {
   std::vector<int> w;
   for (int g = 0; g < m->nbface; g++) {
     const int t = m->mark_type[m->bface_mark[g]];
     if (t == CSU_BC_WALL || t == CSU_BC_WALLT) w.push_back(g);
   }
-  const size_t n = w.size();
-  std::vector<double> seg(4 * (n ? n : 1));
-  for (size_t k = 0; k < n; k++) {
-    const int32_t* q = m->bface + 3 * w[k];
-    seg[k] = m->node_xy[2 * q[1]];
-    seg[n + k] = m->node_xy[2 * q[1] + 1];
-    seg[2 * n + k] = m->node_xy[2 * q[2]];
-    seg[3 * n + k] = m->node_xy[2 * q[2] + 1];
+  const size_t n = w.size(), nk = (n + WD_GROUP - 1) / WD_GROUP;
+  std::vector<double> seg(6 * n + 4 * nk + 1);
+  double* box = seg.data() + 6 * n;
+  for (size_t k = 0; k < nk; k++) {
+    box[k] = box[2 * nk + k] = INFINITY;
+    box[nk + k] = box[3 * nk + k] = -INFINITY;
+  }
+  for (size_t j = 0; j < n; j++) {
+    const int32_t* q = m->bface + 3 * w[j];
+    const double x0 = m->node_xy[2 * q[1]], y0 = m->node_xy[2 * q[1] + 1];
+    const double x1 = m->node_xy[2 * q[2]], y1 = m->node_xy[2 * q[2] + 1];
+    const double ex = x1 - x0, ey = y1 - y0, den = ex * ex + ey * ey;
+    seg[j] = x0; seg[n + j] = y0; seg[2 * n + j] = ex; seg[3 * n + j] = ey; seg[4 * n + j] = den;
+    seg[5 * n + j] = 1.0 / den;
+    box[4 * nk] = fmax(box[4 * nk], fmax(fmax(fabs(x0), fabs(x1)), fmax(fabs(y0), fabs(y1))));
+    if (!(den > 0.0)) continue;  // its distance is NaN: never the nearest
+    const size_t k = j / WD_GROUP;
+    box[k] = fmin(box[k], fmin(x0, x1)); box[nk + k] = fmax(box[nk + k], fmax(x0, x1));
+    box[2 * nk + k] = fmin(box[2 * nk + k], fmin(y0, y1)); box[3 * nk + k] = fmax(box[3 * nk + k], fmax(y0, y1));
   }
   *nw = (int)n;
+  *ng = (int)nk;
   return seg;
 }
 
-// Wall distance on the device into dist[nc] (device memory), from device
-// cell centres; synchronous on `st`.
-static int wall_distance_launch(const csu_mesh_desc* m, hipStream_t st, const double* xc, const double* yc,
-                                double* dist) {
-  int nw = 0;
-  std::vector<double> seg = wall_segments(m, &nw);
-  double* dseg = nullptr;
-  if (hipMalloc(&dseg, seg.size() * sizeof(double)) != hipSuccess)
-    return set_err(CSU_ERR_NOMEM, "hipMalloc of %zu wall-segment bytes failed", seg.size() * sizeof(double));
+// Wall distance on the device into dist[nc] (device memory), from the cells'
+// centres, or where cv is given from their vertices (all device memory);
+// dseg: device room for the segments.  Enqueued on `st`.
+static int wall_distance_on(const csu_mesh_desc* m, hipStream_t st, const std::vector<double>& seg, int nw, int ng,
+                            double* dseg, const double* xc, const double* yc, const int4* cv, const double2* node,
+                            double* dist) {
   int rc = CSU_OK;
   if (hipMemcpyAsync(dseg, seg.data(), seg.size() * sizeof(double), hipMemcpyHostToDevice, st) != hipSuccess)
     rc = set_err(CSU_ERR_HIP, "wall-segment upload failed");
   if (!rc && m->ncell > 0) {
-    hipLaunchKernelGGL(k_wall_dist, dim3(nblk(m->ncell)), dim3(CSU_BLOCK), 0, st, m->ncell, xc, yc, nw, dseg, dist);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(nblk(m->ncell)), dim3(CSU_BLOCK), 0, st, m->ncell, xc, yc, cv, node, m->nnode, nw,
+                         dseg, ng, dseg + 6 * (size_t)nw, dist);
+    };
+    cv ? go(k_wall_dist<true>) : go(k_wall_dist<false>);
     if (hipGetLastError() != hipSuccess) rc = set_err(CSU_ERR_HIP, "k_wall_dist launch failed");
   }
+  return rc;
+}
+
+static int wall_distance_launch(const csu_mesh_desc* m, hipStream_t st, const double* xc, const double* yc,
+                                double* dist) {
+  int nw = 0, ng = 0;
+  const std::vector<double> seg = wall_segments(m, &nw, &ng);
+  double* dseg = nullptr;
+  if (hipMalloc(&dseg, seg.size() * sizeof(double)) != hipSuccess)
+    return set_err(CSU_ERR_NOMEM, "hipMalloc of %zu wall-segment bytes failed", seg.size() * sizeof(double));
+  int rc = wall_distance_on(m, st, seg, nw, ng, dseg, xc, yc, nullptr, nullptr, dist);
   if (hipStreamSynchronize(st) != hipSuccess && !rc) rc = set_err(CSU_ERR_HIP, "k_wall_dist failed");
   (void)hipFree(dseg);
   return rc;
@@ -309,29 +336,31 @@ static int wall_distance_launch(const csu_mesh_desc* m, hipStream_t st, const do
 extern "C" int csu_wall_distance_dev(const csu_mesh_desc* m, double* wd) {
   if (!m || !wd || m->ncell <= 0 || !m->node_xy || !m->cell_vert) return set_err(CSU_ERR_ARG, "bad mesh or output");
   if (m->nbface > 0 && (!m->bface || !m->bface_mark || !m->mark_type)) return set_err(CSU_ERR_ARG, "bad boundary");
-  const int nc = m->ncell;
-  std::vector<double> xy(2 * (size_t)nc);
-  for (int i = 0; i < nc; i++) elem_center(m, i, &xy[i], &xy[nc + i]);
-  double *dxy = nullptr, *dd = nullptr;
-  if (hipMalloc(&dxy, xy.size() * sizeof(double)) != hipSuccess) return set_err(CSU_ERR_NOMEM, "hipMalloc failed");
-  if (hipMalloc(&dd, (size_t)nc * sizeof(double)) != hipSuccess) {
-    (void)hipFree(dxy);
+  const size_t nc = m->ncell, nn = m->nnode > 0 ? m->nnode : 1;
+  int nw = 0, ng = 0;
+  const std::vector<double> seg = wall_segments(m, &nw, &ng);
+  // one allocation, 16-byte parts first: nodes, cell vertices, distances,
+  // segments
+  double* buf = nullptr;
+  if (hipMalloc(&buf, (2 * nn + 2 * nc + nc + seg.size()) * sizeof(double)) != hipSuccess)
     return set_err(CSU_ERR_NOMEM, "hipMalloc failed");
-  }
+  int4* const cv = (int4*)(buf + 2 * nn);
+  double *dd = buf + 2 * nn + 2 * nc, *dseg = dd + nc;
   int rc = CSU_OK;
   hipStream_t st = nullptr;
   if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) rc = set_err(CSU_ERR_HIP, "stream");
-  if (!rc && hipMemcpyAsync(dxy, xy.data(), xy.size() * sizeof(double), hipMemcpyHostToDevice, st) != hipSuccess)
-    rc = set_err(CSU_ERR_HIP, "centre upload failed");
-  if (!rc) rc = wall_distance_launch(m, st, dxy, dxy + nc, dd);
-  if (!rc && hipMemcpyAsync(wd, dd, (size_t)nc * sizeof(double), hipMemcpyDeviceToHost, st) != hipSuccess)
+  if (!rc && (hipMemcpyAsync(buf, m->node_xy, 2 * (size_t)m->nnode * sizeof(double), hipMemcpyHostToDevice, st) !=
+                  hipSuccess ||
+              hipMemcpyAsync(cv, m->cell_vert, 4 * nc * sizeof(int32_t), hipMemcpyHostToDevice, st) != hipSuccess))
+    rc = set_err(CSU_ERR_HIP, "mesh upload failed");
+  if (!rc) rc = wall_distance_on(m, st, seg, nw, ng, dseg, nullptr, nullptr, cv, (const double2*)buf, dd);
+  if (!rc && hipMemcpyAsync(wd, dd, nc * sizeof(double), hipMemcpyDeviceToHost, st) != hipSuccess)
     rc = set_err(CSU_ERR_HIP, "wall-distance download failed");
   if (st) {
     if (hipStreamSynchronize(st) != hipSuccess && !rc) rc = set_err(CSU_ERR_HIP, "wall distance");
     (void)hipStreamDestroy(st);
   }
-  (void)hipFree(dxy);
-  (void)hipFree(dd);
+  (void)hipFree(buf);
   return rc;
 }
 
@@ -886,13 +915,16 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
       (rc = upload(d, &g.bxm, H.bxm)) || (rc = upload(d, &g.bym, H.bym)) || (rc = upload(d, &g.bnx, H.bnx)) ||
       (rc = upload(d, &g.bny, H.bny)) || (rc = upload(d, &g.bds2, H.bds2)) || (rc = upload(d, &wall_d, H.wall)) ||
       (rc = upload(d, &pref_d, pref)) ||
-      (rc = dalloc(d, &d->U, nvc)) || (rc = dalloc(d, &d->Uaux, nvc)) || (rc = dalloc(d, &d->R, nvc)) ||
+      (rc = dalloc(d, &d->U, nvc)) || (rc = dalloc(d, &d->Uaux, nvc)) ||
       (rc = dalloc(d, &d->dtl, nc + 1)) || (rc = dalloc(d, &d->dtg, ns)) ||
       (rc = dalloc(d, &d->red, 2 * (size_t)nv * d->nred + (size_t)(nc / SLOT_CELLS) + 16)) ||
-      (rc = dalloc(d, &s.P, (size_t)(nv + 1) * nc)) || (rc = dalloc(d, &s.Pb, (size_t)(nv + 1) * nb)) ||
-      (rc = dalloc(d, &s.dPx, nvc)) || (rc = dalloc(d, &s.dPy, nvc)) || (rc = dalloc(d, &s.phi, nvc)) ||
+      (rc = dalloc(d, &d->fields, 4 * nvc + 2 * (size_t)nc + (size_t)(nv + 1) * (nc + nb))) ||
       (rc = dalloc(d, &s.fflux, (size_t)nv * nf)) || (rc = dalloc(d, &s.bflux, (size_t)nv * nb)))
     return rc;
+  // what csu_dev_residual returns, in one run (one copy of a small mesh's):
+  // R, dPx, dPy, phi, dTx, dTy, P, Pb
+  d->R = d->fields; s.dPx = d->R + nvc; s.dPy = s.dPx + nvc; s.phi = s.dPy + nvc; s.dTx = s.phi + nvc;
+  s.dTy = s.dTx + nc; s.P = s.dTy + nc; s.Pb = s.P + (size_t)(nv + 1) * nc;
   d->wall = const_cast<int*>(wall_d);
   s.pref2 = const_cast<double*>(pref_d);
   if (sol) {
@@ -981,8 +1013,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     g.wdist = wdd;
   }
   if (d->visc) {
-    if ((rc = dalloc(d, &s.dTx, nc)) || (rc = dalloc(d, &s.dTy, nc)) ||
-        (rc = dalloc(d, &s.vflux, (size_t)(nv - 1) * nf)) || (rc = dalloc(d, &s.bvflux, (size_t)(nv - 1) * nb)) ||
+    if ((rc = dalloc(d, &s.vflux, (size_t)(nv - 1) * nf)) || (rc = dalloc(d, &s.bvflux, (size_t)(nv - 1) * nb)) ||
         (rc = dalloc(d, &s.wfric, 2 * (size_t)nb)) || (rc = dalloc(d, &s.miT, nf)) ||
         (rc = dalloc(d, &s.src, 2 * (size_t)nc)) || (rc = dalloc(d, &s.dq, 6 * (size_t)nc)) ||
         (rc = dalloc(d, &s.wten, 4 * (size_t)nb)))
@@ -1366,8 +1397,29 @@ extern "C" int csu_dev_residual(csu_dev* d, double* R, double* dPx, double* dPy,
   int rc = d->nv == 6 ? residual_t<6, true>(d)
            : d->nv == 5 ? residual_t<5, true>(d) : d->visc ? residual_t<4, true>(d) : residual_t<4, false>(d);
   if (rc) return rc;
-  const size_t nvc = (size_t)d->nv * d->nc;
-  const size_t nc = d->nc;
+  const size_t nvc = (size_t)d->nv * d->nc, nc = d->nc, nb = d->nb;
+  const int ns = d->nv + 1;
+  const size_t all = 4 * nvc + 2 * nc + ns * (nc + nb);
+  if (all * sizeof(double) <= RESIDUAL_ONE_COPY && d->st.P == d->fields + 4 * nvc + 2 * nc) {
+    // a small mesh: the copies' fixed cost (about 13 us each into pageable
+    // memory) outweighs the second pass over the values on the host.  1,394
+    // cells: 145 -> 68 us; above the bound the second pass costs more.
+    std::vector<double> h(all);
+    HIPCHK(hipMemcpyAsync(h.data(), d->fields, all * sizeof(double), hipMemcpyDeviceToHost, d->stream));
+    HIPCHK(hipStreamSynchronize(d->stream));
+    double* const out[4] = {R, dPx, dPy, phi};
+    for (int q = 0; q < 4; q++)
+      if (out[q]) memcpy(out[q], h.data() + q * nvc, nvc * sizeof(double));
+    if (d->visc)  // the reference's gradient slot 3 holds grad T (solverGrad_T, solver.c:477-490)
+      for (int q = 0; q < 2; q++)
+        if (out[1 + q]) memcpy(out[1 + q] + 3 * nc, h.data() + 4 * nvc + q * nc, nc * sizeof(double));
+    const double *hp = h.data() + 4 * nvc + 2 * nc, *hb = hp + ns * nc;
+    for (size_t i = 0; P && i < nc; i++)
+      for (int m = 0; m < ns; m++) P[i * ns + m] = hp[m * nc + i];
+    for (size_t i = 0; Pb && i < nb; i++)
+      for (int m = 0; m < ns; m++) Pb[i * ns + m] = hb[m * nb + i];
+    return CSU_OK;
+  }
   if (R) HIPCHK(hipMemcpyAsync(R, d->R, nvc * sizeof(double), hipMemcpyDeviceToHost, d->stream));
   if (dPx) HIPCHK(hipMemcpyAsync(dPx, d->st.dPx, nvc * sizeof(double), hipMemcpyDeviceToHost, d->stream));
   if (dPy) HIPCHK(hipMemcpyAsync(dPy, d->st.dPy, nvc * sizeof(double), hipMemcpyDeviceToHost, d->stream));
@@ -1379,7 +1431,6 @@ extern "C" int csu_dev_residual(csu_dev* d, double* R, double* dPx, double* dPy,
   }
   if (phi) HIPCHK(hipMemcpyAsync(phi, d->st.phi, nvc * sizeof(double), hipMemcpyDeviceToHost, d->stream));
   std::vector<double> tmp;
-  const int ns = d->nv + 1;
   if (P) {
     // device P is SoA [nv+1][nc]; the ABI returns [nc][nv+1]
     tmp.resize((size_t)ns * d->nc);
@@ -1611,14 +1662,13 @@ static int enqueue_iterations(csu_dev* d, int niter) {
     // the iteration count
     HIPCHK(hipStreamSynchronize(d->stream));
     graphs_drop(d);
-    dfree(d, d->res_hist, sizeof(double) * (size_t)d->hist_cap * d->nsolve * d->nv);
-    dfree(d, d->coef_hist, sizeof(double) * (size_t)d->hist_cap * d->nsolve * 4);
+    dfree(d, d->res_hist, sizeof(double) * (size_t)d->hist_cap * d->nsolve * (d->nv + 4));
     d->res_hist = d->coef_hist = nullptr;
     d->hist_cap = 0;
     int rc;
-    if ((rc = dalloc(d, &d->res_hist, (size_t)niter * d->nsolve * d->nv)) ||
-        (rc = dalloc(d, &d->coef_hist, (size_t)niter * d->nsolve * 4)))
-      return rc;
+    // norms, then forces: one copy brings both
+    if ((rc = dalloc(d, &d->res_hist, (size_t)niter * d->nsolve * (d->nv + 4)))) return rc;
+    d->coef_hist = d->res_hist + (size_t)niter * d->nsolve * d->nv;
     d->hist_cap = niter;
   }
   int rc;
@@ -1645,14 +1695,14 @@ extern "C" int csu_dev_iterate(csu_dev* d, int32_t niter, double* res, double* c
   if (res || coef) {
     // a slot holds every solve's row: [nsolve][nvar] norms, [nsolve][4] forces
     const size_t rn = (size_t)d->nsolve * d->nv, cn = (size_t)d->nsolve * 4;
-    std::vector<double> rh((size_t)d->hist_cap * rn), ch((size_t)d->hist_cap * cn);
+    std::vector<double> rh((size_t)d->hist_cap * (rn + cn));
     HIPCHK(hipMemcpyAsync(rh.data(), d->res_hist, rh.size() * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-    HIPCHK(hipMemcpyAsync(ch.data(), d->coef_hist, ch.size() * sizeof(double), hipMemcpyDeviceToHost, d->stream));
     HIPCHK(hipStreamSynchronize(d->stream));
+    const double* ch = rh.data() + (size_t)d->hist_cap * rn;
     for (int it = 0; it < niter; it++) {
       int slot = (start + it) % d->hist_cap;
       if (res) memcpy(res + (size_t)it * rn, rh.data() + (size_t)slot * rn, sizeof(double) * rn);
-      if (coef) memcpy(coef + (size_t)it * cn, ch.data() + (size_t)slot * cn, sizeof(double) * cn);
+      if (coef) memcpy(coef + (size_t)it * cn, ch + (size_t)slot * cn, sizeof(double) * cn);
     }
   }
   return prof_collect(d);
@@ -1800,9 +1850,8 @@ extern "C" int csu_batch_set_state(csu_dev* d, int32_t q, const double* U) {
   if (!U) return set_err(CSU_ERR_ARG, "null state");
   const SolveP& v = d->sol_host[q];
   const size_t n = (size_t)(v.c1 - v.c0);
-  for (int k = 0; k < d->nv; k++)
-    HIPCHK(hipMemcpyAsync(d->U + (size_t)k * d->nc + v.c0, U + k * n, n * sizeof(double), hipMemcpyHostToDevice,
-                          d->stream));
+  HIPCHK(hipMemcpy2DAsync(d->U + v.c0, (size_t)d->nc * sizeof(double), U, n * sizeof(double), n * sizeof(double), d->nv,
+                          hipMemcpyHostToDevice, d->stream));
   HIPCHK(hipStreamSynchronize(d->stream));
   d->fresh = 1;
   return CSU_OK;
@@ -1814,9 +1863,8 @@ extern "C" int csu_batch_get_state(csu_dev* d, int32_t q, double* U) {
   if (!U) return set_err(CSU_ERR_ARG, "null state");
   const SolveP& v = d->sol_host[q];
   const size_t n = (size_t)(v.c1 - v.c0);
-  for (int k = 0; k < d->nv; k++)
-    HIPCHK(hipMemcpyAsync(U + k * n, d->U + (size_t)k * d->nc + v.c0, n * sizeof(double), hipMemcpyDeviceToHost,
-                          d->stream));
+  HIPCHK(hipMemcpy2DAsync(U, n * sizeof(double), d->U + v.c0, (size_t)d->nc * sizeof(double), n * sizeof(double), d->nv,
+                          hipMemcpyDeviceToHost, d->stream));
   HIPCHK(hipStreamSynchronize(d->stream));
   return CSU_OK;
 }
@@ -2275,9 +2323,9 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
   double b = 0;
   b += nc * (4 + 16 + 16 + 48 + 64 + 64 + 8) + nf * (8 + 1 + 24) + nb * (12 + 64 + 4);  // geometry
   b += nc * (24 * nv + 8) + 2 * nv * 8 * (nc / 256 + 1) + 8 * (nc / SLOT_CELLS) + 128;                           // U, Uaux, R, dt, reductions
-  b += (nv + 1) * 8 * (nc + nb) + 24 * nv * nc + 8 * nv * nf;                             // P, Pb, grad, phi, fflux
+  b += (nv + 1) * 8 * (nc + nb) + (24 * nv + 16) * nc + 8 * nv * nf;                      // P, Pb, grad, phi, fflux
   if (p->order == 2) b += 32 * nv * nc;                                                   // edge states
-  if (visc) b += nc * (16 + 16 + 48) + nf * (8 * (nv - 1) + 8) + nb * (8 * (nv - 1) + 16);
+  if (visc) b += nc * (16 + 48) + nf * (8 * (nv - 1) + 8) + nb * (8 * (nv - 1) + 16);
   if (p->time_scheme != CSU_TIME_RK) b += nc * (8 + 16 * nv + 8 + 16);
   if (p->time_scheme == CSU_TIME_LUSGS) b += nc * 24 + nf * 24;
   if (p->time_scheme == CSU_TIME_DPLUR) b += 32 * nv * nv * nc + 8.0 * (p->nlinear > 0 ? p->nlinear : 1) * (nc / 256 + 1);
