@@ -1028,10 +1028,10 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     HIPCHK(hipMemsetAsync(d->dW1, 0, nvc * sizeof(double), d->stream));   // implicitInitDPLUR
   }
   if (p->time_scheme == CSU_TIME_DPLUR) {
-    if ((rc = dalloc(d, &d->A, (size_t)4 * nv * nv * nc)) || (rc = dalloc(d, &d->jstate, 2 * (size_t)ns)) ||
+    if ((rc = dalloc(d, &d->A, block_total(nv, nc))) || (rc = dalloc(d, &d->jstate, 2 * (size_t)ns)) ||
         (rc = dalloc(d, &d->jred, (size_t)(p->nlinear > 0 ? p->nlinear : 1) * nblk(nc))))
       return rc;
-    HIPCHK(hipMemsetAsync(d->A, 0, (size_t)4 * nv * nv * nc * sizeof(double), d->stream));
+    HIPCHK(hipMemsetAsync(d->A, 0, block_total(nv, nc) * sizeof(double), d->stream));
     HIPCHK(hipMemsetAsync(d->jstate, 0, 2 * sizeof(int) * (size_t)ns, d->stream));
   }
   if (p->time_scheme == CSU_TIME_LUSGS) {
@@ -1634,10 +1634,10 @@ static int implicit_iteration(csu_dev* d) {
     for (int mm = 0; mm < d->prm.nlinear; mm++)
       hipLaunchKernelGGL(k_jacobi<NV>, dim3(nb), dim3(CSU_BLOCK), 0, d->stream, kp, d->geo, d->A, d->Dp, d->dtg,
                          d->R, d->dW0, d->dW1, (const int*)d->jstate, d->jred, mm, d->st.dq);
+    hipLaunchKernelGGL(k_jac_base, dim3(d->nsolve), dim3(64), 0, d->stream, d->jstate, (const double*)d->jred,
+                       d->prm.nlinear, nb, d->geo.sol);
     hipLaunchKernelGGL(k_upd_imp<NV>, dim3(nb), dim3(CSU_BLOCK), 0, d->stream, nc, d->U, d->dW0, d->dW1,
-                       (const int*)d->jstate, (const double*)d->jred, d->prm.nlinear, nb, d->geo.sol, d->geo.csolk);
-    hipLaunchKernelGGL(k_jac_base, dim3((d->nsolve + 63) / 64), dim3(64), 0, d->stream, d->jstate,
-                       (const double*)d->jred, d->prm.nlinear, nb, d->geo.sol, d->nsolve);
+                       (const int*)d->jstate, d->geo.sol, d->geo.csolk);
   }
   HIPCHK(hipGetLastError());
   return CSU_OK;
@@ -1719,7 +1719,7 @@ static int tune_reset(csu_dev* d, const double* saved) {
   HIPCHK(hipMemsetAsync(d->hctr, 0, 2 * sizeof(int), d->stream));
   if (d->dW0) HIPCHK(hipMemsetAsync(d->dW0, 0, nvc * sizeof(double), d->stream));
   if (d->dW1) HIPCHK(hipMemsetAsync(d->dW1, 0, nvc * sizeof(double), d->stream));
-  if (d->A) HIPCHK(hipMemsetAsync(d->A, 0, (size_t)4 * d->nv * d->nv * d->nc * sizeof(double), d->stream));
+  if (d->A) HIPCHK(hipMemsetAsync(d->A, 0, block_total(d->nv, d->nc) * sizeof(double), d->stream));
   if (d->jstate) HIPCHK(hipMemsetAsync(d->jstate, 0, 2 * sizeof(int) * (size_t)d->nsolve, d->stream));
   HIPCHK(hipStreamSynchronize(d->stream));
   d->iter = 0;
@@ -2328,7 +2328,7 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
   if (visc) b += nc * (16 + 48) + nf * (8 * (nv - 1) + 8) + nb * (8 * (nv - 1) + 16);
   if (p->time_scheme != CSU_TIME_RK) b += nc * (8 + 16 * nv + 8 + 16);
   if (p->time_scheme == CSU_TIME_LUSGS) b += nc * 24 + nf * 24;
-  if (p->time_scheme == CSU_TIME_DPLUR) b += 32 * nv * nv * nc + 8.0 * (p->nlinear > 0 ? p->nlinear : 1) * (nc / 256 + 1);
+  if (p->time_scheme == CSU_TIME_DPLUR) b += 8.0 * block_total((int)nv, m->ncell) + 8.0 * (p->nlinear > 0 ? p->nlinear : 1) * (nc / 256 + 1);
   if (p->precision == 1) b += nc * 64 + nf * (12 + 4 * nv) + (p->order == 2 ? 16 * nv * nc : 0);  // FP32 copies
   if (p->time_scheme == CSU_TIME_RK && !visc && p->order == 2 && p->limiter != 1 && m->axi == 0 && p->tp == 0) {
     // tile form: second primitive buffer, places, face copies, halo cells (at
