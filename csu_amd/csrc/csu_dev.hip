@@ -89,7 +89,7 @@ struct csu_dev {
   int tile_nt;                 // threads per tile
   int tl_capb;                 // boundary entries its LDS array holds
   size_t tl_n;                 // interior entries in all
-  double* P2;                  // tile form: second primitive buffer (a stage never writes the buffer it reads)
+  dbl2 *Pa, *Pb4;              // tile form: primitives r u v p [nc][4], current and the one a stage writes
   int tuned;                   // launch shapes from the autotuner (1) or the defaults (0)
   // implicit schemes
   double *Dp, *dW0, *dW1, *A;  // diagonal (without the dt term), increments, DPLUR blocks
@@ -102,7 +102,8 @@ struct csu_dev {
   // step x which buffer holds U; implicit keyed by nothing
   int* hctr;                   // device iteration counter (slot of res/coef history), k_tail's finished workgroups
   hipGraphExec_t gexec[4];
-  double *gU[4], *gP[4];       // d->U, d->st.P at capture
+  double* gU[4];               // d->U at capture
+  dbl2* gP[4];                 // d->Pa at capture
   double* Ubase;               // the buffer U starts in (graph parity key)
   size_t bytes;                // device bytes allocated by this context
   // asynchronous iteration: history rows copied to pinned host memory
@@ -900,13 +901,16 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   Geo& g = d->geo;
   St& s = d->st;
   const size_t nvc = (size_t)nv * nc;
+  std::vector<double> wg(16 * (size_t)nc);  // weights and edge offsets, cell by cell
+  for (size_t t = 0; t < 4 * (size_t)nc; t++) {
+    wg[4 * t] = H.lwx[t]; wg[4 * t + 1] = H.lwy[t]; wg[4 * t + 2] = H.edx[t]; wg[4 * t + 3] = H.edy[t];
+  }
   const double* pref_d = nullptr;
   const int* wall_d = nullptr;
   if ((rc = upload(d, &g.cnp, H.cnp)) || (rc = upload(d, &g.cnbr, H.cnbr)) || (rc = upload(d, &g.cface, H.cface)) ||
       (rc = upload(d, &g.xc, H.xc)) || (rc = upload(d, &g.yc, H.yc)) || (rc = upload(d, &g.omega, H.om)) ||
       (rc = upload(d, &g.dsxm, H.dsxm)) || (rc = upload(d, &g.dsym, H.dsym)) || (rc = upload(d, &g.dslat, H.dslat)) ||
-      (rc = upload(d, &g.edx, H.edx)) || (rc = upload(d, &g.edy, H.edy)) ||
-      (rc = upload(d, &g.lwx, H.lwx)) || (rc = upload(d, &g.lwy, H.lwy)) || (rc = upload(d, &g.fsl, H.fsl)) ||
+      (rc = upload(d, &g.wg, wg)) || (rc = upload(d, &g.fsl, H.fsl)) ||
       (rc = upload(d, &g.bmask, H.bmask)) ||
       (rc = upload(d, &g.fe0, H.fe0)) || (rc = upload(d, &g.fe1, H.fe1)) || (rc = upload(d, &g.fdsx, H.fdsx)) ||
       (rc = upload(d, &g.fdsy, H.fdsy)) || (rc = upload(d, &g.fds, H.fds)) ||
@@ -967,7 +971,8 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
           (rc = upload(d, &tl.bown, T.bown)) || (rc = upload(d, &tl.hoff, T.hoff)) || (rc = upload(d, &tl.tbq, T.tbq)) || (rc = upload(d, &tl.tbc, T.tbc)) ||
           (rc = upload(d, &tl.hcell, T.hcell)) || (rc = upload(d, &tl.fx, T.fx)) || (rc = upload(d, &tl.fy, T.fy)) ||
           (rc = upload(d, &tl.fs, T.fs)) || (rc = upload(d, &tl.csl, T.csl)) || (rc = upload(d, &tl.hsl, T.hsl)) ||
-          (rc = upload(d, &tl.cel, T.cel)) || (rc = upload(d, &tl.hel, T.hel)) || (rc = dalloc(d, &d->P2, 5 * (size_t)nc)))
+          (rc = upload(d, &tl.cel, T.cel)) || (rc = upload(d, &tl.hel, T.hel)) || (rc = dalloc(d, &d->Pa, 2 * (size_t)nc)) ||
+          (rc = dalloc(d, &d->Pb4, 2 * (size_t)nc)))
         return rc;
       if (kp.mixed) {
         auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
@@ -987,8 +992,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   else if (!d->tuned && (double)d->tl.nh <= 1.25 * nc) d->tile = 1;
   if (kp.mixed) {
     auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
-    if ((rc = upload(d, &g.lwx32, f32(H.lwx))) || (rc = upload(d, &g.lwy32, f32(H.lwy))) ||
-        (rc = upload(d, &g.edx32, f32(H.edx))) || (rc = upload(d, &g.edy32, f32(H.edy))) ||
+    if ((rc = upload(d, &g.wg32, f32(wg))) ||
         (rc = upload(d, &g.fdsx32, f32(H.fdsx))) || (rc = upload(d, &g.fdsy32, f32(H.fdsy))) ||
         (rc = upload(d, &g.fds32, f32(H.fds))) || (rc = dalloc(d, &s.fflux32, (size_t)nv * nf)) ||
         (p->order == 2 && (rc = dalloc(d, &s.rec32, 4 * nvc))))
@@ -1083,12 +1087,12 @@ static csu_dev* dev_new() {
   d->Dp = d->dW0 = d->dW1 = d->A = d->caux = nullptr; d->jstate = nullptr; d->jred = nullptr; d->cellsL = d->cellsU = nullptr;
   d->hctr = nullptr; d->use_graphs = 1; d->bytes = 0; d->tstate = nullptr;
   d->hres = d->hcoef = nullptr; d->hcap = 0; d->async_start = 0; d->async_n = 0;
-  for (int k = 0; k < 4; k++) { d->gexec[k] = nullptr; d->gU[k] = d->gP[k] = nullptr; }
+  for (int k = 0; k < 4; k++) { d->gexec[k] = nullptr; d->gU[k] = nullptr; d->gP[k] = nullptr; }
   memset((void*)&d->kp, 0, sizeof(KP));
   memset((void*)&d->geo, 0, sizeof(Geo));
   memset((void*)&d->st, 0, sizeof(St));
   memset((void*)&d->tl, 0, sizeof(Tile));
-  d->P2 = nullptr; d->quads = 1; d->tl_capb = 0; d->tl_n = 0;
+  d->Pa = d->Pb4 = nullptr; d->quads = 1; d->tl_capb = 0; d->tl_n = 0;
   return d;
 }
 
@@ -1358,7 +1362,7 @@ static int tile_stage(csu_dev* d, int flags, double sigma, double rk_a) {
   Prof p(d, "k_stage");
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, gu, bu, lds, d->stream, kp, d->geo, st, d->tl, flags, sigma, rk_a, d->prm.cfl, d->dtl,
-                       d->dtg, d->U, d->Uaux, d->P2, d->red, rdt);
+                       d->dtg, d->U, d->Uaux, (const dbl2*)d->Pa, d->Pb4, d->red, rdt);
   };
   const bool roe = kp.flux == 0;
   if (kp.lsq_ld) go(k_stage<NT, 4, -1, false, true>);
@@ -1366,7 +1370,7 @@ static int tile_stage(csu_dev* d, int flags, double sigma, double rk_a) {
   else if (kp.mixed) roe ? go(k_stage<NT, 4, 0, true, false>) : go(k_stage<NT, 4, -1, true, false>);
   else if (!d->quads) roe ? go(k_stage<NT, 3, 0, false, false>) : go(k_stage<NT, 3, -1, false, false>);
   else roe ? go(k_stage<NT, 4, 0, false, false>) : go(k_stage<NT, 4, -1, false, false>);
-  std::swap(d->st.P, d->P2);
+  std::swap(d->Pa, d->Pb4);
   HIPCHK(hipGetLastError());
   return CSU_OK;
 }
@@ -1400,7 +1404,7 @@ extern "C" int csu_dev_residual(csu_dev* d, double* R, double* dPx, double* dPy,
   const size_t nvc = (size_t)d->nv * d->nc, nc = d->nc, nb = d->nb;
   const int ns = d->nv + 1;
   const size_t all = 4 * nvc + 2 * nc + ns * (nc + nb);
-  if (all * sizeof(double) <= RESIDUAL_ONE_COPY && d->st.P == d->fields + 4 * nvc + 2 * nc) {
+  if (all * sizeof(double) <= RESIDUAL_ONE_COPY) {
     // a small mesh: the copies' fixed cost (about 13 us each into pageable
     // memory) outweighs the second pass over the values on the host.  1,394
     // cells: 145 -> 68 us; above the bound the second pass costs more.
@@ -1499,10 +1503,11 @@ static int is_local(const csu_dev* d, int it) {
 // replay slot k when it was captured with the same U buffer.
 template <typename F>
 static int run_graph(csu_dev* d, int k, F body) {
-  if (!d->gexec[k] || d->gU[k] != d->U || d->gP[k] != d->st.P) {
+  if (!d->gexec[k] || d->gU[k] != d->U || d->gP[k] != d->Pa) {
     if (d->gexec[k]) (void)hipGraphExecDestroy(d->gexec[k]);
     d->gexec[k] = nullptr;
-    double *u0 = d->U, *p0 = d->st.P;
+    double* u0 = d->U;
+    dbl2* p0 = d->Pa;
     HIPCHK(hipStreamBeginCapture(d->stream, hipStreamCaptureModeThreadLocal));
     int rc = body();
     hipGraph_t graph = nullptr;
@@ -1540,6 +1545,8 @@ static int rk_iteration(csu_dev* d, int it_index) {
                          d->dtg, d->geo.sol);
     int rc = prim_pass<NV>(d);
     if (rc) return rc;
+    if (d->tile)
+      hipLaunchKernelGGL(k_pack4, dim3(nblk(nc)), dim3(CSU_BLOCK), 0, d->stream, nc, (const double*)d->st.P, d->Pa);
     first_flags = 0;
     d->fresh = 0;
   }
@@ -1811,6 +1818,9 @@ extern "C" int csu_dev_set_launch_shape(csu_dev* d, const int32_t* choice) {
     return set_err(CSU_ERR_ARG, "the tile form needs an inviscid second-order RK run whose tiles fit");
   HIPCHK(hipStreamSynchronize(d->stream));
   graphs_drop(d);  // the shapes are part of the captured launches
+  // the two forms hold the primitives between iterations in different
+  // layouts: the next iteration derives them (and its time step) again
+  if (choice[3] != d->tile) d->fresh = 1;
   d->sblk = choice[0];
   d->lblk = choice[1];
   d->kp.xcd = choice[2];
@@ -2040,8 +2050,7 @@ extern "C" int csu_dev_set_precision(csu_dev* d, int32_t prec) {
     return hipGetLastError() == hipSuccess ? CSU_OK : set_err(CSU_ERR_HIP, "k_to_f32 launch");
   };
   if (prec == CSU_PREC_MIXED) {
-    if (!g.lwx32 && ((rc = f32(g.lwx, &g.lwx32, 4 * nc)) || (rc = f32(g.lwy, &g.lwy32, 4 * nc)) ||
-                     (rc = f32(g.edx, &g.edx32, 4 * nc)) || (rc = f32(g.edy, &g.edy32, 4 * nc)) ||
+    if (!g.wg32 && ((rc = f32(g.wg, &g.wg32, 16 * nc)) ||
                      (rc = f32(g.fdsx, &g.fdsx32, nf)) || (rc = f32(g.fdsy, &g.fdsy32, nf)) ||
                      (rc = f32(g.fds, &g.fds32, nf))))
       return rc;
@@ -2331,11 +2340,11 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
   if (p->time_scheme == CSU_TIME_DPLUR) b += 8.0 * block_total((int)nv, m->ncell) + 8.0 * (p->nlinear > 0 ? p->nlinear : 1) * (nc / 256 + 1);
   if (p->precision == 1) b += nc * 64 + nf * (12 + 4 * nv) + (p->order == 2 ? 16 * nv * nc : 0);  // FP32 copies
   if (p->time_scheme == CSU_TIME_RK && !visc && p->order == 2 && p->limiter != 1 && m->axi == 0 && p->tp == 0) {
-    // tile form: second primitive buffer, places, face copies, halo cells (at
+    // tile form: its two primitive buffers, places, face copies, halo cells (at
     // most one per tile and face between two tiles)
     double cross = 0;
     for (int f = 0; f < m->nface; f++) cross += m->face[4 * (size_t)f] / CSU_CHUNK != m->face[4 * (size_t)f + 1] / CSU_CHUNK;
-    b += nc * (40 + 16) + (nf + cross) * (p->precision == 1 ? 36 : 24) + 2 * cross * 20 + 12 * nb + 16 * (nc / 256 + 2);
+    b += nc * (64 + 16) + (nf + cross) * (p->precision == 1 ? 36 : 24) + 2 * cross * 20 + 12 * nb + 16 * (nc / 256 + 2);
   }
   b += (nv + 4) * 8 * (double)(hist > 0 ? hist : 1);
   // allocation granularity: every array rounds up (at most 2 MiB slack per large array)

@@ -125,11 +125,13 @@ struct Geo {
   const int *cnp, *cnbr, *cface;                        // [nc], [4][nc], [4][nc]
   const int* cfn;  // implicit schemes: [4][nc] the other cell of face slot j, -1 where cface is 0
   const double *xc, *yc, *omega, *dsxm, *dsym, *dslat;  // [nc]
-  const double *edx, *edy;                              // [4][nc] own-edge midpoint offsets
-  const double *lwx, *lwy;                              // [4][nc] LSQ weights per neighbour slot
+  // [4][nc] x {LSQ weights wx, wy of neighbour slot j, midpoint offsets ex, ey
+  // of edge j}: a cell's four values are one 32-byte run (two loads, not four
+  // from as many planes)
+  const double* wg;
   const unsigned char* fsl;                             // [nf] edge of the face in e0 (bits 0-1), e1 (2-3)
   const unsigned char* bmask;                           // [nc] bit j: neighbour slot j is a boundary face
-  const float *lwx32, *lwy32, *edx32, *edy32;           // mixed precision copies of lwx, lwy, edx, edy
+  const float* wg32;                                    // mixed precision copy of wg
   const float *fdsx32, *fdsy32, *fds32;                 // mixed precision face vectors
   const double *wdist;                                  // [nc] wall distance (SA/SST)
   const int *fe0, *fe1;                                 // [nf]
@@ -138,6 +140,9 @@ struct Geo {
   const int *be0, *btype, *bdonor;                      // [nb]
   const double *bdsx, *bdsy, *bds, *bxm, *bym, *bnx, *bny, *bds2;
 };
+
+typedef double dbl2 __attribute__((ext_vector_type(2)));
+typedef float flt4 __attribute__((ext_vector_type(4)));
 
 // Mutable per-stage arrays, passed by value.
 struct St {

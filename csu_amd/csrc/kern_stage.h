@@ -44,13 +44,32 @@ struct Tile {
   int capf;                         // interior entries the LDS array holds
 };
 
+// Primitives r u v p of cell i: [nc][4], one 32-byte run per gathered
+// neighbour instead of one line in each of four planes.
+__device__ __forceinline__ void load4(const dbl2* P, int i, double* v) {
+  const dbl2 a = P[2 * (size_t)i], b = P[2 * (size_t)i + 1];
+  v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+}
+__device__ __forceinline__ void store4(dbl2* P, int i, const double* v) {
+  P[2 * (size_t)i] = dbl2{v[0], v[1]};
+  P[2 * (size_t)i + 1] = dbl2{v[2], v[3]};
+}
+// That layout from the planes k_prim writes (after the state was set from the
+// host).
+__global__ __launch_bounds__(CSU_BLOCK) void k_pack4(int nc, const double* __restrict__ P, dbl2* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nc) return;
+  const double v[4] = {P[i], P[nc + i], P[2 * nc + i], P[3 * nc + i]};
+  store4(out, i, v);
+}
+
 // Phase 1 of one cell: its reconstructed edge states into the halves of the
 // tile's faces (sf: [8][cap], left then right state).  sl, el: the cell's
 // slot and edge places; sb: the boundary entries ([place][8]: flux, ghost
 // state).
 template <int NE, bool MIX, bool LD, typename TF>
 __device__ __forceinline__ void stage_cell(const KP& kp, const Geo& g, const St& s, const Tile& tl,
-                                           const SolveP* sv, const double* __restrict__ pref, int i, const short* sl,
+                                           const dbl2* __restrict__ Pin, const SolveP* sv, const double* __restrict__ pref, int i, const short* sl,
                                            const short* el, int lst, TF* sf, const double* sb) {
   const int nc = kp.nc, cap = tl.capf;
   // NE 3: a mesh of triangles only; 4: slot 3 exists for quads
@@ -58,34 +77,25 @@ __device__ __forceinline__ void stage_cell(const KP& kp, const Geo& g, const St&
   int nbr[4];
 #pragma unroll
   for (int j = 0; j < NE; j++) nbr[j] = j == 3 && np < 4 ? i : g.cnbr[j * nc + i];
-  double Pi[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) Pi[k] = s.P[k * nc + i];
-  double un[4][4];
+  double Pi[4], un[4][4];
+  load4(Pin, i, Pi);
 #pragma unroll
   for (int j = 0; j < NE; j++) {
     if (j == 3 && np < 4) break;
-    const int n = nbr[j] >= 0 ? nbr[j] : i;
-#pragma unroll
-    for (int k = 0; k < 4; k++) un[j][k] = s.P[k * nc + n];
+    load4(Pin, nbr[j] >= 0 ? nbr[j] : i, un[j]);
   }
   TF ex[4], ey[4], wx[4], wy[4];
 #pragma unroll
   for (int j = 0; j < NE; j++) {
     ex[j] = ey[j] = wx[j] = wy[j] = 0;
     if (j == 3 && np < 4) break;
+    const size_t w = 4 * ((size_t)j * nc + i);
     if (MIX) {
-      ex[j] = g.edx32[j * nc + i];
-      ey[j] = g.edy32[j * nc + i];
-      wx[j] = g.lwx32[j * nc + i];
-      wy[j] = g.lwy32[j * nc + i];
+      const flt4 v = *(const flt4*)(g.wg32 + w);
+      wx[j] = v.x; wy[j] = v.y; ex[j] = v.z; ey[j] = v.w;
     } else {
-      ex[j] = g.edx[j * nc + i];
-      ey[j] = g.edy[j * nc + i];
-      if (!LD) {
-        wx[j] = g.lwx[j * nc + i];
-        wy[j] = g.lwy[j * nc + i];
-      }
+      const dbl2 v = *(const dbl2*)(g.wg + w), e = *((const dbl2*)(g.wg + w) + 1);
+      wx[j] = v.x; wy[j] = v.y; ex[j] = e.x; ey[j] = e.y;
     }
   }
   int pl[4];
@@ -194,13 +204,12 @@ __device__ __forceinline__ void stage_cell(const KP& kp, const Geo& g, const St&
 // for one of the tile's own cells, its convective flux (bc_flux,
 // kern_common.h, with the two states at hand).
 template <int FLX>
-__device__ __forceinline__ void stage_bface(const KP& kp, const Geo& g, const St& s, int q, int i, bool own,
-                                            bool lastst, double* o) {
-  const int nc = kp.nc, nb = kp.nb, type = g.btype[q];
+__device__ __forceinline__ void stage_bface(const KP& kp, const Geo& g, const St& s, const dbl2* Pin, int q, int i,
+                                            bool own, bool lastst, double* o) {
+  const int nb = kp.nb, type = g.btype[q];
   const double dSx = g.bdsx[q], dSy = g.bdsy[q], dS = g.bds[q];
   double PL[4], PR[5], fl[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) PL[k] = s.P[k * nc + i];
+  load4(Pin, i, PL);
   ghost_state<4>(kp, type, dSx, dSy, dS, PL, 0.0, PR);
 #pragma unroll
   for (int k = 0; k < 4; k++) o[4 + k] = PR[k];
@@ -223,7 +232,7 @@ __device__ __forceinline__ void stage_bface(const KP& kp, const Geo& g, const St
   for (int k = 0; k < 4; k++) o[k] = dS > 0 ? 0.0 + fl[k] * dS : 0.0;
 }
 
-// One RK stage: the primitives r u v p of the stage's state (s.P, read with
+// One RK stage: the primitives r u v p of the stage's state (Pin, read with
 // the neighbours' and the halo's) -> those of the next stage's state (Pout,
 // another buffer); the last stage also writes the state (Uout).  Un, the
 // iteration's start state, is clamped where it is used (F_CLAMP_UN:
@@ -235,7 +244,8 @@ __device__ __forceinline__ void stage_bface(const KP& kp, const Geo& g, const St
 template <int NT, int NE, int FLX, bool MIX, bool LD>
 __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, int flags, double sigma, double rk_a,
                                               double cfl, double* dtl, const double* dtg,
-                                              const double* __restrict__ Un, double* __restrict__ Uout, double* __restrict__ Pout,
+                                              const double* __restrict__ Un, double* __restrict__ Uout,
+                                              const dbl2* __restrict__ Pin, dbl2* __restrict__ Pout,
                                               double* __restrict__ red_res, double* __restrict__ red_dt) {
   using TF = typename std::conditional<MIX, float, double>::type;
   kp.gas.tp = 0;  // the tile form exists for the ideal gas only
@@ -264,14 +274,14 @@ __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, in
 #pragma unroll
     for (int k = 0; k < 7; k++) kb.pin[k] = sv ? sv->pin[k] : kp.pin[k];
     for (int k = t; k < nbt; k += NT)
-      stage_bface<FLX>(kb, g, s, tl.tbq[b0 + k], tl.tbc[b0 + k], k < tl.bown[tile], lastst, sb + 8 * k);
+      stage_bface<FLX>(kb, g, s, Pin, tl.tbq[b0 + k], tl.tbc[b0 + k], k < tl.bown[tile], lastst, sb + 8 * k);
     __syncthreads();
   }
   for (int k = t; k < CSU_CHUNK + nh; k += NT) {
     const bool own = k < CSU_CHUNK;
     if (own && k >= nown) continue;
     const int h = h0 + k - CSU_CHUNK, i = own ? c0 + k : tl.hcell[h];
-    stage_cell<NE, MIX, LD, TF>(kp, g, s, tl, sv, s.pref2 + 6 * sid, i, own ? tl.csl + i : tl.hsl + h, own ? tl.cel + i : tl.hel + h,
+    stage_cell<NE, MIX, LD, TF>(kp, g, s, tl, Pin, sv, s.pref2 + 6 * sid, i, own ? tl.csl + i : tl.hsl + h, own ? tl.cel + i : tl.hel + h,
                             own ? nc : tl.nh, sf, sb);
   }
   __syncthreads();
@@ -343,8 +353,7 @@ __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, in
       for (int kk = 0; kk < 4; kk++) Uout[kk * nc + i] = unew[kk];
     }
     prim_point<4>(kp, unew, p);
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) Pout[kk * nc + i] = p[kk];
+    store4(Pout, i, p);
   }
   if (!lastst) return;
   // residual-norm partials and time-step minimum, as k_update's

@@ -155,17 +155,21 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   // every cell has slots 0-2; slot 3 (quads only) is read only by quads,
   // a branch that is uniform on triangle and quad meshes alike
   TF ex[4] = {0, 0, 0, 0}, ey[4] = {0, 0, 0, 0};
+  TF wx[4] = {0, 0, 0, 0}, wy[4] = {0, 0, 0, 0};  // past np the weight is 0
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     if (j == 3 && np < 4) break;
+    const size_t w = 4 * ((size_t)j * nc + i);
     if (MIX) {
-      ex[j] = g.edx32[j * nc + i];
-      ey[j] = g.edy32[j * nc + i];
+      const flt4 v = *(const flt4*)(g.wg32 + w);
+      wx[j] = v.x; wy[j] = v.y; ex[j] = v.z; ey[j] = v.w;
     } else {
-      // read once per stage: non-temporal, so they do not displace the
-      // neighbour states in the caches
-      ex[j] = __builtin_nontemporal_load(&g.edx[j * nc + i]);
-      ey[j] = __builtin_nontemporal_load(&g.edy[j * nc + i]);
+      const dbl2 e = *((const dbl2*)(g.wg + w) + 1);
+      ex[j] = e.x; ey[j] = e.y;
+      if (!LD) {
+        const dbl2 v = *(const dbl2*)(g.wg + w);
+        wx[j] = v.x; wy[j] = v.y;
+      }
     }
   }
   // Least squares (solver.c:1031-1074).  Default: gx = sum_j wx_j du_j with
@@ -173,7 +177,6 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
   // cell in long double.  LD: the normal-equation sums of every call in
   // double-double, as the reference's x87 long double accumulators do.
   dd a = {0, 0}, b = {0, 0}, c = {0, 0}, det = {0, 0}, nb_ = {0, 0};
-  TF wx[4], wy[4];
   if (LD) {
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -184,21 +187,6 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_grad(KP kp, Geo g, St s) {
     }
     det = dd_sub(dd_mul(a, c), dd_mul(b, b));
     nb_ = dd_neg(b);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      // slot 3 only for quads (past np the weight is 0)
-      wx[j] = 0;
-      wy[j] = 0;
-      if (j == 3 && np < 4) break;
-      if (MIX) {
-        wx[j] = g.lwx32[j * nc + i];
-        wy[j] = g.lwy32[j * nc + i];
-      } else {
-        wx[j] = __builtin_nontemporal_load(&g.lwx[j * nc + i]);
-        wy[j] = __builtin_nontemporal_load(&g.lwy[j * nc + i]);
-      }
-    }
   }
   auto grad = [&](const double* du, double& gx, double& gy) {
     if (LD) {
