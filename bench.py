@@ -39,60 +39,42 @@ HBM_PEAK_GBS = 8000.0
 def alg_bytes(kernel: str, nc: int, nf: int, nb: int, nv: int, pu: bool = False, tile_entries: int = 0) -> float:
     """Compulsory HBM bytes of one launch: every array the kernel must touch,
     each element counted once (neighbour re-reads are cache traffic).
-    pu: the stages recover the primitives from the conservative state (the
-    inviscid RK form), so k_grad reads U instead of P and k_update writes no
-    P.  tile_entries > 0: the tile form, whose k_update also evaluates the
-    face fluxes (the face kernel's bytes without the face-flux array, plus
-    the tiles' face lists of that many entries)."""
+    pu: the stages pass primitives r u v p to each other (the inviscid RK
+    form), so k_grad reads and k_update writes four rows and no state.
+    tile_entries > 0: the tile form, one kernel per stage (k_stage), with the
+    tiles' face lists of that many entries."""
     ns = nv + 1
     if kernel == "k_prim":
         return nc * (8 * nv + 8 * ns)
     edges = 2 * nf + nb                 # cell-edge slots (interior faces count twice)
     if kernel == "k_grad":
-        # own P (or U), cnp, cnbr, omega; per slot LSQ weights and edge
-        # offsets; the edge states written; ghost states read
-        return nc * (8 * (nv if pu else ns) + 4 + 16 + 8) + edges * (16 + 16 + 8 * nv) + nb * 8 * ns
+        # own P, cnp, cnbr, omega; per slot LSQ weights and edge offsets; the
+        # edge states written; ghost states written and read
+        return nc * (8 * (nv if pu else ns) + 4 + 16 + 8) + edges * (16 + 16 + 8 * nv) + nb * 16 * ns
     if kernel == "k_flux":
         # e0, e1, edge slots, face vector; both edge states; the flux
         return nf * (8 + 1 + 24 + 2 * 8 * nv + 8 * nv)
-    if kernel == "k_update" and tile_entries:
-        # each face's e0, e1, edge slots, face vector and both edge states;
-        # the tiles' face lists; per cell the slots' list places, boundary
-        # mask, U^n, U out, dt; boundary fluxes
-        return (nf * (8 + 1 + 24 + 2 * 8 * nv) + tile_entries * 4 + (nc // 256 + 1) * 4
-                + nc * (8 + 1 + 8 * nv * 2 + 8 + 8) + nb * 8 * nv)
+    if kernel == "k_stage":
+        # P in and out, U^n, dt, omega, neighbours; per slot weights, offsets
+        # and two places in the tile's lists; each entry's face vector; per
+        # boundary face its geometry and ids
+        return (nc * (3 * 8 * nv + 8 + 8 + 16 + 1) + edges * (32 + 4) + tile_entries * 24 + nb * 36
+                + (nc // 256 + 1) * 16)
     if kernel == "k_update":
-        # face list, boundary mask, U^n, U out, P out (not with pu), omega,
-        # dt; each face flux once
+        # face list, boundary mask, U^n, U and P out (pu: P only), omega, dt;
+        # each face flux once
         return nc * (16 + 1 + 8 * nv * 2 + (0 if pu else 8 * ns) + 8 + 8) + nf * 8 * nv + nb * 8 * nv
     return 0.0
 
 
-# HBM bytes per launch on the default 2000x1000x2 workload (primitives-from-
-# state stages), from rocprofv3 FETCH_SIZE (x2.0) and WRITE_SIZE (x1.0)
-# passes, both scaled by what the counters read for the library's streaming
-# kernel (1 GiB read, 1 GiB written), per launch shape (gradient/face
-# workgroup size, XCD tile map, tile form; the residual kernel always runs
-# 256-thread workgroups) and cell order: the bytes depend on them through
-# the caches.  A counter
+# HBM bytes per launch on the default 2000x1000x2 workload, from rocprofv3
+# FETCH_SIZE (x2.0) and WRITE_SIZE (x1.0) passes, both scaled by what the
+# counters read for the library's streaming kernel (1 GiB read, 1 GiB
+# written), per launch shape (gradient/face workgroup size, XCD tile map, tile
+# form) and cell order: the bytes depend on them through the caches.  A counter
 # pass cannot run inside this timed process, so the figure is reported for
 # that workload and the shapes measured only.
-MEASURED_TRAFFIC = {("k_grad", 2000, 1000, 128, 0, 0, "column"): 1089.2e6,
-                    ("k_flux", 2000, 1000, 128, 0, 0, "column"): 930.6e6,
-                    ("k_update", 2000, 1000, 128, 0, 0, "column"): 664.3e6,
-                    ("k_grad", 2000, 1000, 256, 1, 0, "column"): 993.9e6,
-                    ("k_flux", 2000, 1000, 256, 1, 0, "column"): 775.6e6,
-                    ("k_update", 2000, 1000, 256, 1, 0, "column"): 626.5e6,
-                    ("k_grad", 2000, 1000, 256, 0, 1, "morton"): 1190.8e6,
-                    ("k_update", 2000, 1000, 256, 0, 1, "morton"): 1555.0e6,
-                    ("k_grad", 2000, 1000, 128, 0, 1, "morton"): 1264.0e6,
-                    ("k_update", 2000, 1000, 128, 0, 1, "morton"): 1554.9e6,
-                    ("k_grad", 2000, 1000, 64, 1, 1, "morton"): 999.7e6,
-                    ("k_update", 2000, 1000, 64, 1, 1, "morton"): 1165.1e6,
-                    ("k_grad", 2000, 1000, 128, 1, 1, "morton"): 999.7e6,
-                    ("k_update", 2000, 1000, 128, 1, 1, "morton"): 1164.9e6,
-                    ("k_grad", 2000, 1000, 256, 1, 1, "morton"): 999.7e6,
-                    ("k_update", 2000, 1000, 256, 1, 1, "morton"): 1165.1e6}
+MEASURED_TRAFFIC = {("k_stage", 2000, 1000, 256, 1, 1, "morton"): 1.5601e9}
 
 
 _MESHES = {}
@@ -746,7 +728,7 @@ def main():
                          "graph-replayed iterations; prints its JSON (the form kernel traces of it profile)")
     ap.add_argument("--shape", default=None, metavar="B,L,X[,T]",
                     help="launch shapes of the ramp runs instead of the autotuner's (e.g. 128,64,0,0: the choice a "
-                         "timed run reported; T 1: the tile form of the face flux + update), so that profiling "
+                         "timed run reported; T 1: the tile form, one kernel per stage), so that profiling "
                          "runs launch the kernels the timed run did")
     ap.add_argument("--order", choices=["morton", "column"], default="morton",
                     help="cell order of the ramp meshes: renumbered along a Morton curve (default) or the "
@@ -841,13 +823,16 @@ def main():
     kt = big["kernels"]
     dom = max((k for k in kt if alg_bytes(k, 1, 1, 1, 4) > 0), key=lambda k: kt[k][0] * kt[k][1])
     avg_ms = kt[dom][0]
-    # the default workload runs the primitives-from-state stages unless the
-    # stored form is selected through the library's environment switch
+    # the default workload's stages pass primitives only unless the stored
+    # form is selected through the library's environment switch
     pu = os.environ.get("CSU_STORED_PRIMITIVES", "0") != "1"
     from csu_amd import native as _nat
     stream = _nat.stream_rate(2 ** 30, 10)
     traffic_alg = alg_bytes(dom, big["nc"], big["nf"], big["nb"], big["nv"], pu, big.get("tile_entries", 0))
     achieved = traffic_alg / (avg_ms * 1e-3) / 1e9
+    # a five-stage iteration: every stage kernel's compulsory bytes
+    iter_alg = 5 * sum(alg_bytes(k, nc, big["nf"], big["nb"], big["nv"], pu, big.get("tile_entries", 0))
+                       for k in kt if k != "k_prim") / nc
     roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
             "traffic": MEASURED_TRAFFIC.get((dom, a.nx, a.ny, big["launch_shape"]["block"],
@@ -862,8 +847,8 @@ def main():
             "launch_shape": big["launch_shape"],
             "stream_kernel_gbs": stream,
             "kernel_frac_of_stream": achieved / stream,
-            "iteration_alg_bytes_per_cell": 2334.5,
-            "iteration_frac": value * 2334.5 / (HBM_PEAK_GBS * 1e9)}
+            "iteration_alg_bytes_per_cell": iter_alg,
+            "iteration_frac": value * iter_alg / (HBM_PEAK_GBS * 1e9)}
     others = None if a.no_configs else other_configs(log)
     if others is not None and not a.no_converge:
         others["time_to_converge"] = converge_configs(log)
