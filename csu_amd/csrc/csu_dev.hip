@@ -374,7 +374,7 @@ struct HostMesh {
   std::vector<int> cnp, cnbr, cface;                              // [nc], [4][nc], [4][nc]
   std::vector<int> cfn;  // [4][nc] the other cell of face slot j, -1 where cface is 0
   std::vector<double> xc, yc, om, dsxm, dsym, dslat;              // [nc]
-  std::vector<double> edx, edy, lwx, lwy;                         // [4][nc]
+  std::vector<double> wg;                                         // [4][nc]x{LSQ weight x, y, edge offset x, y}
   std::vector<unsigned char> fsl, bmask;                          // [nf], [nc]
   std::vector<int> fe0, fe1;                                      // [nf]
   std::vector<double> fdsx, fdsy, fds;                            // [nf]
@@ -396,7 +396,7 @@ static int host_mesh(const csu_mesh_desc* m, const csu_params* p, HostMesh& h) {
   h.cnp.assign(nc, 0); h.cnbr.assign(c4, 0); h.cface.assign(c4, 0);
   h.xc.assign(nc, 0.0); h.yc.assign(nc, 0.0); h.om.assign(nc, 0.0);
   h.dsxm.assign(nc, 0.0); h.dsym.assign(nc, 0.0); h.dslat.assign(nc, 0.0);
-  h.edx.assign(c4, 0.0); h.edy.assign(c4, 0.0); h.lwx.assign(c4, 0.0); h.lwy.assign(c4, 0.0);
+  h.wg.assign(4 * c4, 0.0);
   h.volmax = 0.0;
   for (int i = 0; i < nc; i++) {
     const int32_t* v = m->cell_vert + 4 * i;
@@ -418,8 +418,8 @@ static int host_mesh(const csu_mesh_desc* m, const csu_params* p, HostMesh& h) {
       sy += fabs(dSy);
       double xm = (m->node_xy[2 * p0] + m->node_xy[2 * p1]) * 0.5;
       double ym = (m->node_xy[2 * p0 + 1] + m->node_xy[2 * p1 + 1]) * 0.5;
-      h.edx[(size_t)j * nc + i] = xm - h.xc[i];
-      h.edy[(size_t)j * nc + i] = ym - h.yc[i];
+      h.wg[4 * ((size_t)j * nc + i) + 2] = xm - h.xc[i];
+      h.wg[4 * ((size_t)j * nc + i) + 3] = ym - h.yc[i];
     }
     h.dsxm[i] = sx * 0.5;
     h.dsym[i] = sy * 0.5;
@@ -463,8 +463,8 @@ static int host_mesh(const csu_mesh_desc* m, const csu_params* p, HostMesh& h) {
           const int32_t* q = m->bface + 3 * (-1 - n);
           calc_ds(m, q[1], q[2], &sx, &sy);
         }
-        h.lwx[(size_t)j * nc + i] = 0.5 * sx / h.om[i];
-        h.lwy[(size_t)j * nc + i] = 0.5 * sy / h.om[i];
+        h.wg[4 * ((size_t)j * nc + i)] = 0.5 * sx / h.om[i];
+        h.wg[4 * ((size_t)j * nc + i) + 1] = 0.5 * sy / h.om[i];
       }
   }
   // Least-squares weights per neighbour slot (solverCalcGrad3, solver.c:1031-1074):
@@ -490,8 +490,8 @@ static int host_mesh(const csu_mesh_desc* m, const csu_params* p, HostMesh& h) {
     }
     const long double det = a * c - b * b;
     for (int j = 0; j < h.cnp[i]; j++) {
-      h.lwx[(size_t)j * nc + i] = (double)((c * dx[j] - b * dy[j]) / det);
-      h.lwy[(size_t)j * nc + i] = (double)((a * dy[j] - b * dx[j]) / det);
+      h.wg[4 * ((size_t)j * nc + i)] = (double)((c * dx[j] - b * dy[j]) / det);
+      h.wg[4 * ((size_t)j * nc + i) + 1] = (double)((a * dy[j] - b * dx[j]) / det);
     }
   }
   // edge index of a face in a cell's vertex loop (the limiter and the
@@ -612,7 +612,7 @@ static void host_concat(const std::vector<HostMesh>& part, HostMesh& H, std::vec
   H.cnp.assign(NC, 0); H.cnbr.assign(C4, INT32_MAX); H.cface.assign(C4, 0); H.cfn.assign(C4, -1);
   H.xc.assign(NC, 0.0); H.yc.assign(NC, 0.0); H.om.assign(NC, 1.0);
   H.dsxm.assign(NC, 1.0); H.dsym.assign(NC, 1.0); H.dslat.assign(NC, 0.0);
-  H.edx.assign(C4, 0.0); H.edy.assign(C4, 0.0); H.lwx.assign(C4, 0.0); H.lwy.assign(C4, 0.0);
+  H.wg.assign(4 * C4, 0.0);
   H.fsl.assign(NF ? NF : 1, 0); H.bmask.assign(NC, 0);
   H.fe0.assign(NF, 0); H.fe1.assign(NF, 0);
   H.fdsx.assign(NF, 0.0); H.fdsy.assign(NF, 0.0); H.fds.assign(NF, 1.0);
@@ -637,7 +637,7 @@ static void host_concat(const std::vector<HostMesh>& part, HostMesh& H, std::vec
         H.cnbr[gj] = nbr == INT32_MAX ? nbr : nbr >= 0 ? nbr + c0 : -1 - ((-1 - nbr) + b0);
         H.cface[gj] = f > 0 ? f + f0 : f < 0 ? f - f0 : 0;
         H.cfn[gj] = h.cfn[lj] >= 0 ? h.cfn[lj] + c0 : -1;
-        H.edx[gj] = h.edx[lj]; H.edy[gj] = h.edy[lj]; H.lwx[gj] = h.lwx[lj]; H.lwy[gj] = h.lwy[lj];
+        std::copy_n(&h.wg[4 * lj], 4, &H.wg[4 * gj]);
       }
       if (lev) { H.levL[gi] = h.levL[i]; H.levU[gi] = h.levU[i]; }
     }
@@ -901,16 +901,12 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   Geo& g = d->geo;
   St& s = d->st;
   const size_t nvc = (size_t)nv * nc;
-  std::vector<double> wg(16 * (size_t)nc);  // weights and edge offsets, cell by cell
-  for (size_t t = 0; t < 4 * (size_t)nc; t++) {
-    wg[4 * t] = H.lwx[t]; wg[4 * t + 1] = H.lwy[t]; wg[4 * t + 2] = H.edx[t]; wg[4 * t + 3] = H.edy[t];
-  }
   const double* pref_d = nullptr;
   const int* wall_d = nullptr;
   if ((rc = upload(d, &g.cnp, H.cnp)) || (rc = upload(d, &g.cnbr, H.cnbr)) || (rc = upload(d, &g.cface, H.cface)) ||
       (rc = upload(d, &g.xc, H.xc)) || (rc = upload(d, &g.yc, H.yc)) || (rc = upload(d, &g.omega, H.om)) ||
       (rc = upload(d, &g.dsxm, H.dsxm)) || (rc = upload(d, &g.dsym, H.dsym)) || (rc = upload(d, &g.dslat, H.dslat)) ||
-      (rc = upload(d, &g.wg, wg)) || (rc = upload(d, &g.fsl, H.fsl)) ||
+      (rc = upload(d, &g.wg, H.wg)) || (rc = upload(d, &g.fsl, H.fsl)) ||
       (rc = upload(d, &g.bmask, H.bmask)) ||
       (rc = upload(d, &g.fe0, H.fe0)) || (rc = upload(d, &g.fe1, H.fe1)) || (rc = upload(d, &g.fdsx, H.fdsx)) ||
       (rc = upload(d, &g.fdsy, H.fdsy)) || (rc = upload(d, &g.fds, H.fds)) ||
@@ -992,7 +988,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   else if (!d->tuned && (double)d->tl.nh <= 1.25 * nc) d->tile = 1;
   if (kp.mixed) {
     auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
-    if ((rc = upload(d, &g.wg32, f32(wg))) ||
+    if ((rc = upload(d, &g.wg32, f32(H.wg))) ||
         (rc = upload(d, &g.fdsx32, f32(H.fdsx))) || (rc = upload(d, &g.fdsy32, f32(H.fdsy))) ||
         (rc = upload(d, &g.fds32, f32(H.fds))) || (rc = dalloc(d, &s.fflux32, (size_t)nv * nf)) ||
         (p->order == 2 && (rc = dalloc(d, &s.rec32, 4 * nvc))))

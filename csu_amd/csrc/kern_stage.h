@@ -2,7 +2,7 @@
 // (reference solverCalcR + solverRK, solver.c:685-766) as one kernel.
 //
 // A workgroup owns a tile of CSU_CHUNK consecutive cells and keeps what the
-// three split kernels (k_grad, k_flux, k_update, and k_bcflux before them)
+// three split kernels (k_grad, k_flux, k_update)
 // pass to each other through memory in LDS:
 //   0  boundary faces of the tile's cells and of its halo (the cells across
 //      its outer faces): ghost states, and the tile's own boundary fluxes
@@ -15,13 +15,16 @@
 // the same bit for bit.  A halo cell's gradient and a face between two tiles
 // are evaluated by every tile that needs them.
 //
-// What bounds it: FP64 issue and the latency of its phases, not bytes.  It
-// moves about 280 B per cell where the split kernels moved 540 (edge states
-// and face fluxes written and read back), at the price of the halo's
-// gradients (a third more of phase 1 in Morton order).  RK5 iterations,
-// split kernels with separate face fluxes in the update -> this kernel:
-// 2.0M cells, Morton order 1,247 -> 942 us; 406k cells 333 -> 222 us (mixed
-// precision 250 -> 193 us); 40k cells 114 -> 71 us (launches: 22 -> 7).
+// What bounds it: memory traffic and FP64 issue about alike.  4.0M cells in
+// Morton order: 315 us a stage, 1,560 MB counted (277 B per cell that it
+// cannot do without; the split kernels' stage 540: edge states and face
+// fluxes written and read back), 4.95 TB/s or 0.74 of the streaming rate,
+// with FP64 instructions issuing in 62 % of its cycles; the halo's gradients
+// are a third of phase 1.  Contiguous copies of the halo cells' geometry
+// changed nothing.  Below about 100k cells: the latency of its four phases.
+// RK5 iterations, split kernels with the face fluxes in the update -> this
+// kernel: 2.0M cells 1,247 -> 890 us (4.0M 2,380 -> 1,607 us); 406k cells in
+// mixed precision 250 -> 190 us; 40k cells 114 -> 71 us (launches: 22 -> 7).
 #pragma once
 #include "kernels.h"
 
