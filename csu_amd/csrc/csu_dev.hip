@@ -87,6 +87,7 @@ struct csu_dev {
   Tile tl;                     // the tile form's lists
   int quads;                   // 1: the mesh has cells of four edges
   int tile_nt;                 // threads per tile
+  int tile1;                   // 1: a first-order RK run in the tile form (no launch-shape choice)
   int tl_capb;                 // boundary entries its LDS array holds
   size_t tl_n;                 // interior entries in all
   dbl2 *Pa, *Pb4;              // tile form: primitives r u v p [nc][4], current and the one a stage writes
@@ -861,6 +862,12 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   const char* sp = getenv("CSU_STORED_PRIMITIVES");
   d->pu = nv == 4 && !p->laminar && p->time_scheme == CSU_TIME_RK && p->order == 2 && p->limiter != 1 &&
           kp.axi == 0 && p->tp == 0 && !(sp && sp[0] == '1');
+  // First-order runs of the same kind take the tile form too, without a
+  // launch-shape choice, under the untuned default's bound on the halos:
+  // shock tube, 32,800 cells, 16.2 -> 11.1 us per stage (three kernels of
+  // about 5 us -> one).
+  const bool first = nv == 4 && !p->laminar && p->time_scheme == CSU_TIME_RK && p->order == 1 && kp.axi == 0 &&
+                     p->tp == 0 && !(sp && sp[0] == '1');
   kp.rlim = p->rlim; kp.pout = p->pout; kp.twall = p->twall; kp.efix = p->efix; kp.minf = p->mach_inf;
   kp.sst_owall = p->sst_owallfactor;
   {
@@ -945,7 +952,8 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     d->sol_host = *sol;
   }
   if (p->order == 2 && !kp.mixed && (rc = dalloc(d, &s.rec, 4 * nvc))) return rc;
-  if (d->pu) {
+  d->tile1 = 0;
+  if (d->pu || first) {
     d->quads = 0;
     for (int n : H.cnp) d->quads |= n == 4;
     HostTile T;
@@ -976,7 +984,8 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
             (rc = upload(d, &tl.fs32, f32(T.fs))))
           return rc;
       }
-      d->tile_ok = 1;
+      d->tile_ok = d->pu;
+      d->tile1 = first && (double)d->tl.nh <= 1.25 * nc;
     }
   }
   if (!d->tile_ok) d->tile = 0;
@@ -1088,7 +1097,7 @@ static csu_dev* dev_new() {
   memset((void*)&d->geo, 0, sizeof(Geo));
   memset((void*)&d->st, 0, sizeof(St));
   memset((void*)&d->tl, 0, sizeof(Tile));
-  d->Pa = d->Pb4 = nullptr; d->quads = 1; d->tl_capb = 0; d->tl_n = 0;
+  d->Pa = d->Pb4 = nullptr; d->quads = 1; d->tl_capb = 0; d->tl_n = 0; d->tile1 = 0;
   return d;
 }
 
@@ -1361,7 +1370,10 @@ static int tile_stage(csu_dev* d, int flags, double sigma, double rk_a) {
                        d->dtg, d->U, d->Uaux, (const dbl2*)d->Pa, d->Pb4, d->red, rdt);
   };
   const bool roe = kp.flux == 0;
-  if (kp.lsq_ld) go(k_stage<NT, 4, -1, false, true>);
+  if (d->tile1) {
+    if (kp.mixed) roe ? go(k_stage<NT, 4, 0, true, false, true>) : go(k_stage<NT, 4, -1, true, false, true>);
+    else roe ? go(k_stage<NT, 4, 0, false, false, true>) : go(k_stage<NT, 4, -1, false, false, true>);
+  } else if (kp.lsq_ld) go(k_stage<NT, 4, -1, false, true>);
   else if (kp.mixed && !d->quads) roe ? go(k_stage<NT, 3, 0, true, false>) : go(k_stage<NT, 3, -1, true, false>);
   else if (kp.mixed) roe ? go(k_stage<NT, 4, 0, true, false>) : go(k_stage<NT, 4, -1, true, false>);
   else if (!d->quads) roe ? go(k_stage<NT, 3, 0, false, false>) : go(k_stage<NT, 3, -1, false, false>);
@@ -1531,6 +1543,7 @@ static int rk_iteration(csu_dev* d, int it_index) {
   double* red_dt = d->red + (size_t)NV * d->nred;
   const int cur_local = is_local(d, it_index), next_local = is_local(d, it_index + 1);
   int first_flags = F_CLAMP_UN;
+  const bool tile = NV == 4 && !VISC && (d->tile || d->tile1);
   if (d->fresh) {
     // time step from the unclamped state (solverCalcDt), then primitives
     Prof p(d, "k_dt");
@@ -1541,7 +1554,7 @@ static int rk_iteration(csu_dev* d, int it_index) {
                          d->dtg, d->geo.sol);
     int rc = prim_pass<NV>(d);
     if (rc) return rc;
-    if (d->tile)
+    if (tile)
       hipLaunchKernelGGL(k_pack4, dim3(nblk(nc)), dim3(CSU_BLOCK), 0, d->stream, nc, (const double*)d->st.P, d->Pa);
     first_flags = 0;
     d->fresh = 0;
@@ -1550,9 +1563,9 @@ static int rk_iteration(csu_dev* d, int it_index) {
     hipLaunchKernelGGL(k_time_clamp, dim3(1), dim3(64), 0, d->stream, d->tstate, d->dtg, d->prm.stages);
   for (int s = 0; s < d->prm.stages; s++) {
     const bool last = s == d->prm.stages - 1;
-    int flags = F_RK | (cur_local ? F_CUR_LOCAL : 0) | (s == 0 || d->tile ? first_flags : 0);
+    int flags = F_RK | (cur_local ? F_CUR_LOCAL : 0) | (s == 0 || tile ? first_flags : 0);
     if (last) flags |= F_LAST | (next_local ? F_NEXT_LOCAL : 0);
-    if (d->tile) {
+    if (tile) {
       int rc = d->tile_nt == 512 ? tile_stage<512>(d, flags, sigma, a[s]) : tile_stage<256>(d, flags, sigma, a[s]);
       if (rc) return rc;
       continue;
@@ -2052,7 +2065,7 @@ extern "C" int csu_dev_set_precision(csu_dev* d, int32_t prec) {
       return rc;
     if (!s.fflux32 && (rc = dalloc(d, &s.fflux32, (size_t)d->nv * nf))) return rc;
     if (d->prm.order == 2 && !s.rec32 && (rc = dalloc(d, &s.rec32, 4 * nvc))) return rc;
-    if (d->tile_ok && !d->tl.fx32 && ((rc = f32(d->tl.fx, &d->tl.fx32, d->tl_n)) ||
+    if ((d->tile_ok || d->tile1) && !d->tl.fx32 && ((rc = f32(d->tl.fx, &d->tl.fx32, d->tl_n)) ||
                                       (rc = f32(d->tl.fy, &d->tl.fy32, d->tl_n)) ||
                                       (rc = f32(d->tl.fs, &d->tl.fs32, d->tl_n))))
       return rc;
@@ -2335,7 +2348,7 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
   if (p->time_scheme == CSU_TIME_LUSGS) b += nc * 24 + nf * 24;
   if (p->time_scheme == CSU_TIME_DPLUR) b += 8.0 * block_total((int)nv, m->ncell) + 8.0 * (p->nlinear > 0 ? p->nlinear : 1) * (nc / 256 + 1);
   if (p->precision == 1) b += nc * 64 + nf * (12 + 4 * nv) + (p->order == 2 ? 16 * nv * nc : 0);  // FP32 copies
-  if (p->time_scheme == CSU_TIME_RK && !visc && p->order == 2 && p->limiter != 1 && m->axi == 0 && p->tp == 0) {
+  if (p->time_scheme == CSU_TIME_RK && !visc && (p->order == 1 || p->limiter != 1) && m->axi == 0 && p->tp == 0) {
     // tile form: its two primitive buffers, places, face copies, halo cells (at
     // most one per tile and face between two tiles)
     double cross = 0;

@@ -203,6 +203,25 @@ __device__ __forceinline__ void stage_cell(const KP& kp, const Geo& g, const St&
   }
 }
 
+// Phase 1 of a first-order run's cell: its own primitives are its edge states
+// (launch and phase latency bound it: 11 us a stage at 32,800 cells).
+template <int NE, typename TF>
+__device__ __forceinline__ void stage_cell1(const dbl2* __restrict__ Pin, int i, const short* el, int lst, int cap,
+                                            TF* sf) {
+  double Pi[4];
+  load4(Pin, i, Pi);
+  int pl[NE];
+#pragma unroll
+  for (int j = 0; j < NE; j++) pl[j] = el[j * lst];
+#pragma unroll
+  for (int j = 0; j < NE; j++) {
+    const int p = pl[j];
+    if (p == 0) continue;
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) sf[(p > 0 ? kk * cap + p - 1 : (4 + kk) * cap - p - 1)] = (TF)Pi[kk];
+  }
+}
+
 // Phase 0 of one boundary face: its ghost state (boundaryCalcPrimitive) and,
 // for one of the tile's own cells, its convective flux (bc_flux,
 // kern_common.h, with the two states at hand).
@@ -243,8 +262,8 @@ __device__ __forceinline__ void stage_bface(const KP& kp, const Geo& g, const St
 // they are a function of U^n alone, so every stage can repeat them).
 // FLX: the flux function, -1: kp.flux (one function inlined instead of five
 // keeps the code in the instruction cache: 64 KB with all of them); NE: the
-// most edges of a cell.
-template <int NT, int NE, int FLX, bool MIX, bool LD>
+// most edges of a cell; O1: a first-order run (no gradients).
+template <int NT, int NE, int FLX, bool MIX, bool LD, bool O1 = false>
 __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, int flags, double sigma, double rk_a,
                                               double cfl, double* dtl, const double* dtg,
                                               const double* __restrict__ Un, double* __restrict__ Uout,
@@ -284,8 +303,11 @@ __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, in
     const bool own = k < CSU_CHUNK;
     if (own && k >= nown) continue;
     const int h = h0 + k - CSU_CHUNK, i = own ? c0 + k : tl.hcell[h];
-    stage_cell<NE, MIX, LD, TF>(kp, g, s, tl, Pin, sv, s.pref2 + 6 * sid, i, own ? tl.csl + i : tl.hsl + h, own ? tl.cel + i : tl.hel + h,
-                            own ? nc : tl.nh, sf, sb);
+    if constexpr (O1)
+      stage_cell1<NE, TF>(Pin, i, own ? tl.cel + i : tl.hel + h, own ? nc : tl.nh, tl.capf, sf);
+    else
+      stage_cell<NE, MIX, LD, TF>(kp, g, s, tl, Pin, sv, s.pref2 + 6 * sid, i, own ? tl.csl + i : tl.hsl + h,
+                                  own ? tl.cel + i : tl.hel + h, own ? nc : tl.nh, sf, sb);
   }
   __syncthreads();
   for (int k = t; k < nft; k += NT) {

@@ -82,3 +82,38 @@ def test_stage_tile_clamps_and_holds(tmpcase):
     assert np.array_equal(out[1][2], U0)
     for x, y in zip(*out):
         assert np.array_equal(x, y, equal_nan=True)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("form", ["one_short_tile", "remainder", "quads_ausm_1", "wide_tiles", "tube"])
+def test_first_order_tile_equals_split(tmpcase, monkeypatch, form, precision):
+    """First-order runs (edge states = cell states) in one kernel per stage:
+    the split kernels' results bit for bit, a time-accurate run past its
+    last step included."""
+    d = tmpcase("o1")
+    if form == "tube":
+        m = cases.tube_mesh(nx=90, ny=7, seed=0)
+        cases.write_case(d, m, cases.tube_input(threads=1, tmax=0.004, precision=precision))
+    else:
+        nx, ny, split, inp = FORMS[form]
+        m = cases.ramp_mesh(nx=nx, ny=ny, seed=3, split=split)
+        cases.write_case(d, m, cases.ramp_input(threads=1, nmax=1, order=1, precision=precision, **inp))
+    c = native.HostCase(d)
+    U0 = c.initial_state() * (1 + 0.02 * np.random.default_rng(5).standard_normal((c.nvar, c.ncell)))
+    got = []
+    for stored in ("1", "0"):
+        monkeypatch.setenv("CSU_STORED_PRIMITIVES", stored)
+        dev = native.Device(c)
+        dev.set_state(U0)
+        if form == "tube":
+            dev.advance_time(c.tmax)
+        parts = [dev.iterate(n) for n in (1, 5, 4)]
+        dev.set_profiling(True)
+        dev.iterate(1)
+        assert ("k_stage" in dev.kernel_times()) == (stored == "0")
+        got.append((np.concatenate([p[0] for p in parts]), np.concatenate([p[1] for p in parts]), dev.get_state(),
+                    dev.residual()["R"]))
+        dev.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b, equal_nan=True)  # the tube's forces: 0/0, its free stream is at rest
+    assert np.isfinite(got[1][2]).all()
