@@ -712,6 +712,7 @@ static void tune_lookup(csu_dev* d) {
 struct HostTile {
   std::vector<int> toff, boff, bown, hoff, tbq, tbc, hcell;
   std::vector<double> fx, fy, fs;
+  std::vector<int> fa, fb;
   std::vector<short> csl, hsl, cel, hel;
   int capf = 0, capb = 0;
 };
@@ -745,6 +746,8 @@ static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, HostTi
     if (b != a) ent[fill[b]++] = f;
   });
   T.fx.resize(ne ? ne : 1); T.fy.resize(ne ? ne : 1); T.fs.resize(ne ? ne : 1);
+  T.fa.resize(ne ? ne : 1); T.fb.resize(ne ? ne : 1);
+  for (size_t e = 0; e < ne; e++) { T.fa[e] = H.fe0[ent[e]]; T.fb[e] = H.fe1[ent[e]]; }
   for (size_t e = 0; e < ne; e++) { T.fx[e] = H.fdsx[ent[e]]; T.fy[e] = H.fdsy[ent[e]]; T.fs[e] = H.fds[ent[e]]; }
   // halo cells of each tile, ascending
   T.hoff.assign(nt + 1, 0);
@@ -864,7 +867,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
           kp.axi == 0 && p->tp == 0 && !(sp && sp[0] == '1');
   // First-order runs of the same kind take the tile form too, without a
   // launch-shape choice, under the untuned default's bound on the halos:
-  // shock tube, 32,800 cells, 16.2 -> 11.1 us per stage (three kernels of
+  // shock tube, 32,800 cells, 16.2 -> 9.8 us per stage (three kernels of
   // about 5 us -> one).
   const bool first = nv == 4 && !p->laminar && p->time_scheme == CSU_TIME_RK && p->order == 1 && kp.axi == 0 &&
                      p->tp == 0 && !(sp && sp[0] == '1');
@@ -984,6 +987,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
             (rc = upload(d, &tl.fs32, f32(T.fs))))
           return rc;
       }
+      if (first && ((rc = upload(d, &tl.fa, T.fa)) || (rc = upload(d, &tl.fb, T.fb)))) return rc;
       d->tile_ok = d->pu;
       d->tile1 = first && (double)d->tl.nh <= 1.25 * nc;
     }
@@ -2353,7 +2357,7 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
     // most one per tile and face between two tiles)
     double cross = 0;
     for (int f = 0; f < m->nface; f++) cross += m->face[4 * (size_t)f] / CSU_CHUNK != m->face[4 * (size_t)f + 1] / CSU_CHUNK;
-    b += nc * (64 + 16) + (nf + cross) * (p->precision == 1 ? 36 : 24) + 2 * cross * 20 + 12 * nb + 16 * (nc / 256 + 2);
+    b += nc * (64 + 16) + (nf + cross) * ((p->precision == 1 ? 36 : 24) + (p->order == 1 ? 8 : 0)) + 2 * cross * 20 + 12 * nb + 16 * (nc / 256 + 2);
   }
   b += (nv + 4) * 8 * (double)(hist > 0 ? hist : 1);
   // allocation granularity: every array rounds up (at most 2 MiB slack per large array)

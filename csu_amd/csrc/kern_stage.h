@@ -43,6 +43,7 @@ struct Tile {
   const short *csl, *hsl;           // [4][nc], [4][nh]: slot j's entry, +(1 + place) where the cell is the face's
                                     // e0, -(1 + place) where e1; boundary slots 1 + place in the boundary list
   const short *cel, *hel;           // [4][nc], [4][nh]: edge j's entry, + left half, - right half, 0 none
+  const int *fa, *fb;               // first-order runs: entry's cells
   int nh;                           // stride of hsl, hel
   int capf;                         // interior entries the LDS array holds
 };
@@ -203,25 +204,6 @@ __device__ __forceinline__ void stage_cell(const KP& kp, const Geo& g, const St&
   }
 }
 
-// Phase 1 of a first-order run's cell: its own primitives are its edge states
-// (launch and phase latency bound it: 11 us a stage at 32,800 cells).
-template <int NE, typename TF>
-__device__ __forceinline__ void stage_cell1(const dbl2* __restrict__ Pin, int i, const short* el, int lst, int cap,
-                                            TF* sf) {
-  double Pi[4];
-  load4(Pin, i, Pi);
-  int pl[NE];
-#pragma unroll
-  for (int j = 0; j < NE; j++) pl[j] = el[j * lst];
-#pragma unroll
-  for (int j = 0; j < NE; j++) {
-    const int p = pl[j];
-    if (p == 0) continue;
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) sf[(p > 0 ? kk * cap + p - 1 : (4 + kk) * cap - p - 1)] = (TF)Pi[kk];
-  }
-}
-
 // Phase 0 of one boundary face: its ghost state (boundaryCalcPrimitive) and,
 // for one of the tile's own cells, its convective flux (bc_flux,
 // kern_common.h, with the two states at hand).
@@ -262,7 +244,9 @@ __device__ __forceinline__ void stage_bface(const KP& kp, const Geo& g, const St
 // they are a function of U^n alone, so every stage can repeat them).
 // FLX: the flux function, -1: kp.flux (one function inlined instead of five
 // keeps the code in the instruction cache: 64 KB with all of them); NE: the
-// most edges of a cell; O1: a first-order run (no gradients).
+// most edges of a cell; O1: a first-order run, whose faces take the states of
+// their cells from memory (phase 2 alone beside the boundary faces: launch and
+// one gather chain bound it).
 template <int NT, int NE, int FLX, bool MIX, bool LD, bool O1 = false>
 __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, int flags, double sigma, double rk_a,
                                               double cfl, double* dtl, const double* dtg,
@@ -297,19 +281,16 @@ __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, in
     for (int k = 0; k < 7; k++) kb.pin[k] = sv ? sv->pin[k] : kp.pin[k];
     for (int k = t; k < nbt; k += NT)
       stage_bface<FLX>(kb, g, s, Pin, tl.tbq[b0 + k], tl.tbc[b0 + k], k < tl.bown[tile], lastst, sb + 8 * k);
-    __syncthreads();
+    if (!O1) __syncthreads();
   }
-  for (int k = t; k < CSU_CHUNK + nh; k += NT) {
+  for (int k = t; !O1 && k < CSU_CHUNK + nh; k += NT) {
     const bool own = k < CSU_CHUNK;
     if (own && k >= nown) continue;
     const int h = h0 + k - CSU_CHUNK, i = own ? c0 + k : tl.hcell[h];
-    if constexpr (O1)
-      stage_cell1<NE, TF>(Pin, i, own ? tl.cel + i : tl.hel + h, own ? nc : tl.nh, tl.capf, sf);
-    else
-      stage_cell<NE, MIX, LD, TF>(kp, g, s, tl, Pin, sv, s.pref2 + 6 * sid, i, own ? tl.csl + i : tl.hsl + h,
-                                  own ? tl.cel + i : tl.hel + h, own ? nc : tl.nh, sf, sb);
+    stage_cell<NE, MIX, LD, TF>(kp, g, s, tl, Pin, sv, s.pref2 + 6 * sid, i, own ? tl.csl + i : tl.hsl + h,
+                                own ? tl.cel + i : tl.hel + h, own ? nc : tl.nh, sf, sb);
   }
-  __syncthreads();
+  if (!O1) __syncthreads();
   for (int k = t; k < nft; k += NT) {
     TF dSx, dSy, dS;
     if (MIX) {
@@ -318,10 +299,18 @@ __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, in
       dSx = tl.fx[f0 + k]; dSy = tl.fy[f0 + k]; dS = tl.fs[f0 + k];
     }
     TF PL[4], PR[4], fl[4];
+    if (O1) {
+      double a[4], b[4];
+      load4(Pin, tl.fa[f0 + k], a);
+      load4(Pin, tl.fb[f0 + k], b);
 #pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-      PL[kk] = sf[kk * tl.capf + k];
-      PR[kk] = sf[(4 + kk) * tl.capf + k];
+      for (int kk = 0; kk < 4; kk++) { PL[kk] = (TF)a[kk]; PR[kk] = (TF)b[kk]; }
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++) {
+        PL[kk] = sf[kk * tl.capf + k];
+        PR[kk] = sf[(4 + kk) * tl.capf + k];
+      }
     }
     const Den<TF> dl(dS);
     rotate<TF>(PL[1], PL[2], dSx, dSy, dl);
