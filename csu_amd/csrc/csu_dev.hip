@@ -707,8 +707,9 @@ static void tune_lookup(csu_dev* d) {
 }
 
 // Lists of the tile form (k_stage, struct Tile) over the 256-cell tiles of a
-// mesh or of a batch's solves.  False when a tile has more interior faces
-// than CSU_TILE_FACES or its LDS arrays do not fit.
+// mesh or of a batch's solves (first: a first-order run, which reads its
+// faces' cells).  False when a tile has more interior faces than
+// CSU_TILE_FACES or its LDS arrays do not fit.
 struct HostTile {
   std::vector<int> toff, boff, bown, hoff, tbq, tbc, hcell;
   std::vector<double> fx, fy, fs;
@@ -717,7 +718,7 @@ struct HostTile {
   int capf = 0, capb = 0;
 };
 
-static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, HostTile& T) {
+static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, bool first, HostTile& T) {
   const int nc = H.nc, B = CSU_CHUNK, nt = (nc + B - 1) / B;
   auto each_face = [&](auto fn) {
     if (sol && !sol->empty()) {
@@ -746,8 +747,8 @@ static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, HostTi
     if (b != a) ent[fill[b]++] = f;
   });
   T.fx.resize(ne ? ne : 1); T.fy.resize(ne ? ne : 1); T.fs.resize(ne ? ne : 1);
-  T.fa.resize(ne ? ne : 1); T.fb.resize(ne ? ne : 1);
-  for (size_t e = 0; e < ne; e++) { T.fa[e] = H.fe0[ent[e]]; T.fb[e] = H.fe1[ent[e]]; }
+  if (first) { T.fa.resize(ne ? ne : 1); T.fb.resize(ne ? ne : 1); }
+  for (size_t e = 0; first && e < ne; e++) { T.fa[e] = H.fe0[ent[e]]; T.fb[e] = H.fe1[ent[e]]; }
   for (size_t e = 0; e < ne; e++) { T.fx[e] = H.fdsx[ent[e]]; T.fy[e] = H.fdsy[ent[e]]; T.fs[e] = H.fds[ent[e]]; }
   // halo cells of each tile, ascending
   T.hoff.assign(nt + 1, 0);
@@ -960,7 +961,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     d->quads = 0;
     for (int n : H.cnp) d->quads |= n == 4;
     HostTile T;
-    if (tile_lists(H, sol, T)) {
+    if (tile_lists(H, sol, first, T)) {
       Tile& tl = d->tl;
       // Threads per tile: 512 let a tile's halo run beside its own cells and
       // both rounds of faces at once, which wins while the tiles leave the

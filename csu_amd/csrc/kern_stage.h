@@ -1,9 +1,10 @@
-// kern_stage.h -- one explicit stage of the inviscid second-order path
-// (reference solverCalcR + solverRK, solver.c:685-766) as one kernel.
+// kern_stage.h -- one explicit stage of the inviscid path (reference
+// solverCalcR + solverRK, solver.c:685-766) as one kernel: second order, and
+// first order without phase 1.
 //
 // A workgroup owns a tile of CSU_CHUNK consecutive cells and keeps what the
-// three split kernels (k_grad, k_flux, k_update)
-// pass to each other through memory in LDS:
+// three split kernels (k_grad, k_flux, k_update) pass to each other through
+// memory in LDS:
 //   0  boundary faces of the tile's cells and of its halo (the cells across
 //      its outer faces): ghost states, and the tile's own boundary fluxes
 //   1  the tile's cells and its halo: gradients, limiter, and the
