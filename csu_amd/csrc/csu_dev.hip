@@ -2355,9 +2355,11 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
   if (p->precision == 1) b += nc * 64 + nf * (12 + 4 * nv) + (p->order == 2 ? 16 * nv * nc : 0);  // FP32 copies
   if (p->time_scheme == CSU_TIME_RK && !visc && (p->order == 1 || p->limiter != 1) && m->axi == 0 && p->tp == 0) {
     // tile form: its two primitive buffers, places, face copies, halo cells (at
-    // most one per tile and face between two tiles)
-    double cross = 0;
-    for (int f = 0; f < m->nface; f++) cross += m->face[4 * (size_t)f] / CSU_CHUNK != m->face[4 * (size_t)f + 1] / CSU_CHUNK;
+    // most one per tile and face between two tiles; a mesh given by its counts
+    // alone: every face may be one)
+    double cross = m->face ? 0 : nf;
+    for (int f = 0; m->face && f < m->nface; f++)
+      cross += m->face[4 * (size_t)f] / CSU_CHUNK != m->face[4 * (size_t)f + 1] / CSU_CHUNK;
     b += nc * (64 + 16) + (nf + cross) * ((p->precision == 1 ? 36 : 24) + (p->order == 1 ? 8 : 0)) + 2 * cross * 20 + 12 * nb + 16 * (nc / 256 + 2);
   }
   b += (nv + 4) * 8 * (double)(hist > 0 ? hist : 1);
