@@ -338,7 +338,14 @@ static int wall_distance_launch(const csu_mesh_desc* m, hipStream_t st, const do
 extern "C" int csu_wall_distance_dev(const csu_mesh_desc* m, double* wd) {
   if (!m || !wd || m->ncell <= 0 || !m->node_xy || !m->cell_vert) return set_err(CSU_ERR_ARG, "bad mesh or output");
   if (m->nbface > 0 && (!m->bface || !m->bface_mark || !m->mark_type)) return set_err(CSU_ERR_ARG, "bad boundary");
-  const size_t nc = m->ncell, nn = m->nnode > 0 ? m->nnode : 1;
+  const size_t nc = m->ncell;
+  // a descriptor without a node count: the nodes that its cells name
+  csu_mesh_desc own = *m;
+  if (m->nnode <= 0) {
+    own.nnode = 1 + std::max(0, *std::max_element(m->cell_vert, m->cell_vert + 4 * nc));
+    m = &own;
+  }
+  const size_t nn = m->nnode;
   int nw = 0, ng = 0;
   const std::vector<double> seg = wall_segments(m, &nw, &ng);
   // one allocation, 16-byte parts first: nodes, cell vertices, distances,
@@ -351,7 +358,7 @@ extern "C" int csu_wall_distance_dev(const csu_mesh_desc* m, double* wd) {
   int rc = CSU_OK;
   hipStream_t st = nullptr;
   if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) rc = set_err(CSU_ERR_HIP, "stream");
-  if (!rc && (hipMemcpyAsync(buf, m->node_xy, 2 * (size_t)m->nnode * sizeof(double), hipMemcpyHostToDevice, st) !=
+  if (!rc && (hipMemcpyAsync(buf, m->node_xy, 2 * nn * sizeof(double), hipMemcpyHostToDevice, st) !=
                   hipSuccess ||
               hipMemcpyAsync(cv, m->cell_vert, 4 * nc * sizeof(int32_t), hipMemcpyHostToDevice, st) != hipSuccess))
     rc = set_err(CSU_ERR_HIP, "mesh upload failed");
