@@ -392,6 +392,7 @@ struct HostMesh {
   std::vector<int> wall;                                          // boundary ids of wall / wallT faces
   std::vector<int> levL, levU;  // LU-SGS: dependency level of each cell, forward / backward sweep (-1: padding)
   double volmax = 0.0;
+  bool linked = true;  // every face slot of a cell names a face of that cell, and is no boundary slot
 };
 
 // Geometry and connectivity of one mesh in the reference's expressions
@@ -534,10 +535,16 @@ static int host_mesh(const csu_mesh_desc* m, const csu_params* p, HostMesh& h) {
   // the implicit kernels' neighbour of each face slot, so that their
   // neighbour gathers do not wait for a face-array lookup
   h.cfn.assign(c4, -1);
-  for (size_t t = 0; t < c4; t++) {
-    const int f = h.cface[t];
-    if (f != 0) h.cfn[t] = f > 0 ? h.fe1[f - 1] : h.fe0[-f - 1];
-  }
+  h.linked = true;
+  for (int j = 0; j < 4; j++)
+    for (int i = 0; i < nc; i++) {
+      const size_t t = (size_t)j * nc + i;
+      const int f = h.cface[t];
+      if (f == 0) continue;
+      const int a = h.fe0[(f > 0 ? f : -f) - 1], b = h.fe1[(f > 0 ? f : -f) - 1];
+      h.cfn[t] = f > 0 ? b : a;
+      if ((f > 0 ? a : b) != i || ((h.bmask[i] >> j) & 1)) h.linked = false;
+    }
   // LU-SGS face terms that depend on the geometry only, in the sweep's own
   // expressions (implicit.c:288-313, 555-595): n = dS/|dS| (seen from e1 it
   // is the exact negation) and the distance of the two cell centres (the
@@ -634,6 +641,7 @@ static void host_concat(const std::vector<HostMesh>& part, HostMesh& H, std::vec
   H.volmax = part.empty() ? 0.0 : part[0].volmax;
   for (size_t s = 0; s < n; s++) {
     const HostMesh& h = part[s];
+    H.linked = H.linked && h.linked;
     const int c0 = sol[s].c0, f0 = sol[s].f0, b0 = sol[s].b0, nc = h.nc;
     for (int i = 0; i < nc; i++) {
       const size_t gi = (size_t)c0 + i;
@@ -713,19 +721,21 @@ static void tune_lookup(csu_dev* d) {
   d->tuned = 1;
 }
 
-// Lists of the tile form (k_stage, struct Tile) over the 256-cell tiles of a
-// mesh or of a batch's solves (first: a first-order run, which reads its
-// faces' cells).  False when a tile has more interior faces than
-// CSU_TILE_FACES or its LDS arrays do not fit.
+// What the host makes of the tile form's lists (k_stage, struct Tile) over the
+// 256-cell tiles of a mesh or of a batch's solves: each tile's interior faces
+// (ent, ascending), halo cells (ascending) and boundary faces.  The face
+// copies and the cells' places in these lists are k_tile_lists' work; made
+// here they took three quarters of the time.  btgt: the slot 4 cell + j of an
+// own cell's boundary face, -1 - (4 place in hcell + j) of a halo cell's.
+// False when a tile has more interior faces than CSU_TILE_FACES or its LDS
+// arrays do not fit.
 struct HostTile {
-  std::vector<int> toff, boff, bown, hoff, tbq, tbc, hcell;
-  std::vector<double> fx, fy, fs;
-  std::vector<int> fa, fb;
-  std::vector<short> csl, hsl, cel, hel;
+  std::vector<int> toff, ent, hoff, hcell, boff, bown, tbq, tbc, btgt;
   int capf = 0, capb = 0;
 };
 
-static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, bool first, HostTile& T) {
+static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, HostTile& T) {
+  if (!H.linked) return false;
   const int nc = H.nc, B = CSU_CHUNK, nt = (nc + B - 1) / B;
   auto each_face = [&](auto fn) {
     if (sol && !sol->empty()) {
@@ -746,89 +756,107 @@ static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, bool f
     T.capf = std::max(T.capf, T.toff[t + 1]);
     T.toff[t + 1] += T.toff[t];
   }
-  const size_t ne = T.toff[nt];
-  std::vector<int> ent(ne ? ne : 1), fill(T.toff.begin(), T.toff.end() - 1);
+  T.capf = (T.capf + 7) & ~7;
+  T.ent.resize(T.toff[nt]);
+  std::vector<int> fill(T.toff.begin(), T.toff.end() - 1);
   each_face([&](int f) {
     const int a = H.fe0[f] / B, b = H.fe1[f] / B;
-    ent[fill[a]++] = f;
-    if (b != a) ent[fill[b]++] = f;
+    T.ent[fill[a]++] = f;
+    if (b != a) T.ent[fill[b]++] = f;
   });
-  T.fx.resize(ne ? ne : 1); T.fy.resize(ne ? ne : 1); T.fs.resize(ne ? ne : 1);
-  if (first) { T.fa.resize(ne ? ne : 1); T.fb.resize(ne ? ne : 1); }
-  for (size_t e = 0; first && e < ne; e++) { T.fa[e] = H.fe0[ent[e]]; T.fb[e] = H.fe1[ent[e]]; }
-  for (size_t e = 0; e < ne; e++) { T.fx[e] = H.fdsx[ent[e]]; T.fy[e] = H.fdsy[ent[e]]; T.fs[e] = H.fds[ent[e]]; }
-  // halo cells of each tile, ascending
+  // a cell belongs to the halos of its neighbours' tiles; cell by cell, so
+  // that each tile's list ascends
   T.hoff.assign(nt + 1, 0);
-  std::vector<int> hc;
-  for (int t = 0; t < nt; t++) {
-    hc.clear();
-    for (int e = T.toff[t]; e < T.toff[t + 1]; e++) {
-      const int a = H.fe0[ent[e]], b = H.fe1[ent[e]];
-      if (a / B != t) hc.push_back(a);
-      if (b / B != t) hc.push_back(b);
-    }
-    std::sort(hc.begin(), hc.end());
-    hc.erase(std::unique(hc.begin(), hc.end()), hc.end());
-    T.hcell.insert(T.hcell.end(), hc.begin(), hc.end());
-    T.hoff[t + 1] = (int)T.hcell.size();
-  }
-  const size_t nh = T.hcell.size();
-  if (nh == 0) T.hcell.push_back(0);
-  const size_t NH = nh ? nh : 1;
-  T.csl.assign(4 * (size_t)nc, 0); T.cel.assign(4 * (size_t)nc, 0);
-  T.hsl.assign(4 * NH, 0); T.hel.assign(4 * NH, 0);
-  // edge places: where each cell's reconstructed edge states go
-  for (int t = 0; t < nt; t++) {
-    const auto h0 = T.hcell.begin() + T.hoff[t], h1 = T.hcell.begin() + T.hoff[t + 1];
-    auto put = [&](int cell, int edge, int v) {
-      if (cell / B == t) T.cel[(size_t)edge * nc + cell] = (short)v;
-      else T.hel[(size_t)edge * NH + (std::lower_bound(h0, h1, cell) - T.hcell.begin())] = (short)v;
-    };
-    for (int e = T.toff[t]; e < T.toff[t + 1]; e++) {
-      const int f = ent[e], k = e - T.toff[t] + 1;
-      put(H.fe0[f], H.fsl[f] & 3, k);
-      put(H.fe1[f], H.fsl[f] >> 2, -k);
-    }
-  }
-  // slot places: interior slots by the face's place, boundary slots by the
-  // place in the tile's boundary list (own cells' first)
-  std::vector<int> loc0(H.nf > 0 ? H.nf : 1, -1), loc1(H.nf > 0 ? H.nf : 1, -1);
-  for (int t = 0; t < nt; t++)
-    for (int e = T.toff[t]; e < T.toff[t + 1]; e++) {
-      const int f = ent[e];
-      if (H.fe0[f] / B == t) loc0[f] = e - T.toff[t];
-      if (H.fe1[f] / B == t) loc1[f] = e - T.toff[t];
-    }
+  std::vector<int> last(nt);
+  auto each_halo = [&](auto fn) {
+    std::fill(last.begin(), last.end(), -1);
+    for (int c = 0; c < nc; c++)
+      for (int j = 0; j < 4; j++) {
+        const int e = H.cfn[(size_t)j * nc + c], t = e / B;
+        if (e < 0 || t == c / B || last[t] == c) continue;
+        last[t] = c;
+        fn(t, c);
+      }
+  };
+  each_halo([&](int t, int) { T.hoff[t + 1]++; });
+  for (int t = 0; t < nt; t++) T.hoff[t + 1] += T.hoff[t];
+  T.hcell.resize(T.hoff[nt]);
+  fill.assign(T.hoff.begin(), T.hoff.end() - 1);
+  each_halo([&](int t, int c) { T.hcell[fill[t]++] = c; });
   T.boff.assign(nt + 1, 0);
   T.bown.assign(nt, 0);
-  for (int t = 0; t < nt; t++) {
-    const int c1 = std::min(nc, (t + 1) * B), nown = c1 - t * B, n = nown + T.hoff[t + 1] - T.hoff[t];
-    int nb = 0;
-    for (int k = 0; k < n; k++) {
-      const bool own = k < nown;
-      const int h = T.hoff[t] + k - nown, i = own ? t * B + k : T.hcell[h];
-      for (int j = 0; j < 4; j++) {
-        short* v = own ? &T.csl[(size_t)j * nc + i] : &T.hsl[(size_t)j * NH + h];
-        const int cf = H.cface[(size_t)j * nc + i];
-        if (cf != 0) {
-          if (!own) continue;
-          const int f = cf > 0 ? cf - 1 : -cf - 1, l = cf > 0 ? loc0[f] : loc1[f];
-          if (l < 0 || (cf > 0 ? H.fe0[f] : H.fe1[f]) != i || ((H.bmask[i] >> j) & 1)) return false;
-          *v = (short)(cf > 0 ? l + 1 : -(l + 1));
-        } else if ((H.bmask[i] >> j) & 1) {
-          T.tbq.push_back(-1 - H.cnbr[(size_t)j * nc + i]);
-          T.tbc.push_back(i);
-          *v = (short)++nb;
-        }
+  auto bounds = [&](int i, int tgt) {
+    for (int j = 0; j < 4; j++)
+      if ((H.bmask[i] >> j) & 1) {
+        T.tbq.push_back(-1 - H.cnbr[(size_t)j * nc + i]);
+        T.tbc.push_back(i);
+        T.btgt.push_back(tgt >= 0 ? tgt + j : tgt - j);
       }
-      if (own) T.bown[t] = nb;
-    }
-    T.capb = std::max(T.capb, nb);
+  };
+  for (int t = 0; t < nt; t++) {
+    for (int i = t * B; i < std::min(nc, (t + 1) * B); i++)
+      if (H.bmask[i]) bounds(i, 4 * i);
+    T.bown[t] = (int)T.tbq.size() - T.boff[t];
+    for (int h = T.hoff[t]; h < T.hoff[t + 1]; h++)
+      if (H.bmask[T.hcell[h]]) bounds(T.hcell[h], -1 - 4 * h);
     T.boff[t + 1] = (int)T.tbq.size();
+    T.capb = std::max(T.capb, T.boff[t + 1] - T.boff[t]);
   }
-  if (T.tbq.empty()) { T.tbq.push_back(0); T.tbc.push_back(0); }
-  T.capf = (T.capf + 7) & ~7;
   return 64 * (size_t)(T.capf + T.capb) <= CSU_TILE_LDS;
+}
+
+// The tile form's device lists and buffers.  scratch: device room for
+// T.ent, whose values end with the call.
+static int tile_setup(csu_dev* d, const HostTile& T, bool first, int* scratch) {
+  Tile& tl = d->tl;
+  const size_t nc = d->nc, ne = T.ent.size(), nh = T.hcell.empty() ? 1 : T.hcell.size();
+  // one array of all the host made that stays
+  std::vector<int> all;
+  std::vector<size_t> at;
+  for (const auto* v : {&T.toff, &T.hoff, &T.hcell, &T.boff, &T.bown, &T.tbq, &T.tbc, &T.btgt}) {
+    at.push_back(all.size());
+    all.insert(all.end(), v->begin(), v->end());
+  }
+  int rc;
+  const int* dv = nullptr;
+  double* f = nullptr;
+  short* sl = nullptr;
+  int* fc = nullptr;
+  if ((rc = upload(d, &dv, all)) || (rc = dalloc(d, &f, 3 * ne)) || (rc = dalloc(d, &sl, 8 * (nc + nh))) ||
+      (rc = dalloc(d, &d->Pa, 2 * nc)) || (rc = dalloc(d, &d->Pb4, 2 * nc)) ||
+      (first && (rc = dalloc(d, &fc, 2 * ne))))
+    return rc;
+  tl.toff = dv + at[0]; tl.hoff = dv + at[1]; tl.hcell = dv + at[2]; tl.boff = dv + at[3]; tl.bown = dv + at[4];
+  tl.tbq = dv + at[5]; tl.tbc = dv + at[6];
+  tl.nh = (int)nh;
+  tl.capf = T.capf;
+  d->tl_capb = T.capb;
+  d->tl_n = ne;
+  short *csl = sl, *cel = csl + 4 * nc, *hsl = cel + 4 * nc, *hel = hsl + 4 * nh;
+  if (ne) HIPCHK(hipMemcpyAsync(scratch, T.ent.data(), ne * sizeof(int), hipMemcpyHostToDevice, d->stream));
+  HIPCHK(hipMemsetAsync(sl, 0, 8 * (nc + nh) * sizeof(short), d->stream));
+  hipLaunchKernelGGL(k_tile_lists, dim3(nblk(d->nc)), dim3(CSU_CHUNK), 0, d->stream, d->nc, d->geo, tl, scratch,
+                     dv + at[7], f, f + ne, f + 2 * ne, first ? fc : nullptr, first ? fc + ne : nullptr, csl, cel, hsl,
+                     hel);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(d->stream));  // T ends with the caller's set-up
+  tl.fx = f; tl.fy = f + ne; tl.fs = f + 2 * ne;
+  tl.fa = fc; tl.fb = fc ? fc + ne : nullptr;
+  tl.csl = csl; tl.cel = cel; tl.hsl = hsl; tl.hel = hel;
+  return CSU_OK;
+}
+
+// FP32 copies of the tile form's face vectors.
+static int tile_f32(csu_dev* d) {
+  const size_t n = 3 * d->tl_n;
+  float* p = nullptr;
+  int rc = dalloc(d, &p, n);
+  if (rc) return rc;
+  if (n) hipLaunchKernelGGL(k_to_f32, dim3((unsigned)((n + CSU_BLOCK - 1) / CSU_BLOCK)), dim3(CSU_BLOCK), 0, d->stream,
+                            d->tl.fx, p, n);
+  HIPCHK(hipGetLastError());
+  d->tl.fx32 = p; d->tl.fy32 = p + d->tl_n; d->tl.fs32 = p + 2 * d->tl_n;
+  return CSU_OK;
 }
 
 // Device state of a context from its host arrays: uploads, allocations, wall
@@ -968,8 +996,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     d->quads = 0;
     for (int n : H.cnp) d->quads |= n == 4;
     HostTile T;
-    if (tile_lists(H, sol, first, T)) {
-      Tile& tl = d->tl;
+    if (tile_lists(H, sol, T)) {
       // Threads per tile: 512 let a tile's halo run beside its own cells and
       // both rounds of faces at once, which wins while the tiles leave the
       // chip idle (40k cells 77 -> 68 us per RK5 iteration, 100k quads 130 ->
@@ -978,24 +1005,9 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
       // in Morton order: 146 us with 256 threads, 157 with 512).
       const size_t halo = T.hoff.back();
       d->tile_nt = nc <= 131072 || 2 * halo > (size_t)nc ? 512 : 256;
-      tl.nh = (int)T.hcell.size();
-      tl.capf = T.capf;
-      d->tl_capb = T.capb;
-      d->tl_n = T.fx.size();
-      if ((rc = upload(d, &tl.toff, T.toff)) || (rc = upload(d, &tl.boff, T.boff)) ||
-          (rc = upload(d, &tl.bown, T.bown)) || (rc = upload(d, &tl.hoff, T.hoff)) || (rc = upload(d, &tl.tbq, T.tbq)) || (rc = upload(d, &tl.tbc, T.tbc)) ||
-          (rc = upload(d, &tl.hcell, T.hcell)) || (rc = upload(d, &tl.fx, T.fx)) || (rc = upload(d, &tl.fy, T.fy)) ||
-          (rc = upload(d, &tl.fs, T.fs)) || (rc = upload(d, &tl.csl, T.csl)) || (rc = upload(d, &tl.hsl, T.hsl)) ||
-          (rc = upload(d, &tl.cel, T.cel)) || (rc = upload(d, &tl.hel, T.hel)) || (rc = dalloc(d, &d->Pa, 2 * (size_t)nc)) ||
-          (rc = dalloc(d, &d->Pb4, 2 * (size_t)nc)))
-        return rc;
-      if (kp.mixed) {
-        auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
-        if ((rc = upload(d, &tl.fx32, f32(T.fx))) || (rc = upload(d, &tl.fy32, f32(T.fy))) ||
-            (rc = upload(d, &tl.fs32, f32(T.fs))))
-          return rc;
-      }
-      if (first && ((rc = upload(d, &tl.fa, T.fa)) || (rc = upload(d, &tl.fb, T.fb)))) return rc;
+      // a face is in at most two tiles' lists: they fit the room of the face fluxes
+      static_assert(2 * sizeof(int) <= 4 * sizeof(double), "entries of the tiles in the room of the face fluxes");
+      if ((rc = tile_setup(d, T, first, (int*)s.fflux)) || (kp.mixed && (rc = tile_f32(d)))) return rc;
       d->tile_ok = d->pu;
       d->tile1 = first && (double)d->tl.nh <= 1.25 * nc;
     }
@@ -2077,10 +2089,7 @@ extern "C" int csu_dev_set_precision(csu_dev* d, int32_t prec) {
       return rc;
     if (!s.fflux32 && (rc = dalloc(d, &s.fflux32, (size_t)d->nv * nf))) return rc;
     if (d->prm.order == 2 && !s.rec32 && (rc = dalloc(d, &s.rec32, 4 * nvc))) return rc;
-    if ((d->tile_ok || d->tile1) && !d->tl.fx32 && ((rc = f32(d->tl.fx, &d->tl.fx32, d->tl_n)) ||
-                                      (rc = f32(d->tl.fy, &d->tl.fy32, d->tl_n)) ||
-                                      (rc = f32(d->tl.fs, &d->tl.fs32, d->tl_n))))
-      return rc;
+    if ((d->tile_ok || d->tile1) && !d->tl.fx32 && (rc = tile_f32(d))) return rc;
   } else if (d->prm.order == 2 && !s.rec && (rc = dalloc(d, &s.rec, 4 * nvc))) {
     return rc;
   }
