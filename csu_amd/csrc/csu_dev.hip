@@ -727,14 +727,23 @@ static void tune_lookup(csu_dev* d) {
 // copies and the cells' places in these lists are k_tile_lists' work; made
 // here they took three quarters of the time.  btgt: the slot 4 cell + j of an
 // own cell's boundary face, -1 - (4 place in hcell + j) of a halo cell's.
-// False when a tile has more interior faces than CSU_TILE_FACES or its LDS
-// arrays do not fit.
+// first: a first-order run, which reads nothing of its halo and takes the form
+// or not by the halos' size alone.  False when a tile has more interior faces
+// than CSU_TILE_FACES, its LDS arrays do not fit, or first and the halos are
+// too large.
+#define TILE_HALO 1.25  // halo cells per cell up to which the tile form is the default (dev_setup)
+// LDS bytes of k_stage: the faces' two states, in place of which their fluxes
+// go (a first-order run keeps the fluxes only), and the boundary entries.
+static size_t tile_lds(bool first, bool mixed, size_t capf, size_t capb) {
+  return (first ? 4 : 8) * (mixed ? sizeof(float) : sizeof(double)) * capf + 8 * sizeof(double) * capb;
+}
+
 struct HostTile {
   std::vector<int> toff, ent, hoff, hcell, boff, bown, tbq, tbc, btgt;
   int capf = 0, capb = 0;
 };
 
-static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, HostTile& T) {
+static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, bool first, HostTile& T) {
   if (!H.linked) return false;
   const int nc = H.nc, B = CSU_CHUNK, nt = (nc + B - 1) / B;
   auto each_face = [&](auto fn) {
@@ -780,9 +789,12 @@ static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, HostTi
   };
   each_halo([&](int t, int) { T.hoff[t + 1]++; });
   for (int t = 0; t < nt; t++) T.hoff[t + 1] += T.hoff[t];
-  T.hcell.resize(T.hoff[nt]);
-  fill.assign(T.hoff.begin(), T.hoff.end() - 1);
-  each_halo([&](int t, int c) { T.hcell[fill[t]++] = c; });
+  if (first && T.hoff[nt] > TILE_HALO * nc) return false;
+  if (!first) {
+    T.hcell.resize(T.hoff[nt]);
+    fill.assign(T.hoff.begin(), T.hoff.end() - 1);
+    each_halo([&](int t, int c) { T.hcell[fill[t]++] = c; });
+  }
   T.boff.assign(nt + 1, 0);
   T.bown.assign(nt, 0);
   auto bounds = [&](int i, int tgt) {
@@ -797,12 +809,12 @@ static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, HostTi
     for (int i = t * B; i < std::min(nc, (t + 1) * B); i++)
       if (H.bmask[i]) bounds(i, 4 * i);
     T.bown[t] = (int)T.tbq.size() - T.boff[t];
-    for (int h = T.hoff[t]; h < T.hoff[t + 1]; h++)
+    for (int h = T.hoff[t]; h < T.hoff[t + 1] && !first; h++)
       if (H.bmask[T.hcell[h]]) bounds(T.hcell[h], -1 - 4 * h);
     T.boff[t + 1] = (int)T.tbq.size();
     T.capb = std::max(T.capb, T.boff[t + 1] - T.boff[t]);
   }
-  return 64 * (size_t)(T.capf + T.capb) <= CSU_TILE_LDS;
+  return tile_lds(first, false, T.capf, T.capb) <= CSU_TILE_LDS;
 }
 
 // The tile form's device lists and buffers.  scratch: device room for
@@ -817,12 +829,11 @@ static int tile_setup(csu_dev* d, const HostTile& T, bool first, int* scratch) {
     at.push_back(all.size());
     all.insert(all.end(), v->begin(), v->end());
   }
-  int rc;
-  const int* dv = nullptr;
+  int rc, *dv = nullptr, *fc = nullptr;
   double* f = nullptr;
   short* sl = nullptr;
-  int* fc = nullptr;
-  if ((rc = upload(d, &dv, all)) || (rc = dalloc(d, &f, 3 * ne)) || (rc = dalloc(d, &sl, 8 * (nc + nh))) ||
+  const size_t nsl = first ? 4 * nc : 8 * (nc + nh);
+  if ((rc = dalloc(d, &dv, all.size())) || (rc = dalloc(d, &f, 3 * ne)) || (rc = dalloc(d, &sl, nsl)) ||
       (rc = dalloc(d, &d->Pa, 2 * nc)) || (rc = dalloc(d, &d->Pb4, 2 * nc)) ||
       (first && (rc = dalloc(d, &fc, 2 * ne))))
     return rc;
@@ -832,14 +843,18 @@ static int tile_setup(csu_dev* d, const HostTile& T, bool first, int* scratch) {
   tl.capf = T.capf;
   d->tl_capb = T.capb;
   d->tl_n = ne;
-  short *csl = sl, *cel = csl + 4 * nc, *hsl = cel + 4 * nc, *hel = hsl + 4 * nh;
+  short *csl = sl, *cel = nullptr, *hsl = nullptr, *hel = nullptr;
+  if (!first) { cel = csl + 4 * nc; hsl = cel + 4 * nc; hel = hsl + 4 * nh; }
+  HIPCHK(hipMemcpyAsync(dv, all.data(), all.size() * sizeof(int), hipMemcpyHostToDevice, d->stream));
   if (ne) HIPCHK(hipMemcpyAsync(scratch, T.ent.data(), ne * sizeof(int), hipMemcpyHostToDevice, d->stream));
-  HIPCHK(hipMemsetAsync(sl, 0, 8 * (nc + nh) * sizeof(short), d->stream));
-  hipLaunchKernelGGL(k_tile_lists, dim3(nblk(d->nc)), dim3(CSU_CHUNK), 0, d->stream, d->nc, d->geo, tl, scratch,
-                     dv + at[7], f, f + ne, f + 2 * ne, first ? fc : nullptr, first ? fc + ne : nullptr, csl, cel, hsl,
-                     hel);
+  HIPCHK(hipMemsetAsync(sl, 0, nsl * sizeof(short), d->stream));
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nblk(d->nc)), dim3(CSU_CHUNK), 0, d->stream, d->nc, d->geo, tl, scratch, dv + at[7],
+                       f, f + ne, f + 2 * ne, fc, first ? fc + ne : nullptr, csl, cel, hsl, hel);
+  };
+  first ? go(k_tile_lists<true>) : go(k_tile_lists<false>);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(d->stream));  // T ends with the caller's set-up
+  HIPCHK(hipStreamSynchronize(d->stream));  // all and T end with the set-up
   tl.fx = f; tl.fy = f + ne; tl.fs = f + 2 * ne;
   tl.fa = fc; tl.fb = fc ? fc + ne : nullptr;
   tl.csl = csl; tl.cel = cel; tl.hsl = hsl; tl.hel = hel;
@@ -996,7 +1011,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     d->quads = 0;
     for (int n : H.cnp) d->quads |= n == 4;
     HostTile T;
-    if (tile_lists(H, sol, T)) {
+    if (tile_lists(H, sol, first, T)) {
       // Threads per tile: 512 let a tile's halo run beside its own cells and
       // both rounds of faces at once, which wins while the tiles leave the
       // chip idle (40k cells 77 -> 68 us per RK5 iteration, 100k quads 130 ->
@@ -1009,7 +1024,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
       static_assert(2 * sizeof(int) <= 4 * sizeof(double), "entries of the tiles in the room of the face fluxes");
       if ((rc = tile_setup(d, T, first, (int*)s.fflux)) || (kp.mixed && (rc = tile_f32(d)))) return rc;
       d->tile_ok = d->pu;
-      d->tile1 = first && (double)d->tl.nh <= 1.25 * nc;
+      d->tile1 = first;
     }
   }
   if (!d->tile_ok) d->tile = 0;
@@ -1018,7 +1033,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   // longer than a tile have one halo cell per cell, and there the two forms
   // measure alike at 2.0M cells (1,309 us, split 1,321) and the tile form
   // wins below (406k cells 288 against 340)
-  else if (!d->tuned && (double)d->tl.nh <= 1.25 * nc) d->tile = 1;
+  else if (!d->tuned && (double)d->tl.nh <= TILE_HALO * nc) d->tile = 1;
   if (kp.mixed) {
     auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
     if ((rc = upload(d, &g.wg32, f32(H.wg))) ||
@@ -1385,7 +1400,7 @@ template <int NT>
 static int tile_stage(csu_dev* d, int flags, double sigma, double rk_a) {
   const KP& kp = d->kp;
   const St& st = d->st;
-  const size_t lds = 8 * ((kp.mixed ? 4 : 8) * (size_t)d->tl.capf + 8 * (size_t)d->tl_capb);
+  const size_t lds = tile_lds(d->tile1, kp.mixed, d->tl.capf, d->tl_capb);
   double* const rdt = d->red + 4 * (size_t)d->nred;
   const dim3 gu(nblk(d->nc)), bu(NT);
   Prof p(d, "k_stage");
@@ -2376,7 +2391,8 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
     double cross = m->face ? 0 : nf;
     for (int f = 0; m->face && f < m->nface; f++)
       cross += m->face[4 * (size_t)f] / CSU_CHUNK != m->face[4 * (size_t)f + 1] / CSU_CHUNK;
-    b += nc * (64 + 16) + (nf + cross) * ((p->precision == 1 ? 36 : 24) + (p->order == 1 ? 8 : 0)) + 2 * cross * 20 + 12 * nb + 16 * (nc / 256 + 2);
+    b += nc * (64 + (p->order == 1 ? 8 : 16)) + (nf + cross) * ((p->precision == 1 ? 36 : 24) + (p->order == 1 ? 8 : 0)) +
+         (p->order == 1 ? 0 : 2 * cross * 20) + 16 * nb + 16 * (nc / 256 + 2);
   }
   b += (nv + 4) * 8 * (double)(hist > 0 ? hist : 1);
   // allocation granularity: every array rounds up (at most 2 MiB slack per large array)

@@ -30,11 +30,13 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_to_f32(const double* __restrict__
 
 // The tile form's lists (struct Tile), a workgroup per tile, from the faces
 // (ent, ascending), halo cells and boundary entries that the host found for
-// it: the faces' vectors (fa non-null: and cells) in entry order, and the
-// places of every own and halo cell's slots and edges in the tile's lists.
+// it: the faces' vectors in entry order, and the places of every own and halo
+// cell's slots and edges in the tile's lists (O1: the faces' cells, and the
+// own cells' slots only).
 // csl, cel, hsl, hel are zero before.  Each own face slot's face is in ent
 // (HostMesh::linked), each cell across an outer face in the halo list.
 // Bound by its gathers, 25 us at 400k cells, where the host's loops took 30 ms.
+template <bool O1>
 __global__ __launch_bounds__(CSU_CHUNK) void k_tile_lists(int nc, Geo g, Tile tl, const int* __restrict__ ent,
                                                           const int* __restrict__ btgt, double* __restrict__ fx,
                                                           double* __restrict__ fy, double* __restrict__ fs,
@@ -61,9 +63,12 @@ __global__ __launch_bounds__(CSU_CHUNK) void k_tile_lists(int nc, Geo g, Tile tl
   for (int k = t; k < n; k += CSU_CHUNK) {
     const int f = ent[e0 + k], a = g.fe0[f], b = g.fe1[f], sl = g.fsl[f];
     fx[e0 + k] = g.fdsx[f]; fy[e0 + k] = g.fdsy[f]; fs[e0 + k] = g.fds[f];
-    if (fa) { fa[e0 + k] = a; fb[e0 + k] = b; }
-    edge(a, sl & 3, k + 1);
-    edge(b, sl >> 2, -(k + 1));
+    if (O1) {
+      fa[e0 + k] = a; fb[e0 + k] = b;
+    } else {
+      edge(a, sl & 3, k + 1);
+      edge(b, sl >> 2, -(k + 1));
+    }
   }
   const int i = tile * CSU_CHUNK + t;
   for (int j = 0; j < 4 && i < nc; j++) {

@@ -269,7 +269,7 @@ __global__ __launch_bounds__(NT, 4) void k_stage(KP kp, Geo g, St s, Tile tl, in
   const SolveP* sv = g.sol ? g.sol + sid : nullptr;
   const double minf = sv ? sv->minf : kp.minf;
   TF* sf = (TF*)smem;
-  double* sb = smem + (MIX ? 4 : 8) * tl.capf;
+  double* sb = smem + (MIX ? 4 : 8) / (O1 ? 2 : 1) * tl.capf;  // O1: sf holds the fluxes only
   const int f0 = tl.toff[tile], nft = tl.toff[tile + 1] - f0;
   const int b0 = tl.boff[tile], h0 = tl.hoff[tile], nh = tl.hoff[tile + 1] - h0;
   const int nown = min(CSU_CHUNK, (sv ? sv->c1 : nc) - c0), nbt = tl.boff[tile + 1] - b0;

@@ -82,3 +82,27 @@ def test_batch_of_such_meshes(tmpcase):
         b.close()
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_first_order_holds_no_lists_it_does_not_read(tmpcase, monkeypatch, precision):
+    """A first-order run takes the form or not by its halos alone: on a
+    scattered numbering it holds what the split form holds, not a byte of
+    lists; where it takes the form, two buffers of primitives, its own cells'
+    slots, its boundary faces, and its tiles' faces with their cells."""
+    held = {}
+    for mesh in ("scattered_triangles", "hybrid"):
+        d = tmpcase("fo")
+        cases.write_case(d, MESHES[mesh](), cases.ramp_input(threads=1, nmax=1, precision=precision, order=1))
+        c = native.HostCase(d)
+        for stored in ("1", "0"):
+            monkeypatch.setenv("CSU_STORED_PRIMITIVES", stored)
+            dev = native.Device(c)
+            held[mesh, stored] = dev.bytes()
+            dev.close()
+    assert held["scattered_triangles", "0"] == held["scattered_triangles", "1"]
+    nt = (c.ncell + 255) // 256
+    e = c.arrays()["face"][:, :2] // 256
+    entries = c.nface + int((e[:, 0] != e[:, 1]).sum())
+    lists = 4 * (3 * (nt + 1) + nt + 3 * c.nbface) + entries * (24 + 8 + 12 * precision) + 8 * c.ncell
+    assert held["hybrid", "0"] - held["hybrid", "1"] == lists + 64 * c.ncell
