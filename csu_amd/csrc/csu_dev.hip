@@ -9,6 +9,7 @@
 #include <math.h>
 #include <algorithm>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <tuple>
 #include <string>
@@ -22,7 +23,7 @@
 using namespace csu;
 
 #define CSU_MAX_DEVICES 64
-#define RESIDUAL_ONE_COPY (4u << 20)  // bytes up to which csu_dev_residual copies everything at once
+#define RESIDUAL_ONE_COPY (2u << 20)  // bytes up to which csu_dev_residual copies its six fields at once
 
 // ---------------------------------------------------------------------------
 // error reporting
@@ -1450,25 +1451,41 @@ extern "C" int csu_dev_residual(csu_dev* d, double* R, double* dPx, double* dPy,
   if (rc) return rc;
   const size_t nvc = (size_t)d->nv * d->nc, nc = d->nc, nb = d->nb;
   const int ns = d->nv + 1;
-  const size_t all = 4 * nvc + 2 * nc + ns * (nc + nb);
-  if (all * sizeof(double) <= RESIDUAL_ONE_COPY) {
-    // a small mesh: the copies' fixed cost (about 13 us each into pageable
-    // memory) outweighs the second pass over the values on the host.  1,394
-    // cells: 145 -> 68 us; above the bound the second pass costs more.
-    std::vector<double> h(all);
-    HIPCHK(hipMemcpyAsync(h.data(), d->fields, all * sizeof(double), hipMemcpyDeviceToHost, d->stream));
+  // Several fields of a small mesh come in one copy of the run from the first
+  // to the last of them: a copy of its own costs about 12 us each into
+  // pageable memory, a byte of the run one more pass on the host.  All six,
+  // separate copies -> one: 2,700 cells 137 -> 70 us, 10,000 cells (1.8 MB)
+  // 200 -> 172 us, 13,200 cells 225 -> 229 us, 20,800 cells 278 -> 327 us,
+  // hence the bound.  It falls with the copies saved: both gradients of 7,200
+  // cells 66 -> 64 us, of 13,200 82 -> 86 us; R and P of 4,800 cells, with
+  // the fields between them, 69 -> 85 us.
+  const int tx = d->visc ? 1 : 0;  // a gradient's slot 3 is a copy of its own
+  const size_t len[8] = {nvc, nvc, nvc, nvc, nc, nc, ns * nc, ns * nb};  // the fields as they lie in d->fields
+  const bool want[8] = {R != nullptr, dPx != nullptr, dPy != nullptr, phi != nullptr, dPx && tx, dPy && tx,
+                        P != nullptr, Pb != nullptr};
+  size_t at[9] = {0}, lo = SIZE_MAX, hi = 0;
+  int copies = 0;
+  for (int q = 0; q < 8; q++) {
+    at[q + 1] = at[q] + len[q];
+    if (!want[q]) continue;
+    copies++;
+    lo = std::min(lo, at[q]);
+    hi = at[q + 1];
+  }
+  if (copies > 1 && (hi - lo) * sizeof(double) <= (size_t)std::min(copies - 1, 5) * (RESIDUAL_ONE_COPY / 5)) {
+    const std::unique_ptr<double[]> buf(new double[hi - lo]);
+    HIPCHK(hipMemcpyAsync(buf.get(), d->fields + lo, (hi - lo) * sizeof(double), hipMemcpyDeviceToHost, d->stream));
     HIPCHK(hipStreamSynchronize(d->stream));
+    auto h = [&](int q) { return buf.get() + (at[q] - lo); };
     double* const out[4] = {R, dPx, dPy, phi};
     for (int q = 0; q < 4; q++)
-      if (out[q]) memcpy(out[q], h.data() + q * nvc, nvc * sizeof(double));
-    if (d->visc)  // the reference's gradient slot 3 holds grad T (solverGrad_T, solver.c:477-490)
-      for (int q = 0; q < 2; q++)
-        if (out[1 + q]) memcpy(out[1 + q] + 3 * nc, h.data() + 4 * nvc + q * nc, nc * sizeof(double));
-    const double *hp = h.data() + 4 * nvc + 2 * nc, *hb = hp + ns * nc;
+      if (out[q]) memcpy(out[q], h(q), nvc * sizeof(double));
+    for (int q = 0; q < 2; q++)  // the reference's gradient slot 3 holds grad T (solverGrad_T, solver.c:477-490)
+      if (want[4 + q]) memcpy(out[1 + q] + 3 * nc, h(4 + q), nc * sizeof(double));
     for (size_t i = 0; P && i < nc; i++)
-      for (int m = 0; m < ns; m++) P[i * ns + m] = hp[m * nc + i];
+      for (int m = 0; m < ns; m++) P[i * ns + m] = h(6)[m * nc + i];
     for (size_t i = 0; Pb && i < nb; i++)
-      for (int m = 0; m < ns; m++) Pb[i * ns + m] = hb[m * nb + i];
+      for (int m = 0; m < ns; m++) Pb[i * ns + m] = h(7)[m * nb + i];
     return CSU_OK;
   }
   if (R) HIPCHK(hipMemcpyAsync(R, d->R, nvc * sizeof(double), hipMemcpyDeviceToHost, d->stream));
