@@ -93,6 +93,7 @@ struct csu_dev {
   size_t tl_n;                 // interior entries in all
   dbl2 *Pa, *Pb4;              // tile form: primitives r u v p [nc][4], current and the one a stage writes
   int tuned;                   // launch shapes from the autotuner (1) or the defaults (0)
+  int shape_set;               // launch shapes set by the caller
   // implicit schemes
   double *Dp, *dW0, *dW1, *A;  // diagonal (without the dt term), increments, DPLUR blocks
   double* caux;                // LU-SGS: per cell c, max(4/(3r), gamma/r), mu/Pr of the iteration's state [3][nc]
@@ -732,7 +733,8 @@ static void tune_lookup(csu_dev* d) {
 // or not by the halos' size alone.  False when a tile has more interior faces
 // than CSU_TILE_FACES, its LDS arrays do not fit, or first and the halos are
 // too large.
-#define TILE_HALO 1.25  // halo cells per cell up to which the tile form is the default (dev_setup)
+#define TILE_SMALL 131072  // cells up to which the tiles leave the chip idle
+#define TILE_HALO 1.25     // halo cells per cell up to which the tile form is the default (tile_default)
 // LDS bytes of k_stage: the faces' two states, in place of which their fluxes
 // go (a first-order run keeps the fluxes only), and the boundary entries.
 static size_t tile_lds(bool first, bool mixed, size_t capf, size_t capb) {
@@ -816,6 +818,27 @@ static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, bool f
     T.capb = std::max(T.capb, T.boff[t + 1] - T.boff[t]);
   }
   return tile_lds(first, false, T.capf, T.capb) <= CSU_TILE_LDS;
+}
+
+// The form of an untuned context: the tile form wherever it exists, unless
+// the halos hold clearly more cells than the tiles (a scattered numbering).
+// What the tile form saves in memory traffic it pays in gradients of the
+// halo, so where a gradient costs more (double-double sums) or the traffic
+// less (mixed precision, above the sizes where launches count) the halo may
+// be half as large as the tiles at most.  RK5 iterations, split -> tile, 0.29
+// halo cells per cell (Morton order) and 1.0 (columns longer than a tile):
+//   FP64, Roe       400k cells 286 -> 202 us | 200k 188 -> 175, 800k 569 -> 474
+//   FP64, AUSM+up   400k 291 -> 229          | 200k 188 -> 196, 800k 577 -> 529
+//   mixed, Roe      400k 217 -> 182          | 200k 154 -> 152, 800k 344 -> 365
+//   mixed, AUSMDV   400k 221 -> 197          | 200k 157 -> 171, 800k 349 -> 444
+//   mixed, 100k columns: Roe 108 -> 91, AUSMDV 114 -> 95
+//   long double least squares, Roe:
+//                   400k 386 -> 377          | 200k 252 -> 319, 800k 717 -> 895
+//                   100k 158 -> 161, quads 180k 245 -> 236 | 100k 160 -> 186
+static int tile_default(const csu_dev* d) {
+  if (!d->tile_ok) return 0;
+  const bool half = d->kp.lsq_ld || (d->kp.mixed && d->nc > TILE_SMALL);
+  return (double)d->tl.nh <= (half ? 0.5 : TILE_HALO) * d->nc;
 }
 
 // The tile form's device lists and buffers.  scratch: device room for
@@ -1020,7 +1043,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
       // cells 205 -> 181 us); above that, more tiles per CU win (200k cells
       // in Morton order: 146 us with 256 threads, 157 with 512).
       const size_t halo = T.hoff.back();
-      d->tile_nt = nc <= 131072 || 2 * halo > (size_t)nc ? 512 : 256;
+      d->tile_nt = nc <= TILE_SMALL || 2 * halo > (size_t)nc ? 512 : 256;
       // a face is in at most two tiles' lists: they fit the room of the face fluxes
       static_assert(2 * sizeof(int) <= 4 * sizeof(double), "entries of the tiles in the room of the face fluxes");
       if ((rc = tile_setup(d, T, first, (int*)s.fflux)) || (kp.mixed && (rc = tile_f32(d)))) return rc;
@@ -1029,12 +1052,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     }
   }
   if (!d->tile_ok) d->tile = 0;
-  // untuned default: the tile form wherever it exists, unless the halos hold
-  // clearly more cells than the tiles (a scattered numbering): columns
-  // longer than a tile have one halo cell per cell, and there the two forms
-  // measure alike at 2.0M cells (1,309 us, split 1,321) and the tile form
-  // wins below (406k cells 288 against 340)
-  else if (!d->tuned && (double)d->tl.nh <= TILE_HALO * nc) d->tile = 1;
+  else if (!d->tuned) d->tile = tile_default(d);
   if (kp.mixed) {
     auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
     if ((rc = upload(d, &g.wg32, f32(H.wg))) ||
@@ -1137,7 +1155,7 @@ static csu_dev* dev_new() {
   memset((void*)&d->geo, 0, sizeof(Geo));
   memset((void*)&d->st, 0, sizeof(St));
   memset((void*)&d->tl, 0, sizeof(Tile));
-  d->Pa = d->Pb4 = nullptr; d->quads = 1; d->tl_capb = 0; d->tl_n = 0; d->tile1 = 0;
+  d->Pa = d->Pb4 = nullptr; d->quads = 1; d->tl_capb = 0; d->tl_n = 0; d->tile1 = 0; d->shape_set = 0;
   return d;
 }
 
@@ -1891,6 +1909,7 @@ extern "C" int csu_dev_set_launch_shape(csu_dev* d, const int32_t* choice) {
   d->kp.xcd = choice[2];
   d->tile = choice[3];
   d->tuned = 0;
+  d->shape_set = 1;
   return CSU_OK;
 }
 
@@ -2130,6 +2149,10 @@ extern "C" int csu_dev_set_precision(csu_dev* d, int32_t prec) {
   d->kp.lsq_ld = prec == CSU_PREC_FP64_LD;
   d->prm.precision = prec;
   graphs_drop(d);  // the captured iterations launch the other kernels
+  if (!d->tuned && !d->shape_set && d->tile != tile_default(d)) {
+    d->tile = tile_default(d);
+    d->fresh = 1;  // as in csu_dev_set_launch_shape
+  }
   return CSU_OK;
 }
 
