@@ -692,36 +692,22 @@ static void limiter_pref(const csu_params* p, double* pref) {
 // ---------------------------------------------------------------------------
 // Launch shapes that do not change any result (no reduction depends on
 // them): workgroup size of the gradient and face kernels, of the LU-SGS
-// level launches, and the XCD-contiguous tile map.  The tuner times each
-// candidate on a context and keeps the fastest; the choice is remembered
-// per kind of run and mesh-size bucket (log2 of the cell count) and taken
-// by every later context of that bucket in the process.
+// level launches, the XCD-contiguous tile map, and the tile form.  The tuner
+// times each candidate on a context and keeps the fastest; the choice is
+// remembered per kind of run and mesh-size bucket (log2 of the cell count) and
+// taken by every later context of that bucket in the process.  form: 0 no tile
+// form, 1 the tile form is the untuned default, 2 it is not (large halos), 3 a
+// first-order run in it; a choice between the forms holds for its like only.
 struct TuneKey {
-  int nv, visc, scheme, prec, order, bucket;
+  int nv, visc, scheme, prec, order, form, bucket;
   bool operator<(const TuneKey& o) const {
-    return std::tie(nv, visc, scheme, prec, order, bucket) < std::tie(o.nv, o.visc, o.scheme, o.prec, o.order, o.bucket);
+    return std::tie(nv, visc, scheme, prec, order, form, bucket) <
+           std::tie(o.nv, o.visc, o.scheme, o.prec, o.order, o.form, o.bucket);
   }
 };
 struct TuneVal { int sblk, lblk, xcd, tile; };
 static std::mutex g_tune_mu;
 static std::map<TuneKey, TuneVal> g_tune;
-
-static TuneKey tune_key(const csu_dev* d) {
-  int b = 0;
-  while ((1 << (b + 1)) <= d->nc && b < 30) b++;
-  return TuneKey{d->nv, d->visc, d->prm.time_scheme, d->prm.precision, d->prm.order, b};
-}
-
-static void tune_lookup(csu_dev* d) {
-  std::lock_guard<std::mutex> lock(g_tune_mu);
-  auto it = g_tune.find(tune_key(d));
-  if (it == g_tune.end()) return;
-  d->sblk = it->second.sblk;
-  d->lblk = it->second.lblk;
-  d->tile = it->second.tile;  // dropped again by dev_setup when the context has no tile lists
-  d->kp.xcd = it->second.xcd;
-  d->tuned = 1;
-}
 
 // What the host makes of the tile form's lists (k_stage, struct Tile) over the
 // 256-cell tiles of a mesh or of a batch's solves: each tile's interior faces
@@ -841,6 +827,25 @@ static int tile_default(const csu_dev* d) {
   return (double)d->tl.nh <= (half ? 0.5 : TILE_HALO) * d->nc;
 }
 
+static TuneKey tune_key(const csu_dev* d) {
+  int b = 0;
+  while ((1 << (b + 1)) <= d->nc && b < 30) b++;
+  const int form = d->tile1 ? 3 : !d->tile_ok ? 0 : tile_default(d) ? 1 : 2;
+  return TuneKey{d->nv, d->visc, d->prm.time_scheme, d->prm.precision, d->prm.order, form, b};
+}
+
+// The remembered choice for a context whose tile lists are made.
+static void tune_lookup(csu_dev* d) {
+  std::lock_guard<std::mutex> lock(g_tune_mu);
+  auto it = g_tune.find(tune_key(d));
+  if (it == g_tune.end()) return;
+  d->sblk = it->second.sblk;
+  d->lblk = it->second.lblk;
+  d->tile = it->second.tile;
+  d->kp.xcd = it->second.xcd;
+  d->tuned = 1;
+}
+
 // The tile form's device lists and buffers.  scratch: device room for
 // T.ent, whose values end with the call.
 static int tile_setup(csu_dev* d, const HostTile& T, bool first, int* scratch) {
@@ -930,7 +935,6 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
   d->tile_ok = 0;
   kp.xcd = 1;
   d->tuned = 0;
-  tune_lookup(d);
   // inviscid ideal-gas second-order RK with the default limiter (any
   // precision): the stages before the last store the next stage's
   // primitives r u v p instead of its state (k_update PO), and the tile form
@@ -1051,8 +1055,8 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
       d->tile1 = first;
     }
   }
-  if (!d->tile_ok) d->tile = 0;
-  else if (!d->tuned) d->tile = tile_default(d);
+  d->tile = tile_default(d);
+  tune_lookup(d);
   if (kp.mixed) {
     auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
     if ((rc = upload(d, &g.wg32, f32(H.wg))) ||
@@ -1841,14 +1845,15 @@ extern "C" int csu_dev_autotune(csu_dev* d, int32_t iters, int32_t* choice) {
   if (!rc) rc = enqueue_iterations(d, 2 * iters + 2);
   const int sbs[3] = {64, 128, 256};
   const bool lus = d->prm.time_scheme == CSU_TIME_LUSGS;
+  const int sblk0 = d->sblk;
   TuneVal best{d->sblk, d->lblk, d->kp.xcd, d->tile};
   float best_ms = 1e30f;
   for (int u = 0; u < (d->tile_ok ? 2 : 1) && !rc; u++)
-  for (int a = u ? 2 : 0; a < 3 && !rc; a++)  // the tile form has no gradient and face workgroups
+  for (int a = u ? 2 : 0; a < 3 && !rc; a++)
     for (int b = 0; b < (lus ? 3 : 1) && !rc; b++)
       for (int x = 1; x >= 0 && !rc; x--) {
         d->tile = u;
-        d->sblk = sbs[a];
+        d->sblk = u ? sblk0 : sbs[a];  // no gradient and face workgroups in the tile form: as they were
         d->lblk = lus ? sbs[b] : d->lblk;
         d->kp.xcd = x;
         if ((rc = tune_reset(d, saved)) || (rc = enqueue_iterations(d, 2))) break;
