@@ -77,5 +77,14 @@ def build(verbose: bool = False) -> str:
     return so
 
 
+def build_test_lib(src: str, name: str, verbose: bool = False) -> str:
+    """A HIP source of the tests as a library of its own beside libcsu.so,
+    with the kernels' flags."""
+    so = os.path.join(LIB, name)
+    _run([HIPCC, *HIP_FLAGS, "-shared", "-o", so + ".tmp", src], verbose)
+    os.replace(so + ".tmp", so)
+    return so
+
+
 if __name__ == "__main__":
     print(build(verbose="-v" in sys.argv))

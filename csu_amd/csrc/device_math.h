@@ -28,9 +28,11 @@ struct GasD {
 // Quotients that share a denominator.  b is inverted once (two Newton steps
 // from the hardware estimate); a quotient is then a*r corrected by its exact
 // remainder (a fused multiply-add), which rounds correctly (Markstein 1990),
-// so each equals a / b bit for bit as long as neither b nor the quotient is
-// near the ends of the exponent range; zeros, infinities and NaN go
-// through the hardware's fix-up as in a / b.  4 instructions per FP64
+// so each equals a / b bit for bit while nothing comes near the ends of the
+// exponent range (it omits a / b's scaling): FP64 for b and quotients from
+// 2^-1000 to 2^1000 and a from 2^-960 on, FP32 for b and quotients from 2^-120
+// to 2^120 and a from 2^-100 on (tests/quotients.hip); zeros, infinities and
+// NaN go through the hardware's fix-up as in a / b.  4 instructions per FP64
 // quotient after 5 for the reciprocal, against 11 for a / b.
 template <typename T>
 struct Den;
@@ -64,8 +66,8 @@ struct Den<float> {  // one Newton step, two remainder corrections
 // Square root, correctly rounded as sqrt() is: Goldschmidt's coupled
 // iteration from the hardware's reciprocal root, then two corrections by the
 // exact remainder (Markstein 1990).  Half of sqrt()'s instructions: no
-// scaling of the argument, which only values near the ends of the exponent
-// range need (below 2^-767).
+// scaling of the argument, which only values below 2^-760 need
+// (tests/quotients.hip).
 __device__ __forceinline__ double fsqrt(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
