@@ -863,9 +863,14 @@ static int tile_setup(csu_dev* d, const HostTile& T, bool first, int* scratch) {
   short* sl = nullptr;
   const size_t nsl = first ? 4 * nc : 8 * (nc + nh);
   if ((rc = dalloc(d, &dv, all.size())) || (rc = dalloc(d, &f, 3 * ne)) || (rc = dalloc(d, &sl, nsl)) ||
-      (rc = dalloc(d, &d->Pa, 2 * nc)) || (rc = dalloc(d, &d->Pb4, 2 * nc)) ||
-      (first && (rc = dalloc(d, &fc, 2 * ne))))
+      (first && ((rc = dalloc(d, &d->Pa, 4 * nc)) || (rc = dalloc(d, &fc, 2 * ne)))))
     return rc;
+  // the two buffers of primitives: second order in the room of the split
+  // kernels' edge states (16 nc doubles, or in mixed precision floats), which
+  // only csu_dev_residual and iterations in the split form write, and after
+  // either the primitives are derived again (fresh)
+  if (!first) d->Pa = d->st.rec ? (dbl2*)d->st.rec : (dbl2*)d->st.rec32;
+  d->Pb4 = d->Pa + 2 * nc;
   tl.toff = dv + at[0]; tl.hoff = dv + at[1]; tl.hcell = dv + at[2]; tl.boff = dv + at[3]; tl.bown = dv + at[4];
   tl.tbq = dv + at[5]; tl.tbc = dv + at[6];
   tl.nh = (int)nh;
@@ -1033,7 +1038,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     g.sol = sol_d;
     d->sol_host = *sol;
   }
-  if (p->order == 2 && !kp.mixed && (rc = dalloc(d, &s.rec, 4 * nvc))) return rc;
+  if (p->order == 2 && (rc = kp.mixed ? dalloc(d, &s.rec32, 4 * nvc) : dalloc(d, &s.rec, 4 * nvc))) return rc;
   d->tile1 = 0;
   if (d->pu || first) {
     d->quads = 0;
@@ -1061,8 +1066,7 @@ static int dev_setup(csu_dev* d, const HostMesh& H, int ns, const csu_mesh_desc*
     auto f32 = [](const std::vector<double>& v) { return std::vector<float>(v.begin(), v.end()); };
     if ((rc = upload(d, &g.wg32, f32(H.wg))) ||
         (rc = upload(d, &g.fdsx32, f32(H.fdsx))) || (rc = upload(d, &g.fdsy32, f32(H.fdsy))) ||
-        (rc = upload(d, &g.fds32, f32(H.fds))) || (rc = dalloc(d, &s.fflux32, (size_t)nv * nf)) ||
-        (p->order == 2 && (rc = dalloc(d, &s.rec32, 4 * nvc))))
+        (rc = upload(d, &g.fds32, f32(H.fds))) || (rc = dalloc(d, &s.fflux32, (size_t)nv * nf)))
       return rc;
   }
   if (p->sa || p->sst) {
@@ -2430,13 +2434,13 @@ extern "C" int64_t csu_dev_footprint(const csu_mesh_desc* m, const csu_params* p
   if (p->time_scheme == CSU_TIME_DPLUR) b += 8.0 * block_total((int)nv, m->ncell) + 8.0 * (p->nlinear > 0 ? p->nlinear : 1) * (nc / 256 + 1);
   if (p->precision == 1) b += nc * 64 + nf * (12 + 4 * nv) + (p->order == 2 ? 16 * nv * nc : 0);  // FP32 copies
   if (p->time_scheme == CSU_TIME_RK && !visc && (p->order == 1 || p->limiter != 1) && m->axi == 0 && p->tp == 0) {
-    // tile form: its two primitive buffers, places, face copies, halo cells (at
-    // most one per tile and face between two tiles; a mesh given by its counts
-    // alone: every face may be one)
+    // tile form: places, face copies, halo cells (at most one per tile and
+    // face between two tiles; a mesh given by its counts alone: every face may
+    // be one); first order: two buffers of primitives
     double cross = m->face ? 0 : nf;
     for (int f = 0; m->face && f < m->nface; f++)
       cross += m->face[4 * (size_t)f] / CSU_CHUNK != m->face[4 * (size_t)f + 1] / CSU_CHUNK;
-    b += nc * (64 + (p->order == 1 ? 8 : 16)) + (nf + cross) * ((p->precision == 1 ? 36 : 24) + (p->order == 1 ? 8 : 0)) +
+    b += nc * (p->order == 1 ? 64 + 8 : 16) + (nf + cross) * ((p->precision == 1 ? 36 : 24) + (p->order == 1 ? 8 : 0)) +
          (p->order == 1 ? 0 : 2 * cross * 20) + 16 * nb + 16 * (nc / 256 + 2);
   }
   b += (nv + 4) * 8 * (double)(hist > 0 ? hist : 1);

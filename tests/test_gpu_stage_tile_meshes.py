@@ -106,3 +106,39 @@ def test_first_order_holds_no_lists_it_does_not_read(tmpcase, monkeypatch, preci
     entries = c.nface + int((e[:, 0] != e[:, 1]).sum())
     lists = 4 * (3 * (nt + 1) + nt + 3 * c.nbface) + entries * (24 + 8 + 12 * precision) + 8 * c.ncell
     assert held["hybrid", "0"] - held["hybrid", "1"] == lists + 64 * c.ncell
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_second_order_shares_the_edge_states_room(tmpcase, monkeypatch, precision):
+    """The tile form's primitives lie where the split kernels keep edge
+    states: a context holds its lists more than one without the form, and
+    residual evaluations and precision changes between iterations (which
+    write edge states, or allocate others) leave the results the split
+    form's."""
+    d = tmpcase("sh")
+    cases.write_case(d, _hybrid(), cases.ramp_input(threads=1, nmax=1, precision=precision, stages=3))
+    c = native.HostCase(d)
+    out, held = [], []
+    for stored in ("1", "0"):
+        monkeypatch.setenv("CSU_STORED_PRIMITIVES", stored)
+        dev = native.Device(c)
+        held.append(dev.bytes())
+        if stored == "0":
+            dev.set_launch_shape(64, 64, 1, 1)
+        rows = []
+        for prec in (precision, 1 - precision, 2, precision):
+            dev.set_precision(prec)
+            rows += [dev.iterate(1)[0], *dev.residual().values(), dev.iterate(5)[0], dev.iterate(2)[0],
+                     dev.primitives(), dev.iterate(4)[0], dev.get_state()]
+        out.append(rows)
+        dev.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    nt = (c.ncell + 255) // 256
+    e = c.arrays()["face"][:, :2]
+    t = e // 256
+    cross = t[:, 0] != t[:, 1]
+    halo = len(set(map(tuple, np.r_[np.c_[t[cross, 0], e[cross, 1]], np.c_[t[cross, 1], e[cross, 0]]])))
+    lists = 4 * (3 * (nt + 1) + nt + halo) + (24 + 12 * precision) * (c.nface + cross.sum()) + 16 * (c.ncell + halo)
+    entries = held[1] - held[0] - lists        # boundary faces, of own and halo cells: three numbers each
+    assert entries % 12 == 0 and 12 * c.nbface <= entries <= 4 * 12 * c.nbface
