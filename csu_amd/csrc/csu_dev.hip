@@ -808,23 +808,27 @@ static bool tile_lists(const HostMesh& H, const std::vector<SolveP>* sol, bool f
 
 // The form of an untuned context: the tile form wherever it exists, unless
 // the halos hold clearly more cells than the tiles (a scattered numbering).
-// What the tile form saves in memory traffic it pays in gradients of the
-// halo, so where a gradient costs more (double-double sums) or the traffic
-// less (mixed precision, above the sizes where launches count) the halo may
-// be half as large as the tiles at most.  RK5 iterations, split -> tile, 0.29
-// halo cells per cell (Morton order) and 1.0 (columns longer than a tile):
-//   FP64, Roe       400k cells 286 -> 202 us | 200k 188 -> 175, 800k 569 -> 474
-//   FP64, AUSM+up   400k 291 -> 229          | 200k 188 -> 196, 800k 577 -> 529
-//   mixed, Roe      400k 217 -> 182          | 200k 154 -> 152, 800k 344 -> 365
-//   mixed, AUSMDV   400k 221 -> 197          | 200k 157 -> 171, 800k 349 -> 444
-//   mixed, 100k columns: Roe 108 -> 91, AUSMDV 114 -> 95
-//   long double least squares, Roe:
-//                   400k 386 -> 377          | 200k 252 -> 319, 800k 717 -> 895
-//                   100k 158 -> 161, quads 180k 245 -> 236 | 100k 160 -> 186
+// What the tile form saves in memory traffic and launches it pays in gradients
+// of the halo.  Long double least squares, whose gradients cost most, take it
+// for halos up to a third of the tiles; mixed precision, with the least
+// traffic to save, up to half once its tiles no longer run all at once (256
+// CUs with three of the Roe form for triangles each, two of the others), the
+// Barth limiter aside, which is cheap.  RK5 iterations, split -> tile, by halo
+// cells per cell:
+//                    0.24-0.29 (Morton)         0.79                    1.0
+//   FP64, Roe        400k cells 286 -> 202 us   160k 161 -> 146         200k 188 -> 175, 800k 569 -> 474
+//   FP64, AUSM+up    400k 291 -> 229            160k 164 -> 165         200k 188 -> 196, 800k 577 -> 529
+//   mixed, Roe       400k 217 -> 182            160k 137 -> 116         200k 154 -> 152, 800k 344 -> 365
+//   mixed, AUSMDV    400k 221 -> 197            160k 140 -> 144         100k 114 -> 95, 200k 157 -> 171, 800k 349 -> 444
+//   mixed, Barth, Roe                           400k 209 -> 199         160k 129 -> 102
+//   long double, Roe 100k 158 -> 161            160k 209 -> 240         200k 252 -> 319, 800k 717 -> 895
+//                    400k 386 -> 377            (0.40: 140k 202 -> 217)
 static int tile_default(const csu_dev* d) {
   if (!d->tile_ok) return 0;
-  const bool half = d->kp.lsq_ld || (d->kp.mixed && d->nc > TILE_SMALL);
-  return (double)d->tl.nh <= (half ? 0.5 : TILE_HALO) * d->nc;
+  const KP& kp = d->kp;
+  const int at_once = 256 * (kp.flux == 0 && !d->quads ? 3 : 2);
+  const double most = kp.lsq_ld ? 0.35 : kp.mixed && kp.limiter != 2 && nblk(d->nc) > at_once ? 0.5 : TILE_HALO;
+  return (double)d->tl.nh <= most * d->nc;
 }
 
 static TuneKey tune_key(const csu_dev* d) {
@@ -1899,8 +1903,8 @@ extern "C" int csu_dev_autotune(csu_dev* d, int32_t iters, int32_t* choice) {
 // Launch shapes chosen by the caller (a shape the autotuner picked in an
 // earlier process, or a fixed one for profiling runs): gradient/face
 // workgroup and LU-SGS level workgroup (64, 128 or 256), XCD tile map (0
-// or 1), tile form of the face flux + update (0 or 1; primitives-from-state
-// runs only).  Results do not depend on them.
+// or 1), tile form (0 or 1; where its lists exist, tile_ok).  Results do not
+// depend on them.
 extern "C" int csu_dev_set_launch_shape(csu_dev* d, const int32_t* choice) {
   if (!d || !choice) return set_err(CSU_ERR_ARG, "null argument");
   auto ok = [](int b) { return b == 64 || b == 128 || b == 256; };
@@ -1923,7 +1927,8 @@ extern "C" int csu_dev_set_launch_shape(csu_dev* d, const int32_t* choice) {
 }
 
 // Launch shapes in use: gradient/face workgroup, LU-SGS level workgroup,
-// XCD tile map, tile form; returns 1 when they came from the autotuner.
+// XCD tile map, tile form (0 for first-order runs, which take it without a
+// choice); returns 1 when they came from the autotuner.
 extern "C" int csu_dev_launch_shape(const csu_dev* d, int32_t* choice) {
   if (!d || !choice) return -set_err(CSU_ERR_ARG, "null argument");
   choice[0] = d->sblk; choice[1] = d->lblk; choice[2] = d->kp.xcd; choice[3] = d->tile;

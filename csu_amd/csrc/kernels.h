@@ -87,7 +87,7 @@ __device__ __forceinline__ void lsq_grad(int np, const double* dx, const double*
   gy = dd_div(dd_add(dd_mul(nb, A), dd_mul(a, B)), det).hi;
 }
 
-// Gradient + limiter (+ boundary work) kernel.  Reference solverUpdateGrad /
+// Gradient + limiter kernel, with the ghost states of the cell's boundary faces.  Reference solverUpdateGrad /
 // solverCalcGrad3 (solver.c:451-474, 1031-1074), solverGrad_T
 // (solver.c:477-490), the limiter loop of inter() (solver.c:496-548,
 // limiter.c:98-147), boundaryCalcPrimitive (boundary.c:514-693).
@@ -826,7 +826,7 @@ __global__ void k_time_clamp(double* __restrict__ ts, double* __restrict__ dtg, 
 
 // End of an iteration: the final level of the residual norm, the wall force
 // coefficients Cx_p, Cx_v, Cy_p, Cy_v (solverCalcCoeff3, solver.c:1342-1401;
-// friction per face comes from k_grad) and, where the next step needs one,
+// friction per face comes from bc_face) and, where the next step needs one,
 // the global time step (k_dt_final).  One workgroup each and per solve,
 // running beside each other: as three launches they cost 4-5 us apiece.
 // The norm's threads sum strided slices of the block partials (rows of
@@ -843,7 +843,7 @@ struct TailP {
   int dtc;  // cells behind one entry of red_dt
   double cfl, sref;
   const SolveP* sol;
-  const double *red, *red_dt;  // red_dt null: no time step
+  const double *red, *red_dt;  // red_dt: read by the third role only (a grid without it: no time step)
   const int* wall;
   const double *Pb, *wfric, *bdsx, *bdsy;
   double *res, *coef, *dtg;

@@ -420,8 +420,8 @@ class Device:
                 "tuned": bool(tuned == 1)}
 
     def set_launch_shape(self, block: int, lusgs_block: int, xcd_map: int, tile: int = 0):
-        """tile 1 (inviscid second-order RK runs): the face fluxes evaluated
-        per cell tile inside the update kernel, no face-flux kernel."""
+        """tile 1 (inviscid second-order RK runs): each stage one kernel over
+        256-cell tiles, edge states and face fluxes in LDS."""
         ch = np.array([block, lusgs_block, xcd_map, tile], np.int32)
         check(lib().csu_dev_set_launch_shape(self._h, _p(ch, C.c_int32)))
 

@@ -287,9 +287,14 @@ int  csu_batch_run(csu_dev* dev, double drop, int32_t max_iter, int32_t chunk,
  * of two runs) and keep the fastest; the context then continues from the
  * state it had, and later contexts of the same kind of run and mesh-size
  * bucket (log2 of the cell count) in the process take the same choice
- * without timing.  Results do not depend on these choices (an untuned
- * context takes the tile form unless its numbering scatters neighbours over
- * the tiles).  choice: [4] (block, LU-SGS block, XCD map, tile) or NULL.
+ * without timing, if the tile form exists for them, and is the default, as
+ * for the one that was timed.  Results do not depend on these choices.  An
+ * untuned context takes the tile form unless its numbering scatters
+ * neighbours over the tiles (long double least squares and large
+ * mixed-precision runs want fewer cells around a tile than column order
+ * has), also when its precision changes; first-order runs take it or not by
+ * themselves and report 0.
+ * choice: [4] (block, LU-SGS block, XCD map, tile) or NULL.
  * csu_dev_launch_shape reports the shapes in use (returns 1 if tuned). */
 int  csu_dev_autotune(csu_dev* dev, int32_t iters, int32_t* choice);
 int  csu_dev_launch_shape(const csu_dev* dev, int32_t* choice);

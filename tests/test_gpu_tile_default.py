@@ -20,21 +20,24 @@ def _case(tmpcase, nx, ny, order, **inp):
     return native.HostCase(d)
 
 
-# halo cells per cell 1.0 (columns longer than a tile), 0.27, 1.0, 0.24 and 2.7:
-# the form in FP64, mixed precision, long double sums
-@pytest.mark.parametrize("nx,ny,order,forms", [(270, 250, "column", (1, 0, 0)), (270, 250, "morton", (1, 1, 1)),
-                                               (100, 150, "column", (1, 1, 0)), (50, 50, "morton", (1, 1, 1)),
-                                               (50, 50, "scattered", (0, 0, 0))])
-def test_default_form(tmpcase, nx, ny, order, forms):
+# halo cells per cell 1.0 (columns longer than a tile), 0.27, 0.24 and 2.7: the
+# form in FP64, mixed precision, long double sums; mixed precision with tiles
+# that run all at once (117; 528: Roe on triangles only) and not (801)
+@pytest.mark.parametrize("nx,ny,order,flux,forms", [
+    (410, 250, "column", "ROE", (1, 0, 0)), (270, 250, "column", "ROE", (1, 1, 0)),
+    (270, 250, "column", "AUSMDV", (1, 0, 0)), (270, 250, "morton", "AUSMDV", (1, 1, 1)),
+    (100, 150, "column", "AUSMDV", (1, 1, 0)), (50, 50, "morton", "ROE", (1, 1, 1)),
+    (50, 50, "scattered", "ROE", (0, 0, 0))])
+def test_default_form(tmpcase, nx, ny, order, flux, forms):
     for precision, tile in enumerate(forms):
-        dev = native.Device(_case(tmpcase, nx, ny, order, precision=precision))
+        dev = native.Device(_case(tmpcase, nx, ny, order, flux=flux, precision=precision))
         sh = dev.launch_shape()
         dev.close()
         assert sh["tuned"] or sh["tile"] == tile, precision
 
 
 def test_form_follows_the_precision(tmpcase):
-    c = _case(tmpcase, 270, 250, "column")
+    c = _case(tmpcase, 270, 250, "column", flux="AUSMDV")
     U0 = c.initial_state() * (1 + 0.02 * np.random.default_rng(5).standard_normal((c.nvar, c.ncell)))
     out = []
     for tile in (None, 0, 1):
