@@ -35,7 +35,8 @@ __global__ __launch_bounds__(CSU_BLOCK) void k_to_f32(const double* __restrict__
 // own cells' slots only).
 // csl, cel, hsl, hel are zero before.  Each own face slot's face is in ent
 // (HostMesh::linked), each cell across an outer face in the halo list.
-// Bound by its gathers, 25 us at 400k cells, where the host's loops took 30 ms.
+// Bound by its gathers: 33 us at 400k cells in Morton order, where the host's
+// loops took 30 ms.
 template <bool O1>
 __global__ __launch_bounds__(CSU_CHUNK) void k_tile_lists(int nc, Geo g, Tile tl, const int* __restrict__ ent,
                                                           const int* __restrict__ btgt, double* __restrict__ fx,
