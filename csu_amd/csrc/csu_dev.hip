@@ -6,6 +6,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <float.h>
 #include <math.h>
 #include <algorithm>
 #include <map>
@@ -290,7 +291,11 @@ static std::vector<double> wall_segments(const csu_mesh_desc* m, int* nw, int* n
     const int32_t* q = m->bface + 3 * w[j];
     const double x0 = m->node_xy[2 * q[1]], y0 = m->node_xy[2 * q[1] + 1];
     const double x1 = m->node_xy[2 * q[2]], y1 = m->node_xy[2 * q[2] + 1];
-    const double ex = x1 - x0, ey = y1 - y0, den = ex * ex + ey * ey;
+    const double ex = x1 - x0, ey = y1 - y0;
+    double den = ex * ex + ey * ey;
+    // a length whose square has no finite reciprocal (below 1.5e-154): any
+    // point of it is as near as any other, and infinity makes that its first
+    if (den > 0.0 && den < DBL_MIN) den = INFINITY;
     seg[j] = x0; seg[n + j] = y0; seg[2 * n + j] = ex; seg[3 * n + j] = ey; seg[4 * n + j] = den;
     seg[5 * n + j] = 1.0 / den;
     box[4 * nk] = fmax(box[4 * nk], fmax(fmax(fabs(x0), fabs(x1)), fmax(fabs(y0), fabs(y1))));
